@@ -30,6 +30,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "sa/rng.hpp"
 
 namespace sa {
@@ -1165,13 +1167,26 @@ __global__ void __launch_bounds__(256) k_sweep2d_odd(sweep_args p, int color) {
 
 // ---------------------------------------------------------------- measure
 // Per system and lane: number of satisfied -x,-y[,-z] bonds and of set spins.
-// Each lane keeps bit-sliced counters (bit k of plane b = bit b of lane k's count):
-// a full adder folds the bond words of one site into a 2-bit sum that is rippled
-// into six planes; the spin word ripples into five.  Every 16 site groups the
-// planes are turned into ordinary per-lane counts by a 64x64 bit transpose across
-// the wave (six butterfly stages of lane shuffles) and a popcount, so lane k ends
-// up holding the counts of bit k.  Blocks reduce in LDS and add one atomic per
-// lane and counter.
+//
+// Memory bounds it at large ladders: every spin word once plus the couplings.  A thread
+// owns one in-plane site and walks z (3D) with the word below kept in a register, so a
+// plane is read by one block only (a walk over linear site indices read every plane on
+// two XCDs); all system blocks of one unit (in-plane chunk, z segment) have consecutive
+// slots on one XCD, which reads the unit's couplings once into its L2.
+//
+// Counting: per lane bit-sliced counters (bit k of plane b = bit b of lane k's count).
+// Two sites at a time go through full adders into small counters; every 8 sites those
+// ripple into larger ones (about 36 instructions per word; rippling each site through all
+// planes and transposing every 16 sites took about 100).  At the end the block's four
+// waves add their planes through LDS, and a 64x64 bit transpose across the wave (six
+// butterfly stages of lane shuffles) and a popcount turn each plane into ordinary
+// per-lane counts; the transposes are shared out over the waves.  One atomic per lane and
+// counter and block.
+//
+// Measured: 32 systems of 3D L=128 (587 MB read once) 350 -> 182 us, 3.2 TB/s; one site
+// per thread instead of a pair 240, units in the slots' outer order (couplings re-read by
+// every system block) 210.  Three systems, as an exchange step measures: 3D L=32 29 -> 6
+// us, L=128 46 -> 27, 2D L=64 14 -> 6.
 
 // Wave-wide 64x64 bit transpose: lane i holds row i on entry, column i on exit.
 // Stage d exchanges bit d of the lane index with bit d of the bit index.
@@ -1193,153 +1208,375 @@ __device__ __forceinline__ uint64_t wave_transpose64(uint64_t x, int lane) {
   return x;
 }
 
-// The measurement's per-lane counters are kept in kMeasureCopies copies
-// (cnt[copy][listed system][128], copy = block index mod kMeasureCopies), summed on
-// the host: blocks then contend for an address 8 times less.
+// The measurement's per-lane counters are kept in up to kMeasureCopies copies
+// (cnt[copy][listed system][128], copy = unit index mod copies), summed on the host:
+// blocks then contend for an address that much less.  A larger ladder has that many
+// more addresses, and fewer copies to move and sum (32 systems: 8 copies are 131 KB).
 constexpr int kMeasureCopies = 8;
+__host__ __device__ __forceinline__ int measure_copies(int n) { return n <= 8 ? kMeasureCopies : 2; }
 
 // up to four listed systems, passed by value
 struct sys4 {
   int v[4];
 };
 
+// steps (sites) of one thread: 3 bonds each must stay below 2^7, one spin each below 2^6
+constexpr int kMeasWalk = 40;
+constexpr int kMeasE = 7, kMeasM = 6;  // planes of a thread's counters
+constexpr int kMeasPlanes = kMeasE + kMeasM;
+
+struct meas_small {  // up to 8 sites
+  uint64_t e[5], m[4];
+};
+struct meas_big {
+  uint64_t e[kMeasE], m[kMeasM];
+};
+
+// sum of two bit-sliced numbers, a += b (nb planes into na)
+template <int NA, int NB>
+__device__ __forceinline__ void planes_add(uint64_t (&a)[NA], const uint64_t (&b)[NB]) {
+  uint64_t c = a[0] & b[0];
+  a[0] ^= b[0];
+#pragma unroll
+  for (int i = 1; i < NA; ++i) {
+    if (i < NB) {
+      const uint64_t t = maj3(a[i], b[i], c);
+      a[i] = xor3(a[i], b[i], c);
+      c = t;
+    } else {
+      const uint64_t t = a[i] & c;
+      a[i] ^= c;
+      c = t;
+    }
+  }
+}
+
+// two sites' bond words (satisfied bits: sum s of weight 1, carry c of weight 2) and spins
+__device__ __forceinline__ void meas_add2(meas_small &a, uint64_t s1, uint64_t c1, uint64_t w1, uint64_t s2, uint64_t c2,
+                                          uint64_t w2) {
+  const uint64_t c = maj3(a.e[0], s1, s2);
+  a.e[0] = xor3(a.e[0], s1, s2);
+  const uint64_t t = xor3(c1, c2, c), u = maj3(c1, c2, c);
+  const uint64_t v = a.e[1] & t;
+  a.e[1] ^= t;
+  const uint64_t x = maj3(a.e[2], u, v);
+  a.e[2] = xor3(a.e[2], u, v);
+  const uint64_t y = a.e[3] & x;
+  a.e[3] ^= x;
+  a.e[4] ^= y;
+  const uint64_t p = maj3(a.m[0], w1, w2);
+  a.m[0] = xor3(a.m[0], w1, w2);
+  const uint64_t q = a.m[1] & p;
+  a.m[1] ^= p;
+  const uint64_t r = a.m[2] & q;
+  a.m[2] ^= q;
+  a.m[3] ^= r;
+}
+
+// The block's four waves' planes summed, turned into per-lane counts and added to cnt.
+template <int SB>
+struct meas_shared {
+  uint64_t v[2][SB][kMeasPlanes + 2][64];  // planes of two waves / the block's planes
+};
+template <int SB>
+__device__ __forceinline__ void meas_finish(const meas_big (&big)[SB], meas_shared<SB> &sh, int (&red)[SB][2][64],
+                                            int nsys, int sys0, int ns, int unit, int *cnt) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  // the four waves' planes added through LDS: waves 2, 3 into 0, 1, then 1 into 0
+  for (int q = threadIdx.x; q < SB * 128; q += blockDim.x) (&red[0][0][0])[q] = 0;
+  uint64_t e[SB][kMeasE + 2], mm[SB][kMeasM + 2];
+#pragma unroll
+  for (int m = 0; m < SB; ++m) {
+#pragma unroll
+    for (int b = 0; b < kMeasE + 2; ++b) e[m][b] = b < kMeasE ? big[m].e[b < kMeasE ? b : 0] : 0;
+#pragma unroll
+    for (int b = 0; b < kMeasM + 2; ++b) mm[m][b] = b < kMeasM ? big[m].m[b < kMeasM ? b : 0] : 0;
+  }
+#pragma unroll
+  for (int round = 0; round < 2; ++round) {
+    const int from = round == 0 ? 2 : 1;  // waves from .. 2*from-1 hand theirs to wave - from
+    if (wv >= from && wv < 2 * from) {
+#pragma unroll
+      for (int m = 0; m < SB; ++m) {
+#pragma unroll
+        for (int b = 0; b < kMeasE + 1; ++b) sh.v[wv - from][m][b][lane] = e[m][b];
+#pragma unroll
+        for (int b = 0; b < kMeasM + 1; ++b) sh.v[wv - from][m][kMeasE + 1 + b][lane] = mm[m][b];
+      }
+    }
+    __syncthreads();
+    if (wv < from) {
+#pragma unroll
+      for (int m = 0; m < SB; ++m) {
+        uint64_t oe[kMeasE + 1], om[kMeasM + 1];
+#pragma unroll
+        for (int b = 0; b < kMeasE + 1; ++b) oe[b] = sh.v[wv][m][b][lane];
+#pragma unroll
+        for (int b = 0; b < kMeasM + 1; ++b) om[b] = sh.v[wv][m][kMeasE + 1 + b][lane];
+        planes_add(e[m], oe);
+        planes_add(mm[m], om);
+      }
+    }
+    __syncthreads();
+  }
+  // wave 0's planes to all waves; each transposes its share
+  constexpr int PB = kMeasPlanes + 4;  // planes per system: kMeasE + 2 and kMeasM + 2
+  uint64_t *pl = &sh.v[0][0][0][0];      // [SB][PB][64]: 2 * (kMeasPlanes + 2) >= PB planes per system
+  if (wv == 0) {
+#pragma unroll
+    for (int m = 0; m < SB; ++m) {
+#pragma unroll
+      for (int b = 0; b < kMeasE + 2; ++b) pl[(m * PB + b) * 64 + lane] = e[m][b];
+#pragma unroll
+      for (int b = 0; b < kMeasM + 2; ++b) pl[(m * PB + kMeasE + 2 + b) * 64 + lane] = mm[m][b];
+    }
+  }
+  __syncthreads();
+  for (int q = wv; q < SB * PB; q += 4) {
+    const int m = q / PB, b = q - m * PB;
+    const uint64_t v = pl[q * 64 + lane];
+    if (__ballot(v != 0) == 0) continue;  // an empty plane
+    const bool isE = b < kMeasE + 2;
+    atomicAdd(&red[m][isE ? 0 : 1][lane], __popcll(wave_transpose64(v, lane)) << (isE ? b : b - kMeasE - 2));
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < ns * 128; q += blockDim.x)
+    atomicAdd(&cnt[((int64_t)(unit % measure_copies(nsys)) * nsys + sys0) * 128 + q], (&red[0][0][0])[q]);
+}
+
+// Block = one unit (3D: 256 in-plane sites x up to `walk` planes; 2D: 256*walk
+// consecutive sites) of SB systems.
 template <int KIND, int SB>
 __global__ void __launch_bounds__(256) k_measure(const uint64_t *__restrict__ s_all, const uint64_t *__restrict__ jx,
                                                  const uint64_t *__restrict__ jy, const uint64_t *__restrict__ jz,
                                                  int L, int64_t N, int nsys, const int *__restrict__ sys_list,
-                                                 sys4 sel, int *cnt) {
-  // SB: systems per pass over the sites (couplings loaded once per pass); with few
-  // systems one per block row gives more waves in flight
-  constexpr int FLUSH = 16;  // groups between flushes: E <= 3*16 < 64, M <= 16 < 32
+                                                 sys4 sel, int *cnt, int units, int chunks, int walk) {
+  __shared__ meas_shared<SB> sh;
   __shared__ int red[SB][2][64];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int sys0 = blockIdx.y * SB;
+  const int nq = (nsys + SB - 1) / SB;
+  // blocks go round-robin over the 8 XCDs; slot i of XCD b%8: unit 8*(i/nq) + b%8, system block i%nq
+  const int slot = (int)(blockIdx.x >> 3);
+  const int unit = 8 * (slot / nq) + (int)(blockIdx.x & 7);
+  if (unit >= units) return;
+  const int sys0 = (slot % nq) * SB;
   const int ns = (nsys - sys0) < SB ? (nsys - sys0) : SB;
-  for (int q = threadIdx.x; q < SB * 128; q += blockDim.x) (&red[0][0][0])[q] = 0;
-  __syncthreads();
-  const int64_t L2 = (int64_t)L * L;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  uint64_t e[SB][6], mc[SB][5];
-  int sat[SB], up[SB];
+  const uint32_t uL = (uint32_t)L, uL2 = uL * uL;
+  const uint64_t *sp[SB];
 #pragma unroll
   for (int m = 0; m < SB; ++m) {
-    sat[m] = up[m] = 0;
-#pragma unroll
-    for (int b = 0; b < 6; ++b) e[m][b] = 0;
-#pragma unroll
-    for (int b = 0; b < 5; ++b) mc[m][b] = 0;
+    const int q = sys0 + (m < ns ? m : 0);
+    const int sys = sys_list ? sys_list[q] : (sel.v[0] >= 0 ? sel.v[q & 3] : q);  // sel: at most 4 systems
+    sp[m] = s_all + (int64_t)sys * N;
   }
-  int pending = 0;
-  auto flush = [&]() {
+  // the thread's first site (x, y), its plane, and how many steps it takes
+  const uint32_t p0 = (KIND == KIND_3D ? (uint32_t)(unit % chunks) * 256u : (uint32_t)unit * (uint32_t)(256 * walk)) +
+                      threadIdx.x;
+  uint32_t x = p0 % uL, y = p0 / uL;
+  uint32_t z = KIND == KIND_3D ? (uint32_t)(unit / chunks) * (uint32_t)walk : 0u;
+  const uint32_t dx = 256u % uL, dy = 256u / uL;  // 2D: the next step's site is 256 further on
+  int steps;
+  if (KIND == KIND_3D) {
+    steps = p0 < uL2 ? min(walk, (int)(uL - z)) : 0;
+  } else {
+    steps = p0 < uL2 ? min(walk, (int)((uL2 - p0 + 255u) / 256u)) : 0;
+  }
+  const uint32_t iw0 = p0 - x + (x == 0 ? uL - 1 : x - 1), in0 = y == 0 ? p0 + uL2 - uL : p0 - uL;
+  uint64_t below[SB];
+#pragma unroll
+  for (int m = 0; m < SB; ++m)
+    below[m] = (KIND == KIND_3D && steps > 0) ? sp[m][(int64_t)(z == 0 ? uL - 1 : z - 1) * uL2 + p0] : 0;
+  meas_big big[SB];
+#pragma unroll
+  for (int m = 0; m < SB; ++m) {
+#pragma unroll
+    for (int b = 0; b < kMeasE; ++b) big[m].e[b] = 0;
+#pragma unroll
+    for (int b = 0; b < kMeasM; ++b) big[m].m[b] = 0;
+  }
+  // eight steps from j0 on, four at a time with all their loads issued before any of
+  // them is counted; FULL: every lane of the wave has all eight
+  constexpr int U = 4;
+  auto eight = [&](int j0, auto full) {
+    constexpr bool FULL = decltype(full)::value;
+    meas_small a[SB];
 #pragma unroll
     for (int m = 0; m < SB; ++m) {
 #pragma unroll
-      for (int b = 0; b < 6; ++b) {
-        sat[m] += __popcll(wave_transpose64(e[m][b], lane)) << b;
-        e[m][b] = 0;
-      }
+      for (int b = 0; b < 5; ++b) a[m].e[b] = 0;
 #pragma unroll
-      for (int b = 0; b < 5; ++b) {
-        up[m] += __popcll(wave_transpose64(mc[m][b], lane)) << b;
-        mc[m][b] = 0;
-      }
+      for (int b = 0; b < 4; ++b) a[m].m[b] = 0;
     }
-  };
-  // U groups per pass: all their loads are issued before any of them is counted, so
-  // a wave waits for memory once per pass (with one system per block row; with four
-  // the loads of one group already fill the registers)
-  constexpr int U = SB == 1 ? 4 : 1;
-  uint64_t Jw[U], Jn[U], Ju[U], w[U][SB], sw[U][SB], sn[U][SB], su[U][SB];
-  bool west[U];
-  for (int64_t base0 = (int64_t)blockIdx.x * blockDim.x + wv * 64; base0 < N; base0 += U * stride) {
 #pragma unroll
-    for (int g = 0; g < U; ++g) {
-      const int64_t base = base0 + g * stride;
-      // coordinates of the group's first site once per wave (scalar), then per lane
-      // by stepping along the row: no per-site division
-      const uint32_t b32 = (uint32_t)base, uL = (uint32_t)L, uL2 = (uint32_t)L2;
-      const uint32_t zb = b32 / uL2, rem = b32 - zb * uL2, yb = rem / uL, xb = rem - yb * uL;
-      uint32_t x = xb + (uint32_t)lane, y = yb, z = zb;
-      while (x >= uL) {  // at most 64/L steps
-        x -= uL;
-        if (++y == uL) {
-          y = 0;
-          ++z;
+    for (int h = 0; h < 8; h += U) {
+      uint64_t Jw[U], Jn[U], Ju[U], w[U][SB], sw[U][SB], sn[U][SB];
+#pragma unroll
+      for (int g = 0; g < U; ++g) {
+        const int j = j0 + h + g;
+        const bool in = FULL || j < steps;  // steps beyond the range hold zero words and count nothing
+        uint32_t i, iw, inn;
+        bool west = true;
+        int64_t P = 0;
+        if (KIND == KIND_3D) {
+          i = p0;
+          iw = iw0;
+          inn = in0;
+          P = (int64_t)(z + (uint32_t)j) * uL2;
+        } else {
+          i = p0 + 256u * (uint32_t)j;
+          iw = i - x + (x == 0 ? uL - 1 : x - 1);
+          inn = y == 0 ? i + uL2 - uL : i - uL;
+          west = !(KIND == KIND_2P && x == 0);  // no open-x west bond
+          x += dx;
+          y += dy;
+          if (x >= uL) {
+            x -= uL;
+            ++y;
+          }
         }
-      }
-      const uint32_t i = b32 + (uint32_t)lane;
-      const bool in = base < N && (int64_t)i < N;
-      Jw[g] = Jn[g] = Ju[g] = 0;
-      west[g] = true;
-#pragma unroll
-      for (int m = 0; m < SB; ++m) w[g][m] = sw[g][m] = sn[g][m] = su[g][m] = 0;
-      if (in) {
-        const uint32_t iw = i - x + (x == 0 ? uL - 1 : x - 1);
-        const uint32_t inn = (y == 0) ? i + uL2 - uL : i - uL;
-        const uint32_t iu = (KIND == KIND_3D) ? ((z == 0) ? i + (uint32_t)(N - L2) : i - uL2) : 0;
-        Jw[g] = jx[i];
-        Jn[g] = jy[i];
-        west[g] = !(KIND == KIND_2P && x == 0);  // no open-x west bond
-        if (KIND == KIND_3D) Ju[g] = jz[i];
+        Jw[g] = (in && west) ? jx[P + i] : 0;
+        Jn[g] = in ? jy[P + i] : 0;
+        Ju[g] = (in && KIND == KIND_3D) ? jz[P + i] : 0;
 #pragma unroll
         for (int m = 0; m < SB; ++m) {
-          if (m >= ns) break;
-          const int q = sys0 + m;
-          const int sys = sys_list ? sys_list[q] : (sel.v[0] >= 0 ? sel.v[q & 3] : q);  // sel: at most 4 systems
-          const uint64_t *s = s_all + (int64_t)sys * N;
-          w[g][m] = s[i];
-          sw[g][m] = s[iw];
-          sn[g][m] = s[inn];
-          if (KIND == KIND_3D) su[g][m] = s[iu];
+          w[g][m] = in ? sp[m][P + i] : 0;
+          sn[g][m] = in ? sp[m][P + inn] : 0;
+          // without a west bond its word is the site's own: w ^ w = 0 counts nothing
+          sw[g][m] = in ? sp[m][west ? P + iw : P + i] : 0;
         }
       }
-    }
-#pragma unroll
-    for (int g = 0; g < U; ++g) {
-      if (base0 + g * stride >= N) break;  // wave-uniform
 #pragma unroll
       for (int m = 0; m < SB; ++m) {
-        if (m >= ns) break;
-        const uint64_t ww = w[g][m];
-        const uint64_t bw = west[g] ? (Jw[g] ^ ww ^ sw[g][m]) : 0;
-        const uint64_t bn = Jn[g] ^ ww ^ sn[g][m];
-        const uint64_t bu = (KIND == KIND_3D) ? (Ju[g] ^ ww ^ su[g][m]) : 0;
-        // satisfied bonds of this site: sum bit sb (weight 1) and carry cb (weight 2);
-        // lanes outside the lattice hold zero words and count nothing
-        const uint64_t sb = bw ^ bn ^ bu, cb = maj3(bw, bn, bu);
-        uint64_t t = e[m][0] & sb;
-        e[m][0] ^= sb;
-        uint64_t u = maj3(e[m][1], cb, t);
-        e[m][1] ^= cb ^ t;
+        uint64_t sb[U], cb[U];
 #pragma unroll
-        for (int b = 2; b < 6; ++b) {
-          const uint64_t v = e[m][b] & u;
-          e[m][b] ^= u;
-          u = v;
+        for (int g = 0; g < U; ++g) {
+          const uint64_t bw = xor3(Jw[g], w[g][m], sw[g][m]), bn = xor3(Jn[g], w[g][m], sn[g][m]);
+          if (KIND == KIND_3D) {
+            const uint64_t bu = (FULL || j0 + h + g < steps) ? xor3(Ju[g], w[g][m], below[m]) : 0;
+            sb[g] = xor3(bw, bn, bu);
+            cb[g] = maj3(bw, bn, bu);
+            below[m] = w[g][m];
+          } else {
+            sb[g] = bw ^ bn;
+            cb[g] = bw & bn;
+          }
         }
-        t = ww;
 #pragma unroll
-        for (int b = 0; b < 5; ++b) {
-          const uint64_t v = mc[m][b] & t;
-          mc[m][b] ^= t;
-          t = v;
-        }
-      }
-      if (++pending == FLUSH) {
-        flush();
-        pending = 0;
+        for (int g = 0; g < U; g += 2) meas_add2(a[m], sb[g], cb[g], w[g][m], sb[g + 1], cb[g + 1], w[g + 1][m]);
       }
     }
+#pragma unroll
+    for (int m = 0; m < SB; ++m) {
+      planes_add(big[m].e, a[m].e);
+      planes_add(big[m].m, a[m].m);
+    }
+  };
+  for (int j0 = 0; j0 < walk; j0 += 8) {
+    if (__all(j0 + 8 <= steps)) eight(j0, std::true_type{});
+    else eight(j0, std::false_type{});
   }
-  if (pending) flush();
+  meas_finish<SB>(big, sh, red, nsys, sys0, ns, unit, cnt);
+}
+
+// 3D with an even side and spin arrays below 2^31 bytes: a thread owns a pair of
+// neighbouring in-plane sites (128-bit loads; the second site's -x neighbour is the
+// first), buffer loads with the plane offset in a scalar register.  A unit is 512
+// in-plane sites x up to `walk` planes (walk <= kMeasWalk / 2 pairs).
+template <int SB>
+__global__ void __launch_bounds__(256) k_measure3d_pair(const uint64_t *__restrict__ s_all,
+                                                        const uint64_t *__restrict__ jx,
+                                                        const uint64_t *__restrict__ jy,
+                                                        const uint64_t *__restrict__ jz, int L, int64_t N, int nsys,
+                                                        const int *__restrict__ sys_list, sys4 sel, int *cnt, int units,
+                                                        int chunks, int walk) {
+  __shared__ meas_shared<SB> sh;
+  __shared__ int red[SB][2][64];
+  const int nq = (nsys + SB - 1) / SB;
+  const int slot = (int)(blockIdx.x >> 3);  // as in k_measure
+  const int unit = 8 * (slot / nq) + (int)(blockIdx.x & 7);
+  if (unit >= units) return;
+  const int sys0 = (slot % nq) * SB;
+  const int ns = (nsys - sys0) < SB ? (nsys - sys0) : SB;
+  const uint32_t uL = (uint32_t)L, uL2 = uL * uL, bytes = (uint32_t)N * 8u;
+  buf_t sp[SB];
 #pragma unroll
   for (int m = 0; m < SB; ++m) {
-    atomicAdd(&red[m][0][lane], sat[m]);
-    atomicAdd(&red[m][1][lane], up[m]);
+    const int q = sys0 + (m < ns ? m : 0);
+    const int sys = sys_list ? sys_list[q] : (sel.v[0] >= 0 ? sel.v[q & 3] : q);  // sel: at most 4 systems
+    sp[m] = make_buf(s_all + (int64_t)sys * N, bytes);
   }
-  __syncthreads();
-  for (int q = threadIdx.x; q < ns * 128; q += blockDim.x)
-    atomicAdd(&cnt[((int64_t)(blockIdx.x % kMeasureCopies) * nsys + sys0) * 128 + q], (&red[0][0][0])[q]);
+  const buf_t bx = make_buf(jx, bytes), by = make_buf(jy, bytes), bz = make_buf(jz, bytes);
+  const uint32_t p0 = (uint32_t)(unit % chunks) * 512u + threadIdx.x * 2u;
+  const uint32_t x = p0 % uL, y = p0 / uL;
+  const int z0 = (unit / chunks) * walk, steps = min(walk, L - z0);
+  const uint32_t plane = uL2 * 8u;
+  // lanes beyond the plane and steps beyond the range read zeros (offset past the end)
+  const bool in = p0 < uL2;
+  const uint32_t vo = in ? p0 * 8u : kOutOfRange;
+  const uint32_t vw = in ? (p0 - x + (x == 0 ? uL - 1 : x - 1)) * 8u : kOutOfRange;
+  const uint32_t vn = in ? (y == 0 ? p0 + uL2 - uL : p0 - uL) * 8u : kOutOfRange;
+  uint64_t below[SB][2];
+#pragma unroll
+  for (int m = 0; m < SB; ++m) bld2(sp[m], vo, (uint32_t)(z0 == 0 ? L - 1 : z0 - 1) * plane, below[m][0], below[m][1]);
+  meas_big big[SB];
+#pragma unroll
+  for (int m = 0; m < SB; ++m) {
+#pragma unroll
+    for (int b = 0; b < kMeasE; ++b) big[m].e[b] = 0;
+#pragma unroll
+    for (int b = 0; b < kMeasM; ++b) big[m].m[b] = 0;
+  }
+  constexpr int U = 2;  // planes whose loads are issued together
+  for (int j0 = 0; j0 < steps; j0 += 4) {
+    meas_small a[SB];
+#pragma unroll
+    for (int m = 0; m < SB; ++m) {
+#pragma unroll
+      for (int b = 0; b < 5; ++b) a[m].e[b] = 0;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) a[m].m[b] = 0;
+    }
+#pragma unroll
+    for (int h = 0; h < 4; h += U) {
+      uint64_t Jx[U][2], Jy[U][2], Jz[U][2], w[U][SB][2], sw[U][SB], sn[U][SB][2];
+#pragma unroll
+      for (int g = 0; g < U; ++g) {
+        const int j = j0 + h + g;
+        const bool ok = j < steps;  // uniform
+        const uint32_t P = (uint32_t)(z0 + (ok ? j : 0)) * plane;
+        const uint32_t o = ok ? vo : kOutOfRange, ow = ok ? vw : kOutOfRange, on = ok ? vn : kOutOfRange;
+        bld2(bx, o, P, Jx[g][0], Jx[g][1]);
+        bld2(by, o, P, Jy[g][0], Jy[g][1]);
+        bld2(bz, o, P, Jz[g][0], Jz[g][1]);
+#pragma unroll
+        for (int m = 0; m < SB; ++m) {
+          bld2(sp[m], o, P, w[g][m][0], w[g][m][1]);
+          bld2(sp[m], on, P, sn[g][m][0], sn[g][m][1]);
+          sw[g][m] = bld(sp[m], ow, P);
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < U; ++g) {
+        const uint64_t live = j0 + h + g < steps ? ~0ULL : 0ULL;
+#pragma unroll
+        for (int m = 0; m < SB; ++m) {
+          const uint64_t w0 = w[g][m][0], w1 = w[g][m][1];
+          const uint64_t x0 = xor3(Jx[g][0], w0, sw[g][m]), x1 = xor3(Jx[g][1], w1, w0);
+          const uint64_t n0 = xor3(Jy[g][0], w0, sn[g][m][0]), n1 = xor3(Jy[g][1], w1, sn[g][m][1]);
+          // a step beyond the range: the word below is the last plane's
+          const uint64_t u0 = xor3(Jz[g][0], w0, below[m][0] & live), u1 = xor3(Jz[g][1], w1, below[m][1] & live);
+          below[m][0] = w0;
+          below[m][1] = w1;
+          meas_add2(a[m], xor3(x0, n0, u0), maj3(x0, n0, u0), w0, xor3(x1, n1, u1), maj3(x1, n1, u1), w1);
+        }
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < SB; ++m) {
+      planes_add(big[m].e, a[m].e);
+      planes_add(big[m].m, a[m].m);
+    }
+  }
+  meas_finish<SB>(big, sh, red, nsys, sys0, ns, unit, cnt);
 }
 
 static __global__ void k_fill_zero(int *p, int n) {

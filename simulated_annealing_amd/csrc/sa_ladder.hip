@@ -579,25 +579,39 @@ void sa_detail::make_table(int kind, double T, double h, sa::sys_table &t, bool 
 
 void sa_detail::launch_measure(int kind, int L, int64_t N, const uint64_t *s, const uint64_t *jx, const uint64_t *jy,
                                const uint64_t *jz, int n, const int *dlist, sa::sys4 sel, int *cnt, hipStream_t st) {
-  const int all_n = 128 * n * sa::kMeasureCopies;
+  const int all_n = 128 * n * sa::measure_copies(n);
   hipLaunchKernelGGL(sa::k_fill_zero, dim3((all_n + 255) / 256), dim3(256), 0, st, cnt, all_n);
-  // cnt layout [copy][listed system][2][64] (the caller sums the copies); one block
-  // row per SB systems (4, or 1 when there are at most 4: more waves in flight for
-  // the few-system measurement of an exchange step).  A wave converts its bit-sliced
-  // counters (a 64x64 transpose per plane) after 16 site groups or at its end, so
-  // each wave gets at least 16 groups where possible (32 with one system per row,
-  // four of them loaded at a time): more blocks would only add conversions.
-  const int sb = n <= 4 ? 1 : 4;
-  const int yb = (n + sb - 1) / sb;
-  const int64_t want = std::max<int64_t>(1, (sb == 1 ? 4096 : 2048) / yb);
-  const int64_t per = sb == 1 ? 32 : 16;  // site groups per wave (one system per row: 4 in flight at a time)
-  const int64_t blocks = std::min<int64_t>((N + 256 * per - 1) / (256 * per), want);
-  dim3 grid((unsigned)blocks, yb);
+  // cnt layout [copy][listed system][2][64] (the caller sums the copies).  Two systems
+  // per block share its coupling loads; one when at most 4 are measured (the exchange
+  // step), for more waves in flight.  Steps per thread: as many as leave about 4 blocks
+  // per CU, so a small lattice is spread over many short walks (the kernel then takes
+  // one load round trip and one set of transposes) and a large one amortises both.
+  const int sb = n <= 4 ? 1 : 2;
+  const int nq = (n + sb - 1) / sb;
+  const bool pair = kind == SA_KIND_3D && L % 2 == 0 && N * 8 < ((int64_t)1 << 31);
+  const int64_t per_plane = kind == SA_KIND_3D ? (pair ? (N / L + 511) / 512 : (N / L + 255) / 256) : 1;
+  const int64_t length = kind == SA_KIND_3D ? L : (N + 255) / 256;  // steps of a single walk over everything
+  const int64_t want = std::max<int64_t>(1, 1024 / (per_plane * nq));  // walks per chunk
+  const int walk = (int)std::min<int64_t>(pair ? sa::kMeasWalk / 2 : sa::kMeasWalk,
+                                          std::max<int64_t>(1, (length + want - 1) / want));
+  const int64_t units = per_plane * ((length + walk - 1) / walk);
+  const dim3 grid((unsigned)(((units + 7) / 8) * 8 * nq));
+  if (pair) {
+    if (sb == 1)
+      hipLaunchKernelGGL((sa::k_measure3d_pair<1>), grid, dim3(256), 0, st, s, jx, jy, jz, L, N, n, dlist, sel, cnt,
+                         (int)units, (int)per_plane, walk);
+    else
+      hipLaunchKernelGGL((sa::k_measure3d_pair<2>), grid, dim3(256), 0, st, s, jx, jy, jz, L, N, n, dlist, sel, cnt,
+                         (int)units, (int)per_plane, walk);
+    return;
+  }
 #define SA_MEASURE(KINDV)                                                                                        \
   if (sb == 1)                                                                                                   \
-    hipLaunchKernelGGL((sa::k_measure<KINDV, 1>), grid, dim3(256), 0, st, s, jx, jy, jz, L, N, n, dlist, sel, cnt); \
+    hipLaunchKernelGGL((sa::k_measure<KINDV, 1>), grid, dim3(256), 0, st, s, jx, jy, jz, L, N, n, dlist, sel, cnt,  \
+                       (int)units, (int)per_plane, walk);                                                        \
   else                                                                                                           \
-    hipLaunchKernelGGL((sa::k_measure<KINDV, 4>), grid, dim3(256), 0, st, s, jx, jy, jz, L, N, n, dlist, sel, cnt);
+    hipLaunchKernelGGL((sa::k_measure<KINDV, 2>), grid, dim3(256), 0, st, s, jx, jy, jz, L, N, n, dlist, sel, cnt,  \
+                       (int)units, (int)per_plane, walk);
   if (kind == SA_KIND_3D) {
     SA_MEASURE(sa::KIND_3D)
   } else if (kind == SA_KIND_2D) {
@@ -662,7 +676,7 @@ namespace {
 // energies/magnetisations of `n` systems (list = nullptr: systems 0..n-1); results
 // land in cnt_h[(2*j)*64 ...] for the j-th listed system
 int measure_list(sa_ladder *l, const int *list, int n) {
-  const int cnt_n = 128 * n, all_n = cnt_n * sa::kMeasureCopies;
+  const int cnt_n = 128 * n, all_n = cnt_n * sa::measure_copies(n);
   // up to 4 listed systems travel as a kernel argument; more through device memory
   const int *dlist = nullptr;
   sa::sys4 sel{{-1, -1, -1, -1}};
@@ -696,7 +710,7 @@ int measure_list(sa_ladder *l, const int *list, int n) {
     SA_HIP_TRY(hipStreamSynchronize(l->stream));
   }
   // sum the copies into the first
-  for (int c = 1; c < sa::kMeasureCopies; ++c)
+  for (int c = 1; c < sa::measure_copies(n); ++c)
     for (int q = 0; q < cnt_n; ++q) l->cnt_h[q] += l->cnt_h[(size_t)c * cnt_n + q];
   return SA_OK;
 }

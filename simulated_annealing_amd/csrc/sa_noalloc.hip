@@ -29,7 +29,7 @@ __global__ void __launch_bounds__(128) k_noalloc_finish(const int *__restrict__ 
                                                         int32_t *__restrict__ E, int32_t *__restrict__ M) {
   const int j = blockIdx.x, q = threadIdx.x;  // q < 64: bond count of lane q; q >= 64: spin count of lane q-64
   int64_t sum = 0;
-  for (int c = 0; c < sa::kMeasureCopies; ++c) sum += cnt[((int64_t)c * nsys + j) * 128 + q];
+  for (int c = 0; c < sa::measure_copies(nsys); ++c) sum += cnt[((int64_t)c * nsys + j) * 128 + q];
   if (q < 64)
     E[j * 64 + q] = (int32_t)(2 * sum - bonds);
   else
