@@ -33,6 +33,9 @@ struct sa_ladder {
   int *cnt = nullptr;
   std::vector<sa::sys_table> htab;
   std::vector<char> fast;  // per system: symmetric tables, low levels always accept
+  std::vector<char> compact;  // per system: every table is compact (sys_table::base)
+  sa::sys_table *tab_seq = nullptr;  // tables of a run of sweeps at changing temperatures
+  int64_t tab_seq_cap = 0;
   int rng_mode = SA_RNG_REPLAY;
   uint64_t seed = 0, t = 0;
   sa::mt19937_64 eng{};
@@ -49,9 +52,18 @@ struct sa_ladder {
 };
 
 namespace sa_detail {
+// Sweeps of a 2D ladder with an even side held in LDS (sa_tile2d.hpp).  tile2d_sweeps:
+// sweeps of the next launch when `left` are to be done (0: this ladder takes the
+// half-sweep kernels; *bands: the launch needs the second spin array).  tile2d_launch:
+// that launch, `ns` sweeps from index t on; tab_step = tables per sweep in `tab`.
+int tile2d_sweeps(const sa_ladder *l, int64_t left, bool *bands);
+void tile2d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, bool fast, const uint64_t *words,
+                   uint64_t t, int64_t left, int ns);
 // acceptance thresholds of one temperature/field for a ladder of `kind`; fast =
 // the table qualifies for the symmetric low-levels-always kernels
 void make_table(int kind, double T, double h, sa::sys_table &tab, bool &fast, double *boltz_out);
+// every table of the kind is compact
+bool compact_table(int kind, const sa::sys_table &tab);
 // Measurement of n systems of s (nsys x N words; listed by dlist in device memory,
 // by sel for up to four, else systems 0..n-1): clears cnt (kMeasureCopies x n x 128
 // ints) with a fill kernel, then per copy, listed system and lane the satisfied

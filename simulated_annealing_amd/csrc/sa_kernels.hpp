@@ -40,12 +40,17 @@ enum { KIND_2P = 0, KIND_2D = 1, KIND_3D = 2 };
 
 // Acceptance thresholds of one system.  Table 0/1: bulk sites with spin bit 0/1;
 // table 2/3: open-x border sites (2p only).  Level c accepts iff g < thr[t][c]
-// or bit c of always[t] is set.
+// or bit c of always[t] is set.  base[t]: the table is compact -- levels below base[t]
+// always accept, the others (at most four) have non-increasing thresholds -- so the
+// accepted levels of a draw are 0 .. k-1 for one k; kNotCompact where it is not (a
+// negative temperature, say).  Open-x border sites always count the missing bond, so
+// their level 0 never occurs and counts as accepted.
 struct sys_table {
-  uint64_t thr[4][8];
+  uint64_t thr[4][8];  // thr[t][7] is 0 (no such level)
   uint32_t always[4];
-  uint32_t pad[4];
+  uint32_t base[4];
 };
+constexpr uint32_t kNotCompact = 255;
 
 struct sweep_args {
   uint64_t *s;

@@ -37,6 +37,7 @@ void free_all(sa_ladder *l) {
   if (l->s) (void)hipFree(l->s);
   if (l->jx) (void)hipFree(l->jx);  // jy, jz live in the same allocation
   if (l->tab) (void)hipFree(l->tab);
+  if (l->tab_seq) (void)hipFree(l->tab_seq);
   if (l->cnt) (void)hipFree(l->cnt);
   if (l->s_alt) (void)hipFree(l->s_alt);
   if (l->words_d) (void)hipFree(l->words_d);
@@ -283,6 +284,13 @@ void fill_table(sa::sys_table &t, int tb, const double *b, int nlev) {
     t.thr[tb][c] = th.value;
     if (th.always) t.always[tb] |= 1u << c;
   }
+  // compact form (sys_table::base); level 0 of the border tables never occurs
+  const int first = tb >= 2 ? 1 : 0;
+  int base = first;
+  while (base < nlev && ((t.always[tb] >> base) & 1u)) ++base;
+  bool ok = nlev - base <= 4 && (t.always[tb] >> base) == 0;
+  for (int c = base; c + 1 < nlev; ++c) ok = ok && t.thr[tb][c] >= t.thr[tb][c + 1];
+  t.base[tb] = ok ? (uint32_t)base : sa::kNotCompact;
 }
 
 }  // namespace
@@ -342,6 +350,7 @@ int sa_ladder_create(int kind, int L, int nsys, sa_ladder **out) {
   l->jz = l->jx + 2 * N;
   l->htab.assign(nsys, sa::sys_table{});
   l->fast.assign(nsys, 0);
+  l->compact.assign(nsys, 0);
   l->cnt_h.assign((size_t)128 * nsys * sa::kMeasureCopies, 0);
   l->eng.seed(5489u);
   *out = l;
@@ -555,6 +564,12 @@ int64_t sa_detail::ladder_bytes(int kind, int L, int nsys) {
          4 * 128 * nsys * sa::kMeasureCopies + 4 * nsys;
 }
 
+bool sa_detail::compact_table(int kind, const sa::sys_table &t) {
+  bool ok = true;
+  for (int tb = 0; tb < (kind == SA_KIND_2P ? 4 : 2); ++tb) ok = ok && t.base[tb] != sa::kNotCompact;
+  return ok;
+}
+
 void sa_detail::make_table(int kind, double T, double h, sa::sys_table &t, bool &fast, double *boltz_out) {
   double b[20];
   t = sa::sys_table{};
@@ -632,11 +647,48 @@ int sa_ladder_set_temperature(sa_ladder *l, int sys, double T, double h, double 
   sa_detail::make_table(l->kind, T, h, t, fast, boltz_out);
   l->htab[sys] = t;
   l->fast[sys] = fast;
+  l->compact[sys] = sa_detail::compact_table(l->kind, t);
   // stream-ordered: a pageable-source copy is staged before the call returns, so no
   // wait is needed; every later launch on the stream sees the new table
   SA_HIP_TRY(hipMemcpyAsync(l->tab + sys, &l->htab[sys], sizeof(sa::sys_table), hipMemcpyHostToDevice, l->stream));
   return SA_OK;
 }
+
+namespace {
+
+// the second spin array, allocated on first use; false (and no error kept) without memory
+bool have_alt(sa_ladder *l) {
+  if (l->s_alt) return true;
+  if (hipMalloc(&l->s_alt, (size_t)l->nsys * l->N * 8) == hipSuccess) return true;
+  l->s_alt = nullptr;
+  (void)hipGetLastError();
+  return false;
+}
+
+bool all_of(const std::vector<char> &v) {
+  return std::all_of(v.begin(), v.end(), [](char f) { return f != 0; });
+}
+
+// n sweeps at the ladder's own temperatures: words = the replay words of the first (N per sweep)
+int launch_sweeps(sa_ladder *l, const uint64_t *words, uint64_t t, int64_t n) {
+  for (int64_t k = 0; k < n;) {
+    bool bands = false;
+    const uint64_t *w = words ? words + k * l->N : nullptr;
+    int ns = all_of(l->compact) ? sa_detail::tile2d_sweeps(l, n - k, &bands) : 0;
+    if (ns > 0 && bands && !have_alt(l)) ns = 0;
+    if (ns > 0) {
+      sa_detail::tile2d_launch(l, l->tab, 0, all_of(l->fast), w, t + k, n - k, ns);
+      k += ns;
+    } else {
+      launch_sweep(l, w, t + k);
+      ++k;
+    }
+  }
+  SA_HIP_TRY(hipGetLastError());
+  return SA_OK;
+}
+
+}  // namespace
 
 int sa_ladder_sweep(sa_ladder *l, int nsweeps) {
   if (!l) return sa_fail(SA_ERR_ARG, "null ladder");
@@ -650,8 +702,8 @@ int sa_ladder_sweep(sa_ladder *l, int nsweeps) {
     }
   }
   if (l->rng_mode == SA_RNG_COUNTER) {
-    for (int k = 0; k < nsweeps; ++k) launch_sweep(l, nullptr, l->t + k);
-    SA_HIP_TRY(hipGetLastError());
+    const int rc = launch_sweeps(l, nullptr, l->t, nsweeps);
+    if (rc) return rc;
     l->t += nsweeps;
     return SA_OK;
   }
@@ -662,8 +714,8 @@ int sa_ladder_sweep(sa_ladder *l, int nsweeps) {
     const int64_t n = std::min<int64_t>(per_chunk, nsweeps - done);
     l->eng.fill(l->words_h, n * l->N);
     SA_HIP_TRY(hipMemcpyAsync(l->words_d, l->words_h, n * l->N * 8, hipMemcpyHostToDevice, l->stream));
-    for (int64_t k = 0; k < n; ++k) launch_sweep(l, l->words_d + k * l->N, l->t + done + k);
-    SA_HIP_TRY(hipGetLastError());
+    rc = launch_sweeps(l, l->words_d, l->t + done, n);
+    if (rc) return rc;
     SA_HIP_TRY(hipStreamSynchronize(l->stream));
     done += n;
   }
