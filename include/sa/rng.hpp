@@ -170,7 +170,13 @@ struct threshold {
 inline threshold accept_threshold(double b) {
   if (!(b > 0.0)) return {0, false};
   if (b > std::nextafter(1.0, 0.0)) return {0, true};
-  uint64_t lo = 0, hi = ~0ULL;  // canonical64(hi) = 1 - 2^-53 >= b
+  // the answer lies within one rounding step (2^11 at most) of b*2^64, which ldexp gives
+  // exactly: 13 bisection steps instead of 64 (an anneal makes new tables every sweep)
+  const double B = std::ldexp(b, 64);
+  const uint64_t mid0 = B < 18446744073709549568.0 ? (uint64_t)B : ~0ULL - 2047;
+  uint64_t lo = mid0 > 4096 ? mid0 - 4096 : 0, hi = mid0 < ~0ULL - 4096 ? mid0 + 4096 : ~0ULL;
+  if (lo > 0 && canonical64(lo - 1) >= b) lo = 0;
+  if (!(canonical64(hi) >= b)) hi = ~0ULL;  // canonical64(~0) = 1 - 2^-53 >= b
   while (lo < hi) {
     const uint64_t mid = lo + ((hi - lo) >> 1);
     if (canonical64(mid) >= b) hi = mid; else lo = mid + 1;

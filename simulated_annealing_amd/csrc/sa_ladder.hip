@@ -277,6 +277,12 @@ void launch_sweep(sa_ladder *l, const uint64_t *words, uint64_t t) {
 
 // thresholds of one Boltzmann table into sys_table t (levels 0..nb)
 void fill_table(sa::sys_table &t, int tb, const double *b, int nlev) {
+  if (tb == 1 && std::memcmp(b, b - nlev, sizeof(double) * nlev) == 0) {  // no field: as table 0
+    std::memcpy(t.thr[1], t.thr[0], sizeof t.thr[0]);
+    t.always[1] = t.always[0];
+    t.base[1] = t.base[0];
+    return;
+  }
   t.always[tb] = 0;
   for (int c = 0; c < 8; ++c) t.thr[tb][c] = 0;
   for (int c = 0; c < nlev; ++c) {
@@ -777,15 +783,83 @@ void counts_to_EM(const sa_ladder *l, int j, int32_t *E, int32_t *M) {
 
 }  // namespace
 
+namespace {
+
+// Up to `left` sweeps at the temperatures T (nsys per sweep) in launches of several sweeps
+// where the ladder takes the LDS-resident 2D sweeps: their tables are uploaded together.
+// *done = sweeps done, 0 when the ladder takes one sweep per launch (nothing enqueued).
+// One table upload and launch per sweep took 11 us a sweep at 2D L=64 where the sweep
+// itself takes 2.
+int anneal_run_2d(sa_ladder *l, const double *T, int64_t left, double h, int64_t *done) {
+  *done = 0;
+  bool bands = false;
+  if (l->rng_mode != SA_RNG_COUNTER || left < 2 || sa_detail::tile2d_sweeps(l, left, &bands) < 2) return SA_OK;
+  constexpr int64_t kTables = 4096;  // tables per upload (1.1 MB)
+  const int64_t n = std::min<int64_t>(left, std::max<int64_t>(1, kTables / l->nsys));
+  if (n < 2 || (bands && !have_alt(l))) return SA_OK;
+  std::vector<sa::sys_table> tabs((size_t)(n * l->nsys));
+  bool fast = true;
+  for (int64_t q = 0; q < n * l->nsys; ++q) {
+    bool f = false;
+    sa_detail::make_table(l->kind, T[q], h, tabs[q], f, nullptr);
+    fast = fast && f;
+    if (!sa_detail::compact_table(l->kind, tabs[q])) return SA_OK;
+    if (q >= (n - 1) * l->nsys) {  // the ladder is left at the last sweep's temperatures
+      const size_t j = (size_t)(q - (n - 1) * l->nsys);
+      l->htab[j] = tabs[q];
+      l->fast[j] = f;
+      l->compact[j] = 1;
+    }
+  }
+  if (l->tab_seq_cap < n * l->nsys) {
+    SA_HIP_TRY(hipStreamSynchronize(l->stream));  // earlier sweeps may still read the old array
+    if (l->tab_seq) (void)hipFree(l->tab_seq);
+    l->tab_seq = nullptr;
+    l->tab_seq_cap = 0;
+    if (hipMalloc(&l->tab_seq, sizeof(sa::sys_table) * n * l->nsys) != hipSuccess) {
+      l->tab_seq = nullptr;
+      (void)hipGetLastError();
+      return SA_OK;  // one table at a time, in the ladder's own array
+    }
+    l->tab_seq_cap = n * l->nsys;
+  }
+  SA_HIP_TRY(hipMemcpyAsync(l->tab_seq, tabs.data(), sizeof(sa::sys_table) * n * l->nsys, hipMemcpyHostToDevice,
+                            l->stream));
+  SA_HIP_TRY(hipMemcpyAsync(l->tab, tabs.data() + (n - 1) * l->nsys, sizeof(sa::sys_table) * l->nsys,
+                            hipMemcpyHostToDevice, l->stream));
+  for (int64_t k = 0; k < n;) {
+    const int ns = sa_detail::tile2d_sweeps(l, n - k, &bands);
+    sa_detail::tile2d_launch(l, l->tab_seq + k * l->nsys, l->nsys, fast, nullptr, l->t + k, n - k, ns);
+    k += ns;
+  }
+  SA_HIP_TRY(hipGetLastError());
+  l->t += n;
+  *done = n;
+  return SA_OK;
+}
+
+}  // namespace
+
 int sa_ladder_anneal(sa_ladder *l, const double *T, int nsweeps, double h) {
   if (!l || (!T && nsweeps > 0) || nsweeps < 0) return sa_fail(SA_ERR_ARG, "bad argument");
-  for (int t = 0; t < nsweeps; ++t) {
+  bool runs = true;
+  for (int t = 0; t < nsweeps;) {
+    int rc = SA_OK;
+    if (runs) {
+      int64_t done = 0;
+      rc = anneal_run_2d(l, T + (int64_t)t * l->nsys, nsweeps - t, h, &done);
+      if (rc) return rc;
+      t += (int)done;
+      runs = done > 0;
+      continue;
+    }
     for (int j = 0; j < l->nsys; ++j) {
-      const int rc = sa_ladder_set_temperature(l, j, T[(int64_t)t * l->nsys + j], h, nullptr);
+      rc = sa_ladder_set_temperature(l, j, T[(int64_t)t * l->nsys + j], h, nullptr);
       if (rc) return rc;
     }
-    const int rc = sa_ladder_sweep(l, 1);
+    rc = sa_ladder_sweep(l, 1);
     if (rc) return rc;
+    ++t;
   }
   return SA_OK;
 }

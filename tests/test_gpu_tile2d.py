@@ -54,3 +54,28 @@ def test_tile2d_many_systems(orc, L, nsys):
 @pytest.mark.parametrize("T,h", [(0.7, 5.0), (-1.0, 0.0), (1e-3, 0.0), (1e9, 0.0), (0.9, -0.4), (0.9, 2.0)])
 def test_tile2d_table_forms(orc, kind, T, h):
     compare(orc, kind, 22, 2, 4, sa.RNG_COUNTER, [T, 1.0], [h, 0.0])
+
+
+@pytest.mark.parametrize("kind,L,nsys", [(sa.KIND_2D, 20, 2), (sa.KIND_2P, 18, 1), (sa.KIND_2D, 96, 2)])
+@pytest.mark.parametrize("h", [0.0, 0.3])
+@pytest.mark.parametrize("odd_one", [None, -2.0])
+def test_anneal_runs_match_oracle(orc, kind, L, nsys, h, odd_one):
+    """several sweeps per launch at changing temperatures; a table that is not compact
+    (negative temperature) in the schedule sends the call to one sweep per launch"""
+    nsw, seed = 9, 5 * L
+    Ts = np.linspace(2.5, 0.3, nsw * nsys).reshape(nsw, nsys)
+    if odd_one is not None:
+        Ts[5, 0] = odd_one
+    lad = sa.Ladder(kind, L, nsys)
+    lad.set_rng(sa.RNG_COUNTER)
+    lad.seed_like_main(seed)
+    lad.anneal(Ts, h)
+    lad.sweep(2)  # at the last temperatures
+    jx, jy, jz, s0, _ = orc.init_system(kind, L, seed)
+    for j in range(nsys):
+        s = s0.copy()
+        for t in range(nsw + 2):
+            orc.sweep(kind, L, s, jx, jy, jz, orc.boltz(kind, Ts[min(t, nsw - 1), j], h), orc.counter_words(kind, L, seed, t))
+        assert (lad.spins(j) == s).all(), j
+    assert lad.sweep_index == nsw + 2
+    lad.close()
