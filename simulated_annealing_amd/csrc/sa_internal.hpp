@@ -29,6 +29,8 @@ struct sa_ladder {
   hipStream_t stream = nullptr;
   uint64_t *s = nullptr, *jx = nullptr, *jy = nullptr, *jz = nullptr;
   uint64_t *s_alt = nullptr;  // second spin array of the fused 3D sweep (ping-pong)
+  uint64_t *jt = nullptr;  // 3D: the couplings with z fastest (sa_tile3d.hpp), made when first needed
+  bool jt_current = false;  // ... from the present couplings
   sa::sys_table *tab = nullptr;
   int *cnt = nullptr;
   std::vector<sa::sys_table> htab;
@@ -59,6 +61,11 @@ namespace sa_detail {
 int tile2d_sweeps(const sa_ladder *l, int64_t left, bool *bands);
 void tile2d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, bool fast, const uint64_t *words,
                    uint64_t t, int64_t left, int ns);
+// The same for 3D ladders with an even side (sa_tile3d.hpp); *us: the modelled time per sweep.
+int tile3d_sweeps(const sa_ladder *l, int64_t left, bool *second, double *us);
+bool tile3d_couplings(sa_ladder *l);
+void tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, bool fast, const uint64_t *words,
+                   uint64_t t, int64_t left);
 // acceptance thresholds of one temperature/field for a ladder of `kind`; fast =
 // the table qualifies for the symmetric low-levels-always kernels
 void make_table(int kind, double T, double h, sa::sys_table &tab, bool &fast, double *boltz_out);

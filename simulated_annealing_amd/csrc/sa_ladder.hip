@@ -36,6 +36,7 @@ int bonds_per_site(int kind) { return kind == SA_KIND_3D ? 3 : 2; }
 void free_all(sa_ladder *l) {
   if (l->s) (void)hipFree(l->s);
   if (l->jx) (void)hipFree(l->jx);  // jy, jz live in the same allocation
+  if (l->jt) (void)hipFree(l->jt);
   if (l->tab) (void)hipFree(l->tab);
   if (l->tab_seq) (void)hipFree(l->tab_seq);
   if (l->cnt) (void)hipFree(l->cnt);
@@ -209,6 +210,29 @@ fused_cfg pick_fused(const sa_ladder *l) {
     }
   }
   return c;
+}
+
+bool all_of(const std::vector<char> &v) {
+  return std::all_of(v.begin(), v.end(), [](char f) { return f != 0; });
+}
+
+// Sweeps of the next LDS-resident launch (sa_tile2d.hpp, sa_tile3d.hpp) when `left` are to be
+// done, 0 when the ladder takes another kernel; *second: the launch writes the other array.
+// 3D: the fused walk's time is its z walk's latency, about 1 us per plane (2.1 with general
+// tables), until the ladder fills the chip; the tiles' grows with the words.  Measured, us
+// per sweep, walk / tiles: L=64 x4 33 / 15, x16 95 / 43, x32 67 / 78; L=128 x1 83 / 47, x4 133 / 108,
+// x8 196 / 219; with a field L=64 x32 198 / 90, L=96 x16 264 / 195, L=128 x16 397 / 453.  Without a
+// fused walk (sides it does not divide): half-sweep launches, L=200 370 / 248, L=256 660 / 554.
+int tile_sweeps(const sa_ladder *l, int64_t left, bool *second) {
+  if (l->sys_per_thread || !all_of(l->compact)) return 0;
+  if (l->kind != SA_KIND_3D) return sa_detail::tile2d_sweeps(l, left, second);
+  if (l->sweep3d_kernel || l->rows_per_tile || l->xcd_map >= 0) return 0;
+  double us = 0;
+  const int ns = sa_detail::tile3d_sweeps(l, left, second, &us);
+  if (!ns) return 0;
+  const bool walk = pick_fused(l).th > 0;
+  const double limit = walk ? (all_of(l->fast) ? 1.0 : 2.1) * l->L : 12e-6 * ((int64_t)1 << 25);
+  return us < limit ? ns : 0;
 }
 
 bool use_fused(const sa_ladder *l) {
@@ -434,6 +458,7 @@ int sa_ladder_set_engine(sa_ladder *l, const uint64_t state[313]) {
 int sa_ladder_set_couplings(sa_ladder *l, const uint64_t *jx, const uint64_t *jy, const uint64_t *jz) {
   if (!l || !jx || !jy || (l->kind == SA_KIND_3D && !jz)) return sa_fail(SA_ERR_ARG, "null argument");
   const size_t bytes = l->N * 8;
+  l->jt_current = false;
   SA_HIP_TRY(hipMemcpyAsync(l->jx, jx, bytes, hipMemcpyHostToDevice, l->stream));
   SA_HIP_TRY(hipMemcpyAsync(l->jy, jy, bytes, hipMemcpyHostToDevice, l->stream));
   if (l->kind == SA_KIND_3D) SA_HIP_TRY(hipMemcpyAsync(l->jz, jz, bytes, hipMemcpyHostToDevice, l->stream));
@@ -671,19 +696,17 @@ bool have_alt(sa_ladder *l) {
   return false;
 }
 
-bool all_of(const std::vector<char> &v) {
-  return std::all_of(v.begin(), v.end(), [](char f) { return f != 0; });
-}
-
 // n sweeps at the ladder's own temperatures: words = the replay words of the first (N per sweep)
 int launch_sweeps(sa_ladder *l, const uint64_t *words, uint64_t t, int64_t n) {
   for (int64_t k = 0; k < n;) {
-    bool bands = false;
+    bool second = false;  // the launch writes the other spin array
     const uint64_t *w = words ? words + k * l->N : nullptr;
-    int ns = all_of(l->compact) ? sa_detail::tile2d_sweeps(l, n - k, &bands) : 0;
-    if (ns > 0 && bands && !have_alt(l)) ns = 0;
+    int ns = tile_sweeps(l, n - k, &second);
+    if (ns > 0 && second && !have_alt(l)) ns = 0;
+    if (ns > 0 && l->kind == SA_KIND_3D && !sa_detail::tile3d_couplings(l)) ns = 0;
     if (ns > 0) {
-      sa_detail::tile2d_launch(l, l->tab, 0, all_of(l->fast), w, t + k, n - k, ns);
+      if (l->kind == SA_KIND_3D) sa_detail::tile3d_launch(l, l->tab, 0, all_of(l->fast), w, t + k, n - k);
+      else sa_detail::tile2d_launch(l, l->tab, 0, all_of(l->fast), w, t + k, n - k, ns);
       k += ns;
     } else {
       launch_sweep(l, w, t + k);
@@ -700,7 +723,8 @@ int sa_ladder_sweep(sa_ladder *l, int nsweeps) {
   if (!l) return sa_fail(SA_ERR_ARG, "null ladder");
   if (nsweeps < 0) return sa_fail(SA_ERR_ARG, "negative sweep count");
   if (nsweeps == 0) return SA_OK;
-  if (use_fused(l) && !l->s_alt) {
+  bool second = false;
+  if (use_fused(l) && !l->s_alt && !tile_sweeps(l, nsweeps, &second)) {
     const hipError_t e = hipMalloc(&l->s_alt, (size_t)l->nsys * l->N * 8);
     if (e != hipSuccess) {
       l->s_alt = nullptr;
@@ -785,18 +809,19 @@ void counts_to_EM(const sa_ladder *l, int j, int32_t *E, int32_t *M) {
 
 namespace {
 
-// Up to `left` sweeps at the temperatures T (nsys per sweep) in launches of several sweeps
-// where the ladder takes the LDS-resident 2D sweeps: their tables are uploaded together.
+// Up to `left` sweeps at the temperatures T (nsys per sweep) where the ladder takes the
+// LDS-resident sweeps: their tables are uploaded together and several sweeps share a launch.
 // *done = sweeps done, 0 when the ladder takes one sweep per launch (nothing enqueued).
 // One table upload and launch per sweep took 11 us a sweep at 2D L=64 where the sweep
 // itself takes 2.
-int anneal_run_2d(sa_ladder *l, const double *T, int64_t left, double h, int64_t *done) {
+int anneal_run(sa_ladder *l, const double *T, int64_t left, double h, int64_t *done) {
   *done = 0;
-  bool bands = false;
-  if (l->rng_mode != SA_RNG_COUNTER || left < 2 || sa_detail::tile2d_sweeps(l, left, &bands) < 2) return SA_OK;
+  bool second = false;
+  if (l->rng_mode != SA_RNG_COUNTER || left < 2 || !tile_sweeps(l, left, &second)) return SA_OK;
   constexpr int64_t kTables = 4096;  // tables per upload (1.1 MB)
   const int64_t n = std::min<int64_t>(left, std::max<int64_t>(1, kTables / l->nsys));
-  if (n < 2 || (bands && !have_alt(l))) return SA_OK;
+  if (n < 2 || (second && !have_alt(l))) return SA_OK;
+  if (l->kind == SA_KIND_3D && !sa_detail::tile3d_couplings(l)) return SA_OK;
   std::vector<sa::sys_table> tabs((size_t)(n * l->nsys));
   bool fast = true;
   for (int64_t q = 0; q < n * l->nsys; ++q) {
@@ -827,9 +852,18 @@ int anneal_run_2d(sa_ladder *l, const double *T, int64_t left, double h, int64_t
                             l->stream));
   SA_HIP_TRY(hipMemcpyAsync(l->tab, tabs.data() + (n - 1) * l->nsys, sizeof(sa::sys_table) * l->nsys,
                             hipMemcpyHostToDevice, l->stream));
-  for (int64_t k = 0; k < n;) {
-    const int ns = sa_detail::tile2d_sweeps(l, n - k, &bands);
-    sa_detail::tile2d_launch(l, l->tab_seq + k * l->nsys, l->nsys, fast, nullptr, l->t + k, n - k, ns);
+  for (int64_t k = 0; k < n;) {  // the same configuration as above until the last, shorter launch
+    int ns;
+    double us = 0;
+    if (l->kind == SA_KIND_3D) {
+      ns = sa_detail::tile3d_sweeps(l, n - k, &second, &us);
+      if (second && !have_alt(l)) return sa_fail(SA_ERR_NOMEM, "second spin array");
+      sa_detail::tile3d_launch(l, l->tab_seq + k * l->nsys, l->nsys, fast, nullptr, l->t + k, n - k);
+    } else {
+      ns = sa_detail::tile2d_sweeps(l, n - k, &second);
+      if (second && !have_alt(l)) return sa_fail(SA_ERR_NOMEM, "second spin array");
+      sa_detail::tile2d_launch(l, l->tab_seq + k * l->nsys, l->nsys, fast, nullptr, l->t + k, n - k, ns);
+    }
     k += ns;
   }
   SA_HIP_TRY(hipGetLastError());
@@ -847,7 +881,7 @@ int sa_ladder_anneal(sa_ladder *l, const double *T, int nsweeps, double h) {
     int rc = SA_OK;
     if (runs) {
       int64_t done = 0;
-      rc = anneal_run_2d(l, T + (int64_t)t * l->nsys, nsweeps - t, h, &done);
+      rc = anneal_run(l, T + (int64_t)t * l->nsys, nsweeps - t, h, &done);
       if (rc) return rc;
       t += (int)done;
       runs = done > 0;
@@ -926,12 +960,13 @@ int sa_ladder_set_tuning(sa_ladder *l, int key, int value) {
 
 int sa_ladder_get_tuning(const sa_ladder *l, int key, int *value) {
   if (!l || !value) return sa_fail(SA_ERR_ARG, "null argument");
+  bool second = false;
   const bool fused = use_fused(l);
   const fused_cfg c = fused ? pick_fused(l) : fused_cfg{0, 0, 0};
   switch (key) {
     case SA_TUNE_SYS_PER_THREAD: *value = fused ? c.mb : pick_mb(l); return SA_OK;
     case SA_TUNE_SWEEP3D_KERNEL:
-      *value = l->kind != SA_KIND_3D ? 0 : (fused ? 2 : use_zscan(l) ? 3 : 1);
+      *value = l->kind != SA_KIND_3D ? 0 : tile_sweeps(l, 1, &second) ? 4 : (fused ? 2 : use_zscan(l) ? 3 : 1);
       return SA_OK;
     case SA_TUNE_ROWS_PER_TILE: *value = c.th; return SA_OK;
     case SA_TUNE_XCD_MAP: *value = c.xcd; return SA_OK;

@@ -1,0 +1,185 @@
+// sa_tile3d.hip -- choice and launch of the 3D tile sweep (sa_tile3d.hpp).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+
+#include "sa_internal.hpp"
+#include "sa_tile3d.hpp"
+
+namespace {
+
+constexpr size_t kMaxLds = 160 * 1024;
+
+struct tile_cfg {
+  bool whole;
+  int tx, ty, S, G, C, lg, lp, threads, ns, w0, w1;
+};
+
+size_t lds_bytes(const tile_cfg &c, int L) {
+  const int W = c.whole ? L : c.tx + 4, H = c.whole ? L : c.ty + 4;
+  return (size_t)W * H * c.lp * 8;
+}
+
+// The tile of the next launch: the one with the least modelled time per sweep, in us.
+// Fitted to 60 measured shapes (3D L 8..128, 1..32 systems), within 25%: a launch with its
+// load and store, a wave's worth of columns, and the tiles' reads and writes at 8 TB/s;
+// four-plane segments need half the waves but take about twice as long each.  A tile's work grows with
+// its waves, its overhead with its halo: one L=64 system takes 4 x 4 columns (256 tiles, 7.2
+// us per sweep; 8 x 8: 11.0), 16 systems of L=32 16 x 4 (7.4; 4 x 4: 10.0, 16 x 8: 8.6).
+tile_cfg pick(const sa_ladder *l, int64_t left, double &cost) {
+  tile_cfg best{};
+  cost = 1e30;
+  const int L = l->L;
+  if (l->kind != SA_KIND_3D || (L & 1) || L < 4 || L > 256) return best;
+  const bool general = std::any_of(l->fast.begin(), l->fast.end(), [](char f) { return !f; });
+  auto consider = [&](bool whole, int tx, int ty, int S) {
+    tile_cfg c{};
+    c.whole = whole;
+    c.tx = whole ? L : tx;
+    c.ty = whole ? L : ty;
+    c.S = S;
+    c.G = (L + S - 1) / S;
+    if (c.G < 2 || c.G > 64) return;
+    c.lg = 1;
+    while ((1 << c.lg) < c.G) ++c.lg;
+    c.C = 64 >> c.lg;
+    const int W = whole ? L : tx + 4, H = whole ? L : ty + 4;
+    c.lp = L % 4 == 0 ? L + 2 : L;
+    if (lds_bytes(c, L) > kMaxLds) return;
+    const int col0 = whole ? L * L / 2 : (tx / 2 + 1) * (ty + 2), col1 = whole ? col0 : tx / 2 * ty;
+    c.w0 = (col0 + c.C - 1) / c.C;
+    c.w1 = (col1 + c.C - 1) / c.C;
+    c.threads = std::max(std::min(16, c.w0) * 64, (H * W / 2 + 63) / 64 * 64);
+    if (c.threads > 1024) return;
+    c.ns = whole ? (int)std::min<int64_t>(left, 64) : 1;
+    const int64_t tiles = whole ? 1 : (int64_t)((L + tx - 1) / tx) * ((L + ty - 1) / ty);
+    if (tiles * l->nsys >= (int64_t)1 << 24) return;
+    const double per_cu = std::ceil((double)tiles * l->nsys / 256);
+    const double wave = S == 2 ? (general ? 0.195 : 0.13) : (general ? 0.29 : 0.25);
+    const double words = (double)l->nsys * l->N, amp = (double)(W * H) / (c.tx * c.ty);
+    const double t = ((S == 2 ? 4.6 : 6.3) + words * 8 * (amp + 1) / 8e6) / c.ns + per_cu * (c.w0 + c.w1) * wave;
+    if (t < cost) {
+      cost = t;
+      best = c;
+    }
+  };
+  for (int S : {2, 4}) {
+    if (S == 2) consider(true, L, L, S);
+    for (int tx : {4, 8, 16, 32})
+      for (int ty : {4, 8, 16, 32})
+        if (tx <= L && ty <= L) consider(false, tx, ty, S);
+  }
+  return best;
+}
+
+template <bool COUNTER, bool FAST, int S>
+void launch(const sa::tile3d_args &t, const tile_cfg &c, hipStream_t st) {
+  const dim3 grid((unsigned)((t.ntx * t.nty * t.a.nsys + 7) / 8 * 8));
+  const size_t lds = lds_bytes(c, t.a.L);
+  auto go = [&](auto whole, auto one) {
+    constexpr bool WH = decltype(whole)::value, ON = decltype(one)::value;
+    static const hipError_t more = hipFuncSetAttribute((const void *)sa::k_tile3d<COUNTER, FAST, S, WH, ON>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
+    (void)more;  // more than 64 KB of dynamic LDS
+    hipLaunchKernelGGL((sa::k_tile3d<COUNTER, FAST, S, WH, ON>), grid, dim3(c.threads), lds, st, t);
+  };
+  const bool one = c.w0 * 64 <= c.threads;
+  if constexpr (S == 2) {  // the kept couplings fit the registers
+    if (one) return c.whole ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
+  }
+  c.whole ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
+}
+
+// in (rows x cols) to out (cols x rows), 32 x 32 words at a time; blockIdx.z: the array
+__global__ void __launch_bounds__(256) k_transpose(const uint64_t *__restrict__ in, uint64_t *__restrict__ out, int rows,
+                                                   int cols) {
+  __shared__ uint64_t tile[32][33];
+  const int64_t base = (int64_t)blockIdx.z * rows * cols;
+  const int c0 = (int)blockIdx.x * 32, r0 = (int)blockIdx.y * 32, i = (int)threadIdx.x & 31, j0 = (int)threadIdx.x >> 5;
+  for (int j = j0; j < 32; j += 8)
+    if (r0 + j < rows && c0 + i < cols) tile[j][i] = in[base + (int64_t)(r0 + j) * cols + c0 + i];
+  __syncthreads();
+  for (int j = j0; j < 32; j += 8)
+    if (c0 + j < cols && r0 + i < rows) out[base + (int64_t)(c0 + j) * rows + r0 + i] = tile[i][j];
+}
+
+}  // namespace
+
+// the ladder's couplings with z fastest, on its stream; false without memory
+bool sa_detail::tile3d_couplings(sa_ladder *l) {
+  if (!l->jt && hipMalloc(&l->jt, (size_t)3 * l->N * 8) != hipSuccess) {
+    l->jt = nullptr;
+    (void)hipGetLastError();
+    return false;
+  }
+  if (l->jt_current) return true;
+  const int L2 = l->L * l->L;
+  hipLaunchKernelGGL(k_transpose, dim3((unsigned)((L2 + 31) / 32), (unsigned)((l->L + 31) / 32), 3), dim3(256), 0,
+                     l->stream, l->jx, l->jt, l->L, L2);
+  l->jt_current = true;
+  return true;
+}
+
+int sa_detail::tile3d_sweeps(const sa_ladder *l, int64_t left, bool *second, double *us) {
+  double cost = 0;
+  const tile_cfg c = pick(l, left, cost);
+  *second = c.S > 0 && !c.whole;
+  *us = cost;
+  return c.S > 0 ? c.ns : 0;
+}
+
+void sa_detail::tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, bool fast, const uint64_t *words,
+                              uint64_t t, int64_t left) {
+  double cost = 0;
+  const tile_cfg c = pick(l, left, cost);
+  sa::tile3d_args a{};
+  a.a.s = l->s;
+  a.a.jx = l->jx;
+  a.a.jy = l->jy;
+  a.a.jz = l->jz;
+  a.a.tab = tab;
+  a.a.words = words;
+  a.a.seed = l->seed;
+  a.a.sweep = t;
+  a.a.N = l->N;
+  a.a.L = l->L;
+  a.a.nsys = l->nsys;
+  a.out = c.whole ? l->s : l->s_alt;
+  a.tx = c.tx;
+  a.ty = c.ty;
+  a.ntx = (l->L + c.tx - 1) / c.tx;
+  a.nty = (l->L + c.ty - 1) / c.ty;
+  a.G = c.G;
+  a.C = c.C;
+  a.lg = c.lg;
+  a.lp = c.lp;
+  a.jxt = l->jt;
+  a.jyt = l->jt + l->N;
+  a.jzt = l->jt + 2 * l->N;
+  a.chunks0 = c.w0;
+  a.chunks1 = c.w1;
+  auto recip = [](int d) { return ((1 << 20) + d - 1) / d; };
+  const int W = c.whole ? l->L : c.tx + 4, H = c.whole ? l->L : c.ty + 4;
+  a.recip_pairs = recip(W / 2 * H);
+  a.recip_hw = recip(W / 2);
+  a.recip_ntx = recip(a.ntx);
+  a.recip_per = (uint32_t)((((uint64_t)1 << 32) + a.ntx * a.nty - 1) / (a.ntx * a.nty));  // not used with one tile
+  a.zstep = c.threads / (W / 2 * H);
+  a.recip_n0 = recip(c.whole ? l->L / 2 : c.tx / 2 + 1);
+  a.recip_n1 = recip(c.whole ? l->L / 2 : c.tx / 2);
+  a.ns = c.ns;
+  a.tab_step = tab_step;
+  const bool counter = l->rng_mode == SA_RNG_COUNTER;
+#define SA_T3(CO, FA)                                                   \
+  if (counter == CO && fast == FA) {                                    \
+    if (c.S == 2) launch<CO, FA, 2>(a, c, l->stream);                   \
+    else launch<CO, FA, 4>(a, c, l->stream);                            \
+  }
+  SA_T3(true, true)
+  SA_T3(true, false)
+  SA_T3(false, true)
+  SA_T3(false, false)
+#undef SA_T3
+  if (!c.whole) std::swap(l->s, l->s_alt);
+}
