@@ -229,7 +229,9 @@ int tile_sweeps(const sa_ladder *l, int64_t left, bool *second) {
   if (l->sweep3d_kernel || l->rows_per_tile || l->xcd_map >= 0) return 0;
   double us = 0;
   const int ns = sa_detail::tile3d_sweeps(l, left, second, &us);
-  if (!ns) return 0;
+  // odd sides: one lane per column with a skewed walk otherwise, slower at every size (us per
+  // sweep, lanes / tiles: L=27 x12 50 / 11, L=63 x1 134 / 12, x16 145 / 45, L=127 x16 840 / 425)
+  if (!ns || (l->L & 1)) return ns;
   const bool walk = pick_fused(l).th > 0;
   const double limit = walk ? (all_of(l->fast) ? 1.0 : 2.1) * l->L : 12e-6 * ((int64_t)1 << 25);
   return us < limit ? ns : 0;

@@ -18,7 +18,7 @@ struct tile_cfg {
 
 size_t lds_bytes(const tile_cfg &c, int L) {
   const int W = c.whole ? L : c.tx + 4, H = c.whole ? L : c.ty + 4;
-  return (size_t)W * H * c.lp * 8;
+  return ((size_t)W * H * c.lp + (L & 1 ? sa::odd_list_words(W, H) : 0)) * 8;
 }
 
 // The tile of the next launch: the one with the least modelled time per sweep, in us.
@@ -31,7 +31,8 @@ tile_cfg pick(const sa_ladder *l, int64_t left, double &cost) {
   tile_cfg best{};
   cost = 1e30;
   const int L = l->L;
-  if (l->kind != SA_KIND_3D || (L & 1) || L < 4 || L > 256) return best;
+  if (l->kind != SA_KIND_3D || L > 256) return best;
+  const bool odd = L & 1;
   const bool general = std::any_of(l->fast.begin(), l->fast.end(), [](char f) { return !f; });
   auto consider = [&](bool whole, int tx, int ty, int S) {
     tile_cfg c{};
@@ -45,12 +46,14 @@ tile_cfg pick(const sa_ladder *l, int64_t left, double &cost) {
     while ((1 << c.lg) < c.G) ++c.lg;
     c.C = 64 >> c.lg;
     const int W = whole ? L : tx + 4, H = whole ? L : ty + 4;
-    c.lp = L % 4 == 0 ? L + 2 : L;
+    if (odd && !whole && (W > L || H > L)) return;
+    c.lp = sa::column_stride(L) % 4 == 0 ? sa::column_stride(L) + 2 : sa::column_stride(L);
     if (lds_bytes(c, L) > kMaxLds) return;
-    const int col0 = whole ? L * L / 2 : (tx / 2 + 1) * (ty + 2), col1 = whole ? col0 : tx / 2 * ty;
+    // odd sides: one more column per row at most
+    const int col0 = whole ? (L * L + 1) / 2 : (tx / 2 + 1) * (ty + 2), col1 = whole ? L * L / 2 : tx / 2 * ty;
     c.w0 = (col0 + c.C - 1) / c.C;
     c.w1 = (col1 + c.C - 1) / c.C;
-    c.threads = std::max(std::min(16, c.w0) * 64, (H * W / 2 + 63) / 64 * 64);
+    c.threads = std::max(std::min(16, c.w0) * 64, (H * W / (odd ? 1 : 2) + 63) / 64 * 64);
     if (c.threads > 1024) return;
     c.ns = whole ? (int)std::min<int64_t>(left, 64) : 1;
     const int64_t tiles = whole ? 1 : (int64_t)((L + tx - 1) / tx) * ((L + ty - 1) / ty);
@@ -58,7 +61,8 @@ tile_cfg pick(const sa_ladder *l, int64_t left, double &cost) {
     const double per_cu = std::ceil((double)tiles * l->nsys / 256);
     const double wave = S == 2 ? (general ? 0.195 : 0.13) : (general ? 0.29 : 0.25);
     const double words = (double)l->nsys * l->N, amp = (double)(W * H) / (c.tx * c.ty);
-    const double t = ((S == 2 ? 4.6 : 6.3) + words * 8 * (amp + 1) / 8e6) / c.ns + per_cu * (c.w0 + c.w1) * wave;
+    // odd sides: up to three more stages
+    const double t = ((S == 2 ? 4.6 : 6.3) + (odd ? 2.5 : 0) + words * 8 * (amp + 1) / 8e6) / c.ns + per_cu * (c.w0 + c.w1) * wave + (odd && whole ? 2.5 : 0);
     if (t < cost) {
       cost = t;
       best = c;
@@ -84,6 +88,16 @@ void launch(const sa::tile3d_args &t, const tile_cfg &c, hipStream_t st) {
     (void)more;  // more than 64 KB of dynamic LDS
     hipLaunchKernelGGL((sa::k_tile3d<COUNTER, FAST, S, WH, ON>), grid, dim3(c.threads), lds, st, t);
   };
+  if (t.a.L & 1) {
+    auto go_odd = [&](auto whole) {
+      constexpr bool WH = decltype(whole)::value;
+      static const hipError_t more = hipFuncSetAttribute((const void *)sa::k_tile3d_odd<COUNTER, FAST, S, WH>,
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
+      (void)more;
+      hipLaunchKernelGGL((sa::k_tile3d_odd<COUNTER, FAST, S, WH>), grid, dim3(c.threads), lds, st, t);
+    };
+    return c.whole ? go_odd(std::true_type{}) : go_odd(std::false_type{});
+  }
   const bool one = c.w0 * 64 <= c.threads;
   if constexpr (S == 2) {  // the kept couplings fit the registers
     if (one) return c.whole ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
@@ -91,24 +105,26 @@ void launch(const sa::tile3d_args &t, const tile_cfg &c, hipStream_t st) {
   c.whole ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
 }
 
-// in (rows x cols) to out (cols x rows), 32 x 32 words at a time; blockIdx.z: the array
+// in (rows x cols) to out (cols x rows, `stride` words per row), 32 x 32 words at a time;
+// blockIdx.z: the array
 __global__ void __launch_bounds__(256) k_transpose(const uint64_t *__restrict__ in, uint64_t *__restrict__ out, int rows,
-                                                   int cols) {
+                                                   int cols, int stride) {
   __shared__ uint64_t tile[32][33];
-  const int64_t base = (int64_t)blockIdx.z * rows * cols;
+  const int64_t base = (int64_t)blockIdx.z * rows * cols, obase = (int64_t)blockIdx.z * stride * cols;
   const int c0 = (int)blockIdx.x * 32, r0 = (int)blockIdx.y * 32, i = (int)threadIdx.x & 31, j0 = (int)threadIdx.x >> 5;
   for (int j = j0; j < 32; j += 8)
     if (r0 + j < rows && c0 + i < cols) tile[j][i] = in[base + (int64_t)(r0 + j) * cols + c0 + i];
   __syncthreads();
   for (int j = j0; j < 32; j += 8)
-    if (c0 + j < cols && r0 + i < rows) out[base + (int64_t)(c0 + j) * rows + r0 + i] = tile[i][j];
+    if (c0 + j < cols && r0 + i < rows) out[obase + (int64_t)(c0 + j) * stride + r0 + i] = tile[i][j];
 }
 
 }  // namespace
 
 // the ladder's couplings with z fastest, on its stream; false without memory
 bool sa_detail::tile3d_couplings(sa_ladder *l) {
-  if (!l->jt && hipMalloc(&l->jt, (size_t)3 * l->N * 8) != hipSuccess) {
+  const int stride = sa::column_stride(l->L);
+  if (!l->jt && hipMalloc(&l->jt, (size_t)3 * l->L * l->L * stride * 8) != hipSuccess) {
     l->jt = nullptr;
     (void)hipGetLastError();
     return false;
@@ -116,7 +132,7 @@ bool sa_detail::tile3d_couplings(sa_ladder *l) {
   if (l->jt_current) return true;
   const int L2 = l->L * l->L;
   hipLaunchKernelGGL(k_transpose, dim3((unsigned)((L2 + 31) / 32), (unsigned)((l->L + 31) / 32), 3), dim3(256), 0,
-                     l->stream, l->jx, l->jt, l->L, L2);
+                     l->stream, l->jx, l->jt, l->L, L2, stride);
   l->jt_current = true;
   return true;
 }
@@ -155,17 +171,19 @@ void sa_detail::tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t ta
   a.lg = c.lg;
   a.lp = c.lp;
   a.jxt = l->jt;
-  a.jyt = l->jt + l->N;
-  a.jzt = l->jt + 2 * l->N;
+  const int64_t jn = (int64_t)l->L * l->L * sa::column_stride(l->L);
+  a.jyt = l->jt + jn;
+  a.jzt = l->jt + 2 * jn;
   a.chunks0 = c.w0;
   a.chunks1 = c.w1;
   auto recip = [](int d) { return ((1 << 20) + d - 1) / d; };
   const int W = c.whole ? l->L : c.tx + 4, H = c.whole ? l->L : c.ty + 4;
-  a.recip_pairs = recip(W / 2 * H);
-  a.recip_hw = recip(W / 2);
+  const int row = l->L & 1 ? W : W / 2;  // columns or pairs of columns a thread loads
+  a.recip_pairs = recip(row * H);
+  a.recip_hw = recip(row);
   a.recip_ntx = recip(a.ntx);
   a.recip_per = (uint32_t)((((uint64_t)1 << 32) + a.ntx * a.nty - 1) / (a.ntx * a.nty));  // not used with one tile
-  a.zstep = c.threads / (W / 2 * H);
+  a.zstep = c.threads / (row * H);
   a.recip_n0 = recip(c.whole ? l->L / 2 : c.tx / 2 + 1);
   a.recip_n1 = recip(c.whole ? l->L / 2 : c.tx / 2);
   a.ns = c.ns;

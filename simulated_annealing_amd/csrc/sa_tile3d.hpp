@@ -1,4 +1,4 @@
-// sa_tile3d.hpp -- one 3D sweep (both colours) per launch, tiles of columns in LDS (even L).
+// sa_tile3d.hpp -- one 3D sweep (both colours) per launch, tiles of columns in LDS.
 //
 // A ladder too small to fill the chip with column walks is bound by latency: two launches
 // per sweep, each one dependent chain of loads, arithmetic and stores.  Here a workgroup
@@ -13,7 +13,8 @@
 // lane = column * 2^lg + segment (2^lg >= G, the rest idle); the new word of a plane is a
 // per-lane map (f0, f1) of the new word below it.  The count of the five bonds that do not point down is formed once,
 // the two outcomes are two cheap selects of it.  The last of the four-plane segments may be
-// shorter (its missing planes are identity maps), so any even L up to 256 is served.
+// shorter (its missing planes are identity maps), so any even L up to 256 is served, and odd
+// ones in the form further down.
 //
 // Everything a segment reads lies along z: the ladder keeps a copy of its couplings with z
 // fastest, made when the couplings are set and first needed, and LDS holds columns.  A
@@ -85,6 +86,7 @@ struct seg3d {
   uint32_t c0, ce, cs;    // columns x + L*y: the site's, its +x and its +y neighbour's
   int k, kw, ke, kn, ks;  // LDS columns: the site's, its four in-plane neighbours'
   int64_t rank;           // replay word of the column's plane 0
+  uint32_t rstep;         // replay words of this colour per plane
 };
 template <int S>
 struct seg3d_couplings {
@@ -135,17 +137,22 @@ __device__ __forceinline__ seg3d tile3d_segment(const tile3d_args &t, int color,
     q.ks = k + hw;
   }
   q.rank = (int64_t)color * (t.a.N >> 1) + (int64_t)y * (L >> 1) + (x >> 1);
+  q.rstep = (uint32_t)(L * L) >> 1;
   return q;
 }
 
+// words per column of the couplings with z fastest: even, so that pairs of planes are 16 bytes
+__host__ __device__ __forceinline__ int column_stride(int L) { return (L + 1) & ~1; }
+
 // S words of a column from plane z0 on, 16 bytes at a time (z0 even; beyond the lattice, in
-// a short last segment, the last two planes again)
+// a short last segment, the last pair of planes again; an odd side's last pair ends in padding)
 template <int S>
 __device__ __forceinline__ void column_words(const uint64_t *p, uint32_t col, int z0, int L, uint64_t (&w)[S]) {
+  const uint32_t st = (uint32_t)column_stride(L);
 #pragma unroll
   for (int j = 0; j < S; j += 2) {
-    const uint64_t *q = reinterpret_cast<const uint64_t *>(reinterpret_cast<const char *>(p) +
-                                                           (col * (uint32_t)L + (uint32_t)min(z0 + j, L - 2)) * 8u);
+    const uint64_t *q = reinterpret_cast<const uint64_t *>(
+        reinterpret_cast<const char *>(p) + (col * st + (uint32_t)min(z0 + j, (L - 1) & ~1)) * 8u);
     lds_ld2(q, w[j], w[j + 1]);
   }
 }
@@ -160,7 +167,7 @@ __device__ __forceinline__ void tile3d_load(const tile3d_args &t, const seg3d &q
   column_words<S>(t.jyt, q.cs, q.z0, L, d.js);
   column_words<S>(t.jzt, q.c0, q.z0, L, jz);
   const int zn = q.z0 + S;  // the plane above the segment; above the lattice's last, plane 0
-  const uint64_t jn = ld_off(t.jzt, (q.c0 * (uint32_t)L + (uint32_t)(zn >= L ? 0 : zn)) * 8u);
+  const uint64_t jn = ld_off(t.jzt, (q.c0 * (uint32_t)column_stride(L) + (uint32_t)(zn >= L ? 0 : zn)) * 8u);
   d.ju = jz[0];
 #pragma unroll
   for (int j = 0; j < S; ++j) d.jd[j] = (j == S - 1 || q.z0 + j + 1 >= L) ? jn : jz[j + 1 < S ? j + 1 : j];
@@ -180,7 +187,7 @@ __device__ __forceinline__ void tile3d_random(const tile3d_args &t, const uint64
     }
   } else {
 #pragma unroll
-    for (int j = 0; j < S; ++j) g[j] = words[q.rank + (int64_t)min(q.z0 + j, t.a.L - 1) * (L2 >> 1)];
+    for (int j = 0; j < S; ++j) g[j] = words[q.rank + (int64_t)min(q.z0 + j, t.a.L - 1) * q.rstep];
   }
 }
 
@@ -211,8 +218,9 @@ __device__ __forceinline__ void scan_columns(zmap &M, int g, int lg) {
   if (lg > 5) scan_step<kDppBcast31>(M, (g & 32) != 0);
 }
 
-// The colour's update of a segment; A / O: the LDS columns of this colour and the other.
-template <bool FAST, int S>
+// The colour's update of a segment; A / O: the LDS columns of this colour and the other
+// (ODD: all columns, A == O).
+template <bool FAST, int S, bool ODD = false>
 __device__ __forceinline__ void tile3d_update(const tile3d_args &t, const sys_table &tab, const uint64_t (&g64)[S],
                                               const seg3d &q, const seg3d_couplings<S> &d, uint64_t *A,
                                               const uint64_t *O) {
@@ -220,7 +228,7 @@ __device__ __forceinline__ void tile3d_update(const tile3d_args &t, const sys_ta
   uint64_t si[S + 1], nw[S], ne[S], nn[S], ns[S];
 #pragma unroll
   for (int j = 0; j < S; j += 2) {
-    const int z = min(z0 + j, L - 2);
+    const int z = min(z0 + j, (L - 1) & ~1);
     lds_ld2(A + q.k * lp + z, si[j], si[j + 1]);
     lds_ld2(O + q.kw * lp + z, nw[j], nw[j + 1]);
     lds_ld2(O + q.ke * lp + z, ne[j], ne[j + 1]);
@@ -234,32 +242,36 @@ __device__ __forceinline__ void tile3d_update(const tile3d_args &t, const sys_ta
 #pragma unroll
   for (int j = 0; j < S; ++j) {
     const uint64_t s = si[j];
-    // plane L-1 (always an odd j) sees the new plane 0 above it
-    const uint64_t dn = ((j & 1) && z0 + j == L - 1) ? new0 : si[j + 1];
     const uint64_t qw = xor3(d.jw[j], s, nw[j]), qe = xor3(d.je[j], s, ne[j]);
     const uint64_t qn = xor3(d.jn[j], s, nn[j]), qs = xor3(d.js[j], s, ns[j]);
-    const uint64_t qd = xor3(d.jd[j], s, dn);
     const uint64_t s1 = xor3(qw, qe, qn), k1 = maj3(qw, qe, qn);
-    const uint64_t p0 = xor3(qs, qd, s1), k2 = maj3(qs, qd, s1);
-    const uint64_t p1 = k1 ^ k2, p2 = k1 & k2;
-    flips f;
-    if (FAST) {
-      const uint32_t a4 = g64[j] < tab.thr[0][4] ? ~0u : 0u, a5 = g64[j] < tab.thr[0][5] ? ~0u : 0u;
-      const uint32_t a6 = g64[j] < tab.thr[0][6] ? ~0u : 0u;
-      f = flips_fast(a4, a5, a6, p0, p1, p2);
-    } else {
-      f = flips_general(accepted_levels(tab, 0, g64[j]), accepted_levels(tab, 1, g64[j]), p0, p1, p2, s);
-    }
     // bond below with an all-0 word below; plane 0 has the old plane L-1 there
     const uint64_t ju = j == 0 ? d.ju : d.jd[j - 1];
     const uint64_t b = xor3(ju, s, (j == 0 && z0 == 0) ? up0 : 0);
-    F[j].f0 = s ^ sel(b, f.f1, f.f0);
-    F[j].f1 = s ^ sel(b, f.f0, f.f1);
+    // the plane's map with the word dn above it
+    auto map = [&](uint64_t dn) {
+      const uint64_t qd = xor3(d.jd[j], s, dn);
+      const uint64_t p0 = xor3(qs, qd, s1), k2 = maj3(qs, qd, s1);
+      const uint64_t p1 = k1 ^ k2, p2 = k1 & k2;
+      flips f;
+      if (FAST) {
+        const uint32_t a4 = g64[j] < tab.thr[0][4] ? ~0u : 0u, a5 = g64[j] < tab.thr[0][5] ? ~0u : 0u;
+        const uint32_t a6 = g64[j] < tab.thr[0][6] ? ~0u : 0u;
+        f = flips_fast(a4, a5, a6, p0, p1, p2);
+      } else {
+        f = flips_general(accepted_levels(tab, 0, g64[j]), accepted_levels(tab, 1, g64[j]), p0, p1, p2, s);
+      }
+      F[j].f0 = s ^ sel(b, f.f1, f.f0);
+      F[j].f1 = s ^ sel(b, f.f0, f.f1);
+    };
+    // plane L-1 sees the new plane 0 above it
+    map(j > 0 && z0 + j == L - 1 ? new0 : si[j + 1]);
     if (j == 0) {
       if (z0 == 0) F[0].f1 = F[0].f0;
       new0 = shfl64(F[0].f0, q.base);  // segment 0 of this column
+      if (ODD && z0 == L - 1) map(new0);  // a last segment of one plane
     }
-    if (S > 2 && z0 + j >= L) F[j] = zmap{0, ~0ULL};  // no such plane
+    if ((ODD || S > 2) && z0 + j >= L) F[j] = zmap{0, ~0ULL};  // no such plane
   }
   zmap M = F[0];
 #pragma unroll
@@ -272,7 +284,7 @@ __device__ __forceinline__ void tile3d_update(const tile3d_args &t, const sys_ta
     for (int j = 0; j < S; j += 2) {
       const uint64_t v0 = (j == 0 && z0 == 0) ? F[0].f0 : sel(v, F[j].f1, F[j].f0);
       v = sel(v0, F[j + 1].f1, F[j + 1].f0);
-      if (S == 2 || z0 + j < L) lds_st2(A + q.k * lp + z0 + j, v0, v);
+      if (S == 2 || z0 + j < L) lds_st2(A + q.k * lp + z0 + j, v0, v);  // ODD: plane L is padding
     }
   }
 }
@@ -372,6 +384,139 @@ __device__ __forceinline__ void tile3d(const tile3d_args &t, int sys, int bx, in
       lds_st2(out + (int64_t)z * L2, (ty & 1) ? o : e, (ty & 1) ? e : o);
     }
   }
+}
+
+// ---------------------------------------------------------------- odd sides
+// With odd L the sites x = L-1 and x = 0 of a row have the same colour, and so have y = L-1
+// and y = 0: in a half-sweep (L-1, y) sees the new word of (0, y) in its plane, (x, L-1) that
+// of (x, 0), and the corner (L-1, L-1), of colour 0, those of (0, L-1) and (L-1, 0); all other
+// same-colour neighbours across the wrap are seen old (the reference's row-major order,
+// src/cpu_3d.cpp:94-105).  So a colour is updated in stages, each whole columns with a
+// barrier after it: first every column off the last column and row, then those on one of
+// them, then the corner.  In place, a stage reads old what later stages update.
+// The tiles' grid is shifted by two columns so that both wraps lie inside tile 0's own
+// columns, two away from its edge; every other tile is an ordinary one.  A tile is at most
+// L-4 wide, so no column occurs in it twice.  LDS keeps all columns in one array, and each
+// block first lists its columns by colour and stage.  Each stage costs its latency, about
+// 0.8 us; 12 systems of L=27: 50 -> 11 us per sweep, one of L=63 134 -> 12.
+constexpr int kOddShift = 2;
+constexpr int kOddPhases = 5;  // colour 0 stages 1, 2, 3; colour 1 stages 1, 2
+
+// LDS words (64 bit) of the column lists: first stages, second stages, the corner
+__host__ __device__ __forceinline__ int odd_list_cap(int W, int H, int phase) {
+  return phase == 0 || phase == 3 ? H * (W / 2 + 1) : phase == 2 ? 4 : W + H;
+}
+__host__ __device__ __forceinline__ int odd_list_words(int W, int H) {
+  int n = 0;
+  for (int q = 0; q < kOddPhases; ++q) n += odd_list_cap(W, H, q);
+  return (n + 3) / 4 + 4;  // 16-bit entries, five counters
+}
+
+template <bool COUNTER, bool FAST, int S, bool WHOLE>
+__device__ __forceinline__ void tile3d_odd(const tile3d_args &t, int sys, int bx, int by, uint64_t *lds) {
+  const sweep_args &p = t.a;
+  const int L = p.L, W = WHOLE ? L : t.tx + 4, H = WHOLE ? L : t.ty + 4, lp = t.lp, ncols = W * H;
+  const int cx = WHOLE ? L : min(t.tx, L - bx * t.tx), cy = WHOLE ? L : min(t.ty, L - by * t.ty);  // own columns
+  const int ox = WHOLE ? 0 : bx * t.tx - kOddShift - 2, oy = WHOLE ? 0 : by * t.ty - kOddShift - 2;
+  const int64_t L2 = (int64_t)L * L;
+  auto wrap = [&](int v) { return v < 0 ? v + L : v >= L ? v - L : v; };
+  uint64_t *A = lds;
+  int *cnt = reinterpret_cast<int *>(lds + ncols * lp);
+  uint16_t *list[kOddPhases];
+  {
+    uint16_t *q = reinterpret_cast<uint16_t *>(cnt + 8);
+#pragma unroll
+    for (int f = 0; f < kOddPhases; ++f) {
+      list[f] = q;
+      q += odd_list_cap(W, H, f);
+    }
+  }
+  if (threadIdx.x < 8) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  // a thread loads one column's planes zt, zt + zstep, ...
+  const int zt = small_div((int)threadIdx.x, t.recip_pairs), zstep = t.zstep;
+  const int k = (int)threadIdx.x - zt * ncols, ty = small_div(k, t.recip_hw), tx = k - ty * W;
+  const int x = wrap(ox + tx), y = wrap(oy + ty);
+  const uint64_t *col = p.s + (int64_t)sys * p.N + (y * L + x);
+  for (int zb = zt; zb < L; zb += 8 * zstep) {
+    uint64_t a[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = col[min(zb + u * zstep, L - 1) * L2];
+    if (zb == zt && zt == 0) {  // each column once: into its colour's and stage's list
+      const int c = (x + y) & 1, e = (c == 0 ? 1 : 2);
+      const bool in = WHOLE || (tx >= e && tx < cx + 4 - e && ty >= e && ty < cy + 4 - e);
+      if (in) {
+        const int stage = (x == L - 1 ? 1 : 0) + (y == L - 1 ? 1 : 0), f = c == 0 ? stage : 3 + stage;
+        list[0][(f == 0 ? 0 : f == 1 ? list[1] - list[0] : f == 2 ? list[2] - list[0] : f == 3 ? list[3] - list[0]
+                                                                                               : list[4] - list[0]) +
+                atomicAdd(&cnt[f], 1)] = (uint16_t)k;
+      }
+    }
+    if (zt < zstep) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) A[k * lp + min(zb + u * zstep, L - 1)] = a[u];
+    }
+  }
+  __syncthreads();
+  const int lane = (int)threadIdx.x & 63, nw = (int)blockDim.x >> 6, cc = lane >> t.lg;
+  for (int sw = 0; sw < (WHOLE ? t.ns : 1); ++sw) {
+    const sys_table &tab = p.tab[sys + sw * t.tab_step];
+    const uint64_t *words = COUNTER ? nullptr : p.words + (int64_t)sw * p.N;
+    const uint64_t sweep = p.sweep + (uint64_t)sw;
+    const uint16_t *cols = list[0];
+#pragma unroll 1
+    for (int f = 0; f < kOddPhases; ++f) {
+      const int n = cnt[f], color = f < 3 ? 0 : 1;
+      if (n == 0) {  // the same for the whole block
+        cols += odd_list_cap(W, H, f);
+        continue;
+      }
+      for (int ch = (int)threadIdx.x >> 6; ch * t.C < n; ch += nw) {
+        seg3d q;
+        q.base = cc << t.lg;
+        q.g = lane - q.base;
+        q.z0 = q.g < t.G ? q.g * S : 0;
+        const int at = ch * t.C + cc;
+        q.live = q.g < t.G && at < n;
+        q.k = cols[at < n ? at : 0];
+        const int qy = small_div(q.k, t.recip_hw), qx = q.k - qy * W;
+        const int gx = wrap(ox + qx), gy = wrap(oy + qy);
+        q.c0 = (uint32_t)(gx + L * gy);
+        q.ce = (uint32_t)((gx == L - 1 ? 0 : gx + 1) + L * gy);
+        q.cs = (uint32_t)(gx + L * (gy == L - 1 ? 0 : gy + 1));
+        q.kw = WHOLE && qx == 0 ? q.k + L - 1 : q.k - 1;
+        q.ke = WHOLE && qx == L - 1 ? q.k - (L - 1) : q.k + 1;
+        q.kn = WHOLE && qy == 0 ? q.k + (L - 1) * W : q.k - W;
+        q.ks = WHOLE && qy == L - 1 ? q.k - (L - 1) * W : q.k + W;
+        if (!COUNTER) {
+          q.rank = odd_rank(L, L, color, gx, gy, 0);
+          q.rstep = (uint32_t)(color ? L2 / 2 : (L2 + 1) / 2);
+        }
+        seg3d_couplings<S> d;
+        uint64_t g[S];
+        tile3d_load<S>(t, q, d);
+        tile3d_random<COUNTER, S>(t, words, sweep, q, g);
+        tile3d_update<FAST, S, true>(t, tab, g, q, d, A, A);
+      }
+      cols += odd_list_cap(W, H, f);
+      __syncthreads();
+    }
+  }
+  if (zt < zstep && (WHOLE || (tx >= 2 && tx < cx + 2 && ty >= 2 && ty < cy + 2))) {
+    uint64_t *out = (WHOLE ? p.s : t.out) + (int64_t)sys * p.N + (y * L + x);
+    for (int z = zt; z < L; z += zstep) out[z * L2] = A[k * lp + z];
+  }
+}
+
+template <bool COUNTER, bool FAST, int S, bool WHOLE>
+__global__ void __launch_bounds__(1024) k_tile3d_odd(tile3d_args t) {
+  extern __shared__ __align__(16) uint64_t lds[];
+  const uint32_t per = (uint32_t)(t.ntx * t.nty);  // blocks to tiles as in k_tile3d
+  const uint32_t b = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (b >= per * (uint32_t)t.a.nsys) return;
+  const uint32_t sys = per == 1 ? b : (uint32_t)(((uint64_t)b * t.recip_per) >> 32), r = b - sys * per;
+  const int by = small_div((int)r, t.recip_ntx);
+  tile3d_odd<COUNTER, FAST, S, WHOLE>(t, (int)sys, (int)r - by * t.ntx, by, lds);
 }
 
 template <bool COUNTER, bool FAST, int S, bool WHOLE, bool ONE>

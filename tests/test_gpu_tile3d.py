@@ -41,7 +41,22 @@ def test_tile3d_counter(orc, L):
     compare(orc, L, nsys, 2, sa.RNG_COUNTER, [0.6, 1.3], [0.2, 1.0])
 
 
-@pytest.mark.parametrize("L", [4, 10, 16, 28, 36])
+# odd sides: wrap neighbours of one colour.  Held whole up to 25; tiles from 27 on, whose last
+# tile has 1 .. 7 columns; last segments of one, two and three planes
+@pytest.mark.parametrize("L", [3, 5, 7, 9, 11, 13, 15, 17, 19, 21, 23, 25, 27, 29, 31, 33, 35, 37, 41, 49, 63, 71, 99])
+def test_tile3d_odd_counter(orc, L):
+    print("[case] tile3d odd L", L, flush=True)
+    nsys = 2 if L <= 64 else 1
+    compare(orc, L, nsys, 3, sa.RNG_COUNTER, [0.6, 1.3], [0.0, 0.0], steps=[1, 2])
+    compare(orc, L, nsys, 2, sa.RNG_COUNTER, [0.6, 1.3], [0.2, 1.0])
+
+
+@pytest.mark.parametrize("L,nsys", [(9, 33), (27, 12), (45, 8)])
+def test_tile3d_odd_many_systems(orc, L, nsys):
+    compare(orc, L, nsys, 3, sa.RNG_COUNTER, [0.5 + 0.1 * j for j in range(nsys)], [0.0] * nsys)
+
+
+@pytest.mark.parametrize("L", [3, 4, 10, 13, 16, 27, 28, 36])
 def test_tile3d_replay(orc, L):
     compare(orc, L, 2, 4, sa.RNG_REPLAY, [0.7, 1.9], [0.0, 0.0])
     compare(orc, L, 1, 3, sa.RNG_REPLAY, [0.7], [-0.3])
