@@ -18,6 +18,13 @@
 // constant argument, and one one-block kernel at the end of the chunk advances the
 // indices (no index update, and no drain of the whole grid for one, per sweep).
 //
+// Tiles.  Instances with symmetric tables that fit take the LDS-resident sweeps of
+// sa_tile2d.hpp / sa_tile3d.hpp instead: 3D instances tiles of columns, one launch per
+// sweep for all of them, 2D ones with an even side the whole lattice or bands of rows, one
+// launch per four sweeps.  They need a second
+// spin array (tiles and bands read one and write the other) and, in 3D, the couplings with
+// z fastest; where that memory is not to be had, an instance takes the half-sweep kernels.
+//
 // Exchanges.  Chunks end on every parallel-tempering instance's exchange points.
 // There the host draws the pair and the uniform of each due instance (its own
 // mt19937(123), as parallel_tempering::step), one launch measures the coldest
@@ -37,16 +44,26 @@
 
 #include "sa/exchange.hpp"
 #include "sa_internal.hpp"
+#include "sa_tile2d.hpp"
+#include "sa_tile3d.hpp"
 
 namespace {
 
+// how an instance is swept
+enum { FORM_HALF = 0, FORM_3D = 1, FORM_3D_ODD = 2, FORM_2D_WHOLE = 3, FORM_2D_BANDS = 4 };
+__host__ __device__ __forceinline__ bool two_arrays(int form) {
+  return form == FORM_3D || form == FORM_3D_ODD || form == FORM_2D_BANDS;
+}
+
 struct inst_desc {
-  sa::sweep_args a;  // a.s: first spin array; tab: tables (per sweep: nsweeps x nsys, else nsys)
-  uint64_t *s2;      // second spin array (instances that may take the fused 3D sweep)
+  sa::sweep_args a;  // a.s: current spin array at the schedule; tab: tables (per sweep: nsweeps x nsys, else nsys)
+  uint64_t *s2;      // second spin array (forms with two arrays)
   int kind, nsweeps, t, per_sweep, fast;
-  int fused;  // swept by the fused kernel in this schedule (reads the current array, writes the other)
-  int cur;    // 1: s2 holds the current spins
-  int pad;
+  int form;
+  int cur;           // 1: s2 holds the current spins
+  int m;             // sweeps of one visit (forms 3D: 1)
+  int th, bands;     // 2D forms
+  sa::tile3d_args t3;  // 3D forms: geometry and couplings
 };
 
 // t: the instance's sweep index (its index at the chunk start plus the sweep's
@@ -54,7 +71,6 @@ struct inst_desc {
 template <bool FAST>
 __device__ __forceinline__ void batch_item(const inst_desc &in, int t, int color, int k, int sys) {
   sa::sweep_args a = in.a;
-  if (in.cur) a.s = in.s2;  // half-sweeps update the current array in place
   if (in.per_sweep) a.tab += (int64_t)t * a.nsys;
   a.sweep = (uint64_t)t;
   if (a.L & 1) {  // odd L: k is a member lane (3D) or a wrap group (2D), sa_kernels.hpp
@@ -101,35 +117,74 @@ __global__ void k_batch_advance(inst_desc *d, const int *__restrict__ ctrl, int 
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
     const int done = min(k, max(0, d[i].nsweeps - d[i].t));
     d[i].t += done;
-    if (d[i].fused) d[i].cur ^= done & 1;  // each fused sweep wrote the other array
+    if (two_arrays(d[i].form)) d[i].cur ^= ((done + d[i].m - 1) / d[i].m) & 1;  // each visit wrote the other array
   }
 }
 
-// Fused 3D sweeps of one group of instances (same L, band height TH and systems per
-// workgroup MB, so one block size and LDS size): group g's blocks are entries
-// ctrl[2+2g] .. +ctrl[3+2g] of the fused block map, each (descriptor, band index
-// sb * (L/TH) + tile).  Each block runs the single-ladder fused walk on its band.
-constexpr int kMaxFusedGroups = 24;
-template <int MB, int TH>
-__global__ void __launch_bounds__(640) k_batch_fused(const inst_desc *__restrict__ d, const int2 *__restrict__ fmap,
-                                                     const int *__restrict__ ctrl, int g, int s) {
-  extern __shared__ uint64_t lds[];
-  const int off = ctrl[2 + 2 * g], n = ctrl[3 + 2 * g];
-  for (int blk = blockIdx.x; blk < n; blk += gridDim.x) {
-    const int2 bm = fmap[off + blk];
-    const inst_desc &in = d[bm.x];
-    const int t = in.t + s;
-    if (t >= in.nsweeps) continue;  // the whole block skips together
-    sa::sweep_args a = in.a;
-    if (in.per_sweep) a.tab += (int64_t)t * a.nsys;
-    a.sweep = (uint64_t)t;
-    const int cur = in.cur ^ (s & 1);  // every earlier sweep of the chunk was fused too
-    a.s = cur ? in.s2 : in.a.s;
-    uint64_t *out = cur ? in.a.s : in.s2;
-    const int ntile = a.L / TH;
-    const int sb = bm.y / ntile, tile = bm.y - sb * ntile;
-    sa::fused_band<true, true, MB, TH>(a, out, sb, tile, lds);
-    __syncthreads();  // the next band reuses the LDS
+// Launch v of a chunk of k sweeps: sweeps v*m .. of every listed tile, at most m of them.
+// Returns false when the instance has none left; a.s and out are the arrays of this launch.
+__device__ __forceinline__ bool tile_visit(const inst_desc &in, int k, int v, sa::sweep_args &a, uint64_t *&out, int &ns) {
+  const int t = in.t + v * in.m;
+  ns = min(in.m, min(in.nsweeps - t, k - v * in.m));
+  if (ns <= 0) return false;
+  const int cur = two_arrays(in.form) ? in.cur ^ (v & 1) : 0;
+  a = in.a;
+  if (in.per_sweep) a.tab += (int64_t)t * a.nsys;
+  a.sweep = (uint64_t)t;
+  a.s = cur ? in.s2 : in.a.s;
+  out = cur ? in.a.s : in.s2;
+  return true;
+}
+
+// The 3D tiles of a sweep.  Entries (descriptor, tile) are kept per XCD (blocks go
+// round-robin over the 8 XCDs), an instance's tiles together, so its words and couplings
+// stay in one L2: ctrl[2+2x], ctrl[3+2x] = first entry and count of XCD x.
+// Blocks of 512 threads with 80 KB of LDS: two per CU, eight waves each.
+// 13 systems of L=48: 55 -> 22 us per sweep, of L=47 77 -> 25, of L=24 25 -> 8 (column walks
+// in two launches before); segments of four planes take the same.  In one kernel with the 2D
+// tiles the registers spilled and the two kinds' blocks waited for each other (the benchmark
+// mix 73 us per sweep against 52).
+constexpr int kTileThreads = 512, kTileS = 2;
+constexpr size_t kTileLds = 80 * 1024;
+__global__ void __launch_bounds__(kTileThreads, 4) k_batch_tile3d(const inst_desc *__restrict__ d,
+                                                                  const int2 *__restrict__ tmap,
+                                                                  const int *__restrict__ ctrl, int k, int v) {
+  extern __shared__ __align__(16) uint64_t lds[];
+  const int xcd = (int)blockIdx.x & 7, off = ctrl[2 + 2 * xcd], n = ctrl[3 + 2 * xcd];
+  for (int e = (int)blockIdx.x >> 3; e < n; e += (int)gridDim.x >> 3) {  // the same for the whole block
+    const int2 tm = tmap[off + e];
+    const inst_desc &in = d[tm.x];
+    sa::tile3d_args t3 = in.t3;
+    int ns;
+    if (!tile_visit(in, k, v, t3.a, t3.out, ns)) continue;
+    const int per = t3.ntx * t3.nty, sys = tm.y / per, r = tm.y - sys * per, by = r / t3.ntx;
+    if (in.form == FORM_3D) sa::tile3d<true, true, kTileS, false, false>(t3, sys, r - by * t3.ntx, by, lds);
+    else sa::tile3d_odd<true, true, kTileS, false>(t3, sys, r - by * t3.ntx, by, lds);
+    __syncthreads();  // the next tile reuses the LDS
+  }
+}
+
+// The 2D tiles: whole lattices and bands of rows, up to m sweeps per launch (16 systems of
+// L=64: 8.1 -> 3.9 us per sweep, of L=128 10.1 -> 4.2).
+constexpr int kTile2dThreads = 1024, kTile2dItems = 2 * kTile2dThreads;
+constexpr int kSweeps2d = 4;  // sweeps per launch
+__global__ void __launch_bounds__(kTile2dThreads) k_batch_tile2d(const inst_desc *__restrict__ d,
+                                                                 const int2 *__restrict__ tmap,
+                                                                 const int *__restrict__ ctrl, int k, int v) {
+  extern __shared__ __align__(16) uint64_t lds[];
+  const int off = ctrl[18], n = ctrl[19];
+  for (int e = (int)blockIdx.x; e < n; e += (int)gridDim.x) {
+    const int2 tm = tmap[off + e];
+    const inst_desc &in = d[tm.x];
+    sa::tile2d_args t2;
+    if (!tile_visit(in, k, v, t2.a, t2.out, t2.ns)) continue;
+    t2.th = in.th;
+    t2.bands = in.bands;
+    t2.tab_step = in.per_sweep ? t2.a.nsys : 0;
+    const int sys = tm.y / in.bands;
+    if (in.form == FORM_2D_WHOLE) sa::tile2d<true, sa::T2_FAST, 2, true>(t2, sys, 0, lds);
+    else sa::tile2d<true, sa::T2_FAST, 2, false>(t2, sys, tm.y - sys * in.bands, lds);
+    __syncthreads();  // the next tile reuses the LDS
   }
 }
 
@@ -291,27 +346,21 @@ struct pt_state {
 
 struct batch_inst {
   sa_ladder *lad = nullptr;
-  uint64_t *s_first = nullptr;  // the ladder's spin array at attach (s_alt is the other)
   sa::sys_table *tabs = nullptr;
   int nsweeps = 0, per_sweep = 0, t = 0;
   bool fast = true, live = false;
   int64_t work = 0;   // work items per half-sweep (all systems)
   int64_t bytes = 0;  // device memory held
+  int form = FORM_HALF;
   pt_state pt;
 };
 
-// The fused 3D sweep inside the batch (k_batch_fused on forked graph branches) is
-// switched off: one run of its test stopped making progress and no cause has been
-// found in this code.  Off, 3D instances take the half-sweep kernels, no second
-// spin array is allocated and SA_TUNE_BATCH_FUSED = 2 is refused.
-constexpr bool kFusedBatch = false;
-
-// online-tuning candidates: (fused 3D sweep 2 on / 1 off, threads per half-sweep
-// block, sweeps per graph); the first chunks try them in this order
+// online-tuning candidates (threads per half-sweep block, sweeps per graph); the first
+// chunks try them in this order
 struct tune_cand {
-  int fused, block, chunk;
+  int block, chunk;
 };
-const tune_cand kCands[2] = {{1, 128, 32}, {1, 64, 32}};
+const tune_cand kCands[2] = {{128, 32}, {64, 32}};
 const int kNumCands = 2;
 
 }  // namespace
@@ -326,30 +375,22 @@ struct sa_batch {
   dev_array<int> d_ctrl;
   int ndesc = 0, nblocks = 0, bmap_bs = 0;
   std::vector<int> desc_id;  // instance id of each descriptor
-  std::vector<char> desc_fused;  // descriptor swept by the fused kernel
-  // fused 3D groups of the current schedule: (L, TH, MB) and block count each
-  struct fgroup {
-    int L, TH, MB, count;
-  };
-  std::vector<fgroup> groups;
-  dev_array<int2> d_fmap;
-  int sched_fused = -1;  // fused mode the schedule was built with
+  std::vector<int> desc_m;   // sweeps per visit of each descriptor, 0 with one array
+  dev_array<int2> d_tmap;
+  int ntiles = 0, ntiles2 = 0;  // entries of k_batch_tile3d, k_batch_tile2d
   bool dirty = true;
-  std::map<int, hipGraphExec_t> graphs;  // chunk length -> graph over the current arrays, block size, groups
+  // (chunk length, which kernels it launches) -> graph over the current arrays and block size
+  std::map<std::pair<int, int>, hipGraphExec_t> graphs;
   int graph_bs = 0;
-  std::vector<fgroup> graph_groups;
-  std::vector<hipStream_t> side;  // side streams of the fused groups (fork/join inside the graph)
-  std::vector<hipEvent_t> side_done;
-  hipEvent_t fork = nullptr;
   // exchange staging
   pinned h_stage;
   dev_array<meas_item> d_meas;
   dev_array<swap_item> d_swap;
   dev_array<int> d_cnt;
   pinned h_cnt;
-  // tuning: 0 = automatic; fused: 0 automatic, 1 off, 2 on
+  // tuning: 0 = automatic (fused: 0 or 1, the fused band walk is not in the batch)
   int block = 0, chunk = 0, fused = 0;
-  int tuned_block = 0, tuned_chunk = 0, tuned_fused = 0;
+  int tuned_block = 0, tuned_chunk = 0;
   std::vector<std::pair<int, float>> trials;  // (candidate, ms per work item)
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   int64_t bytes_live = 0;
@@ -374,24 +415,35 @@ int grid_for(const sa_batch *b, int bs) {
   return std::max(1, b->cus * 16 * 2 / (bs / 64));
 }
 
-// descriptors and block map of the unfinished instances, largest remaining work first
-// fused 3D configuration of an instance: the tallest band (TH rows) that fits the
-// kernel's launch bound and LDS, two systems per workgroup when nsys is even
-bool fused_cfg(const sa_ladder *l, int &TH, int &MB) {
-  if (l->kind != SA_KIND_3D || (int64_t)l->N * 8 >= ((int64_t)1 << 31)) return false;
-  MB = (l->nsys % 2 == 0) ? 2 : 1;
-  for (int th : {16, 8, 4}) {
-    if (l->L % th || th > l->L || (th + 2) * (l->L / 2) > 640) continue;
-    if ((size_t)3 * (th + 2) * MB * 2 * (l->L / 2) * 8 > 64 * 1024) continue;
-    TH = th;
-    return true;
-  }
-  return false;
+// The form an instance with symmetric tables can take: 3D tiles for 8 <= L <= 128 (from 9
+// where L is odd: a tile is at least 4 columns and its halos wide), 2D with an even L up to
+// 256 (a band of 2048 items then holds four sweeps' halos and 16 rows).
+int tile_form(int kind, int L) {
+  if (kind == SA_KIND_3D) return L < 8 || L > 128 ? FORM_HALF : (L & 1) ? FORM_3D_ODD : FORM_3D;
+  if (kind != SA_KIND_2D || (L & 1) || L > 256) return FORM_HALF;
+  return L * sa::tile2d_groups(L) <= kTile2dItems ? FORM_2D_WHOLE : FORM_2D_BANDS;
 }
 
-// descriptors, the half-sweep block map and the fused groups' block maps of the
-// unfinished instances, largest remaining work first
-int rebuild(sa_batch *b, int bs, bool fused) {
+// device bytes the form needs beside the instance's own
+int64_t form_bytes(int kind, int L, int nsys, int form) {
+  const int64_t L2 = (int64_t)L * L, N = L2 * (kind == SA_KIND_3D ? L : 1);
+  return (two_arrays(form) ? nsys * N * 8 : 0) + (kind == SA_KIND_3D && form ? 3 * L2 * sa::column_stride(L) * 8 : 0);
+}
+
+// 3D tile geometry: wide x high columns, halved until the LDS holds it
+bool tile3d_geometry(sa::tile3d_args &a, int L, int wide, int high) {
+  for (;;) {
+    const size_t lds = sa::tile3d_setup(a, L, false, wide, high, kTileS, kTileThreads);
+    if (lds && lds <= kTileLds) return true;
+    if (wide <= 4 && high <= 4) return false;
+    if (wide >= high) wide /= 2;
+    else high /= 2;
+  }
+}
+
+// descriptors, the half-sweep block map and the tiles of the unfinished instances,
+// largest remaining work first
+int rebuild(sa_batch *b, int bs) {
   std::vector<int> ids;
   for (int i = 0; i < (int)b->inst.size(); ++i)
     if (b->inst[i].live && b->inst[i].t < b->inst[i].nsweeps) ids.push_back(i);
@@ -399,78 +451,35 @@ int rebuild(sa_batch *b, int bs, bool fused) {
     const auto &a = b->inst[x], &c = b->inst[y];
     return a.work * (int64_t)(a.nsweeps - a.t) > c.work * (int64_t)(c.nsweeps - c.t);
   });
-  // which instances take the fused sweep, and their groups
-  std::vector<sa_batch::fgroup> groups;
-  std::vector<std::vector<int2>> gmaps;
-  std::vector<int> gidx(ids.size(), -1);
-  int64_t nblk = 0;
-  for (size_t q = 0; q < ids.size(); ++q) {
-    const batch_inst &in = b->inst[ids[q]];
-    int TH = 0, MB = 0;
-    if (fused && in.fast && in.lad->s_alt && fused_cfg(in.lad, TH, MB)) {
-      int g = -1;
-      for (size_t j = 0; j < groups.size(); ++j)
-        if (groups[j].L == in.lad->L && groups[j].TH == TH && groups[j].MB == MB) g = (int)j;
-      if (g < 0 && (int)groups.size() < kMaxFusedGroups) {
-        g = (int)groups.size();
-        groups.push_back({in.lad->L, TH, MB, 0});
-        gmaps.emplace_back();
-      }
-      if (g >= 0) {
-        gidx[q] = g;
-        const int nb = (in.lad->L / TH) * (in.lad->nsys / MB);
-        for (int k = 0; k < nb; ++k) gmaps[g].push_back(make_int2((int)q, k));
-        groups[g].count += nb;
-        continue;
-      }
-    }
-    nblk += (in.work + bs - 1) / bs;
+  // 3D tiles of 8 x 8 columns when they make two blocks per CU, else smaller ones
+  int64_t tiles8 = 0;
+  for (int id : ids) {
+    const batch_inst &in = b->inst[id];
+    const int64_t side = (in.lad->L + 7) / 8;
+    if (in.form == FORM_3D || in.form == FORM_3D_ODD) tiles8 += side * side * in.lad->nsys;
   }
-  int64_t nf = 0;
-  for (auto &m : gmaps) nf += (int64_t)m.size();
-  if (nblk > INT32_MAX / 2 || nf > INT32_MAX / 2) return sa_fail(SA_ERR_ARG, "batch too large");
-  // earlier launches may still read the old arrays and the staging buffer
-  SA_HIP_TRY(hipStreamSynchronize(b->stream));
-  bool m1 = false, m2 = false, m3 = false, m4 = false;
-  int rc = b->d_desc.ensure(std::max<size_t>(ids.size(), 1), m1);
-  if (!rc) rc = b->d_bmap.ensure(std::max<int64_t>(nblk, 1), m2);
-  if (!rc) rc = b->d_ctrl.ensure(2 + 2 * kMaxFusedGroups, m3);
-  if (!rc) rc = b->d_fmap.ensure(std::max<int64_t>(nf, 1), m4);
-  if (rc) return rc;
-  bool same_groups = groups.size() == b->graph_groups.size();
-  for (size_t j = 0; same_groups && j < groups.size(); ++j)
-    same_groups = groups[j].L == b->graph_groups[j].L && groups[j].TH == b->graph_groups[j].TH &&
-                  groups[j].MB == b->graph_groups[j].MB && groups[j].count <= b->graph_groups[j].count;
-  if (m1 || m2 || m3 || m4 || b->graph_bs != bs || !same_groups) {
-    drop_graphs(b);
-    b->graph_groups = groups;  // block counts at capture size the fused grids
-  }
-  b->graph_bs = bs;
-  const int nctrl = 2 + 2 * kMaxFusedGroups;
-  const size_t bytes = sizeof(int) * nctrl + sizeof(inst_desc) * ids.size() + sizeof(int2) * (nblk + nf) + 64;
-  if (!b->h_stage.ensure(bytes)) return sa_fail(SA_ERR_NOMEM, "pinned staging");
-  int *ctrl = (int *)b->h_stage.p;
-  inst_desc *desc = (inst_desc *)((char *)b->h_stage.p + ((sizeof(int) * nctrl + 15) & ~(size_t)15));
-  int2 *bmap = (int2 *)(desc + ids.size());
-  int2 *fmap = bmap + nblk;
-  int64_t q2 = 0;
-  b->desc_fused.assign(ids.size(), 0);
+  const int wide = tiles8 >= 2 * b->cus / 4 ? 8 : 4, high = tiles8 >= 2 * b->cus / 2 ? 8 : 4;
+  std::vector<inst_desc> descs(ids.size());
+  struct item {
+    int2 e;
+    float cost;
+  };
+  std::vector<item> tiles;
+  std::vector<int2> halves, tiles2;
+  double total = 0;
+  b->desc_m.assign(ids.size(), 0);
   for (size_t q = 0; q < ids.size(); ++q) {
     const batch_inst &in = b->inst[ids[q]];
     const sa_ladder *l = in.lad;
-    inst_desc d;
+    inst_desc &d = descs[q];
     std::memset(&d, 0, sizeof d);
-    // a.s is the ladder's first array; the current one is l->s
-    d.a.s = in.s_first;
-    d.s2 = (l->s == in.s_first) ? l->s_alt : l->s;
-    d.cur = (l->s == in.s_first) ? 0 : 1;
+    d.a.s = l->s;  // the current array
+    d.s2 = l->s_alt;
     d.a.jx = l->jx;
     d.a.jy = l->jy;
     d.a.jz = l->jz;
     d.a.tab = in.tabs;
-    d.a.words = nullptr;
     d.a.seed = l->seed;
-    d.a.sweep = 0;
     d.a.N = l->N;
     d.a.L = l->L;
     d.a.nsys = l->nsys;
@@ -479,89 +488,105 @@ int rebuild(sa_batch *b, int bs, bool fused) {
     d.t = in.t;
     d.per_sweep = in.per_sweep;
     d.fast = in.fast ? 1 : 0;
-    d.fused = gidx[q] >= 0 ? 1 : 0;
-    desc[q] = d;
-    b->desc_fused[q] = (char)d.fused;
-    if (!d.fused)
-      for (int64_t off = 0; off < in.work; off += bs) bmap[q2++] = make_int2((int)q, (int)off);
+    d.form = in.form;
+    d.m = 1;
+    int64_t n = 0;
+    float cost = 0;  // of an entry, about us
+    if ((in.form == FORM_3D || in.form == FORM_3D_ODD) && tile3d_geometry(d.t3, l->L, wide, high)) {
+      const int64_t jn = (int64_t)l->L * l->L * sa::column_stride(l->L);
+      d.t3.jxt = l->jt;
+      d.t3.jyt = l->jt + jn;
+      d.t3.jzt = l->jt + 2 * jn;
+      d.t3.ns = 1;
+      n = (int64_t)d.t3.ntx * d.t3.nty * l->nsys;
+      cost = 2.f + 0.1f * (float)l->L * (float)(d.t3.tx * d.t3.ty) / 64.f;
+    } else if (in.form == FORM_2D_WHOLE || in.form == FORM_2D_BANDS) {
+      const int rows = kTile2dItems / sa::tile2d_groups(l->L);  // rows of a tile
+      const bool whole = in.form == FORM_2D_WHOLE;
+      d.m = kSweeps2d;
+      d.th = whole ? l->L : std::min(16, rows - 4 * d.m);
+      d.bands = whole ? 1 : (l->L + d.th - 1) / d.th;
+      for (int64_t e = 0; e < (int64_t)d.bands * l->nsys; ++e) tiles2.push_back(make_int2((int)q, (int)e));
+    } else {
+      d.form = FORM_HALF;
+    }
+    if (two_arrays(d.form)) b->desc_m[q] = d.m;
+    if (d.form == FORM_2D_WHOLE || d.form == FORM_2D_BANDS) {
+      // entries made above
+    } else if (d.form == FORM_HALF) {
+      for (int64_t off = 0; off < in.work; off += bs) halves.push_back(make_int2((int)q, (int)off));
+    } else {
+      for (int64_t k = 0; k < n; ++k) tiles.push_back({make_int2((int)q, (int)k), cost});
+      total += n * cost;
+    }
+    if (halves.size() > INT32_MAX / 2 || tiles.size() + tiles2.size() > INT32_MAX / 2) return sa_fail(SA_ERR_ARG, "batch too large");
   }
+  // earlier launches may still read the old arrays and the staging buffer
+  SA_HIP_TRY(hipStreamSynchronize(b->stream));
+  constexpr int nctrl = 2 + 16 + 2;
+  const size_t ntile = tiles.size() + tiles2.size();
+  bool m1 = false, m2 = false, m3 = false, m4 = false;
+  int rc = b->d_desc.ensure(std::max<size_t>(ids.size(), 1), m1);
+  if (!rc) rc = b->d_bmap.ensure(std::max<size_t>(halves.size(), 1), m2);
+  if (!rc) rc = b->d_ctrl.ensure(nctrl, m3);
+  if (!rc) rc = b->d_tmap.ensure(std::max<size_t>(ntile, 1), m4);
+  if (rc) return rc;
+  if (m1 || m2 || m3 || m4 || b->graph_bs != bs) drop_graphs(b);
+  b->graph_bs = bs;
+  const size_t o_desc = (sizeof(int) * nctrl + 15) & ~(size_t)15, o_half = o_desc + sizeof(inst_desc) * ids.size();
+  const size_t o_tile = o_half + sizeof(int2) * halves.size();
+  if (!b->h_stage.ensure(o_tile + sizeof(int2) * ntile + 64)) return sa_fail(SA_ERR_NOMEM, "pinned staging");
+  char *st = (char *)b->h_stage.p;
+  int *ctrl = (int *)st;
   std::memset(ctrl, 0, sizeof(int) * nctrl);
-  ctrl[0] = (int)nblk;
+  ctrl[0] = (int)halves.size();
   ctrl[1] = (int)ids.size();
-  int64_t fo = 0;
-  for (size_t g = 0; g < gmaps.size(); ++g) {
-    ctrl[2 + 2 * g] = (int)fo;
-    ctrl[3 + 2 * g] = (int)gmaps[g].size();
-    std::memcpy(fmap + fo, gmaps[g].data(), sizeof(int2) * gmaps[g].size());
-    fo += (int64_t)gmaps[g].size();
+  // the entries in order, an eighth of the cost to each XCD
+  double sum = 0;
+  int2 *tmap = (int2 *)(st + o_tile);
+  for (size_t e = 0; e < tiles.size(); ++e) {
+    const int x = std::min(7, (int)(8 * sum / total));
+    if (ctrl[3 + 2 * x]++ == 0) ctrl[2 + 2 * x] = (int)e;
+    tmap[e] = tiles[e].e;
+    sum += tiles[e].cost;
   }
+  ctrl[18] = (int)tiles.size();
+  ctrl[19] = (int)tiles2.size();
+  std::memcpy(tmap + tiles.size(), tiles2.data(), sizeof(int2) * tiles2.size());
+  std::memcpy(st + o_desc, descs.data(), sizeof(inst_desc) * ids.size());
+  std::memcpy(st + o_half, halves.data(), sizeof(int2) * halves.size());
   SA_HIP_TRY(hipMemcpyAsync(b->d_ctrl.p, ctrl, sizeof(int) * nctrl, hipMemcpyHostToDevice, b->stream));
-  if (!ids.empty()) {
-    SA_HIP_TRY(hipMemcpyAsync(b->d_desc.p, desc, sizeof(inst_desc) * ids.size(), hipMemcpyHostToDevice, b->stream));
-    if (nblk) SA_HIP_TRY(hipMemcpyAsync(b->d_bmap.p, bmap, sizeof(int2) * nblk, hipMemcpyHostToDevice, b->stream));
-    if (nf) SA_HIP_TRY(hipMemcpyAsync(b->d_fmap.p, fmap, sizeof(int2) * nf, hipMemcpyHostToDevice, b->stream));
-  }
+  if (!ids.empty())
+    SA_HIP_TRY(hipMemcpyAsync(b->d_desc.p, st + o_desc, sizeof(inst_desc) * ids.size(), hipMemcpyHostToDevice, b->stream));
+  if (!halves.empty())
+    SA_HIP_TRY(hipMemcpyAsync(b->d_bmap.p, st + o_half, sizeof(int2) * halves.size(), hipMemcpyHostToDevice, b->stream));
+  if (ntile)
+    SA_HIP_TRY(hipMemcpyAsync(b->d_tmap.p, tmap, sizeof(int2) * ntile, hipMemcpyHostToDevice, b->stream));
   b->ndesc = (int)ids.size();
   b->desc_id = ids;
-  b->nblocks = (int)nblk;
+  b->nblocks = (int)halves.size();
+  b->ntiles = (int)tiles.size();
+  b->ntiles2 = (int)tiles2.size();
   b->bmap_bs = bs;
-  b->groups = groups;
-  b->sched_fused = fused ? 1 : 0;
   b->dirty = false;
   return SA_OK;
 }
 
-void launch_fused_group(sa_batch *b, int g, int s, hipStream_t st) {
-  const sa_batch::fgroup &G = b->graph_groups[g];
-  const dim3 grid((unsigned)std::max(1, G.count)), block((unsigned)((G.TH + 2) * (G.L / 2)));
-  const size_t lds = (size_t)3 * (G.TH + 2) * G.MB * 2 * (G.L / 2) * 8;
-#define SA_FUSED_CASE(MBV, THV)                                                                               \
-  if (G.MB == MBV && G.TH == THV) {                                                                         \
-    hipLaunchKernelGGL((k_batch_fused<MBV, THV>), grid, block, lds, st, b->d_desc.p, b->d_fmap.p,            \
-                       b->d_ctrl.p, g, s);                                                                  \
-    return;                                                                                                 \
-  }
-  SA_FUSED_CASE(1, 4)
-  SA_FUSED_CASE(1, 8)
-  SA_FUSED_CASE(1, 16)
-  SA_FUSED_CASE(2, 4)
-  SA_FUSED_CASE(2, 8)
-  SA_FUSED_CASE(2, 16)
-#undef SA_FUSED_CASE
-}
-
-// One sweep = the two half-sweep launches and one launch per fused group; the
-// chunk ends with the advance.  The launches touch disjoint instances, so the fused groups go on side
-// streams forked from and joined back to the batch stream (parallel branches of
-// the captured graph) and overlap each other and the half-sweeps.
-// side streams and events for ng fused groups (created outside any capture)
-int ensure_side(sa_batch *b, int ng) {
-  for (int g = (int)b->side.size(); g < ng; ++g) {
-    hipStream_t st = nullptr;
-    hipEvent_t ev = nullptr;
-    SA_HIP_TRY(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    SA_HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    b->side.push_back(st);
-    b->side_done.push_back(ev);
-  }
-  if (!b->fork) SA_HIP_TRY(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
-  return SA_OK;
-}
-
+// One sweep = a launch of the 3D tiles and two half-sweep launches, of whichever there are,
+// with a launch of the 2D tiles every kSweeps2d sweeps; the chunk ends with the advance.
 int enqueue_sweeps(sa_batch *b, int k) {
   const int grid = grid_for(b, b->bmap_bs);
-  const int ng = (int)b->graph_groups.size();
+  const int tgrid = std::max(8, b->cus / 4 * 8);  // two blocks per CU, a multiple of the 8 XCDs
   for (int s = 0; s < k; ++s) {
-    if (ng) SA_HIP_TRY(hipEventRecord(b->fork, b->stream));
-    for (int g = 0; g < ng; ++g) {
-      SA_HIP_TRY(hipStreamWaitEvent(b->side[g], b->fork, 0));
-      launch_fused_group(b, g, s, b->side[g]);
-      SA_HIP_TRY(hipEventRecord(b->side_done[g], b->side[g]));
-    }
-    for (int color = 0; color < 2; ++color)
+    if (b->ntiles)
+      hipLaunchKernelGGL(k_batch_tile3d, dim3(tgrid), dim3(kTileThreads), kTileLds, b->stream, b->d_desc.p, b->d_tmap.p,
+                         b->d_ctrl.p, k, s);
+    if (b->ntiles2 && s % kSweeps2d == 0)
+      hipLaunchKernelGGL(k_batch_tile2d, dim3(2 * b->cus), dim3(kTile2dThreads), kTile2dItems * 32, b->stream, b->d_desc.p,
+                         b->d_tmap.p, b->d_ctrl.p, k, s / kSweeps2d);
+    for (int color = 0; color < 2 && b->nblocks; ++color)
       hipLaunchKernelGGL(k_batch_half, dim3(grid), dim3(b->bmap_bs), 0, b->stream, b->d_desc.p, b->d_bmap.p,
                          b->d_ctrl.p, color, s);
-    for (int g = 0; g < ng; ++g) SA_HIP_TRY(hipStreamWaitEvent(b->stream, b->side_done[g], 0));
   }
   hipLaunchKernelGGL(k_batch_advance, dim3(1), dim3(256), 0, b->stream, b->d_desc.p, b->d_ctrl.p, k);
   return SA_OK;
@@ -569,14 +594,16 @@ int enqueue_sweeps(sa_batch *b, int k) {
 
 // the graph of k sweeps over the current device arrays (captured on first use)
 int graph_for(sa_batch *b, int k, hipGraphExec_t &out) {
-  auto it = b->graphs.find(k);
+  const std::pair<int, int> key(k, (b->ntiles ? 1 : 0) + (b->nblocks ? 2 : 0) + (b->ntiles2 ? 4 : 0));
+  auto it = b->graphs.find(key);
   if (it != b->graphs.end()) {
     out = it->second;
     return SA_OK;
   }
   hipGraph_t g = nullptr;
-  const int src = ensure_side(b, (int)b->graph_groups.size());
-  if (src) return src;
+  static const hipError_t more = hipFuncSetAttribute((const void *)k_batch_tile3d,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
+  (void)more;
   SA_HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   const int erc = enqueue_sweeps(b, k);
   const hipError_t ee = hipStreamEndCapture(b->stream, &g);
@@ -589,7 +616,7 @@ int graph_for(sa_batch *b, int k, hipGraphExec_t &out) {
   const hipError_t rc = hipGraphInstantiate(&e, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   if (rc != hipSuccess) return sa_fail(SA_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(rc));
-  b->graphs[k] = e;
+  b->graphs[key] = e;
   out = e;
   return SA_OK;
 }
@@ -723,7 +750,8 @@ void advance_host(sa_batch *b, int k, std::vector<int> &due) {
     const int before = in.t;
     in.t = std::min(in.nsweeps, in.t + k);
     in.lad->t = (uint64_t)in.t;
-    if (b->desc_fused[q] && ((in.t - before) & 1)) std::swap(in.lad->s, in.lad->s_alt);  // current array
+    const int m = b->desc_m[q], done = in.t - before;
+    if (m && ((done + m - 1) / m & 1)) std::swap(in.lad->s, in.lad->s_alt);  // each visit wrote the other array
     if (in.t >= in.nsweeps && before < in.nsweeps) b->dirty = true;
     if (in.pt.every && in.t > before && in.t % in.pt.every == 0) due.push_back(id);
   }
@@ -734,11 +762,20 @@ int sync_batch(sa_batch *b) {
   return SA_OK;
 }
 
+// frees what only the tile forms use (the ladder's stream must be idle)
+void drop_extras(sa_ladder *l) {
+  if (l->s_alt) (void)hipFree(l->s_alt);
+  if (l->jt) (void)hipFree(l->jt);
+  l->s_alt = nullptr;
+  l->jt = nullptr;
+  l->jt_current = false;
+}
+
 // Everything an instance needs on the device, done without touching the batch (so
 // it may run on any thread, while chunks execute): its ladder seeded like main,
 // tables uploaded on the ladder's own stream.
 int prepare_instance(int kind, int L, int nsys, uint64_t seed, int nsweeps, const double *T, int per_sweep, double h,
-                     const pt_state *pt, batch_inst &in) {
+                     const pt_state *pt, bool tiles, batch_inst &in) {
   sa_ladder *l = nullptr;
   int rc = sa_ladder_create(kind, L, nsys, &l);
   if (rc) return rc;
@@ -756,17 +793,23 @@ int prepare_instance(int kind, int L, int nsys, uint64_t seed, int nsweeps, cons
     sa_detail::make_table(kind, T[per_sweep && nsweeps == 0 ? q % nsys : q], h, tabs[q], f, nullptr);
     fast = fast && f;
   }
-  // a second spin array for the fused 3D sweep (read one, write the other)
-  int th_ = 0, mb_ = 0;
-  if (!rc && kFusedBatch && fused_cfg(l, th_, mb_) && !l->s_alt && hipMalloc(&l->s_alt, (size_t)nsys * l->N * 8) != hipSuccess) {
+  // what the tiles need beside the instance's own arrays; without it, half-sweeps
+  int form = !rc && fast && tiles ? tile_form(kind, L) : FORM_HALF;
+  if (two_arrays(form) && hipMalloc(&l->s_alt, (size_t)nsys * l->N * 8) != hipSuccess) {
     l->s_alt = nullptr;
-    rc = sa_fail(SA_ERR_NOMEM, "second spin array");
+    (void)hipGetLastError();
+    form = FORM_HALF;
+  }
+  if (form && kind == SA_KIND_3D && !sa_detail::tile3d_couplings(l)) {
+    drop_extras(l);
+    form = FORM_HALF;
   }
   in = batch_inst();
   in.lad = l;
   in.nsweeps = nsweeps;
   in.per_sweep = per_sweep ? 1 : 0;
   in.fast = fast;
+  in.form = form;
   in.work = (int64_t)half_items(kind, L) * nsys;
   if (!rc && hipMalloc(&in.tabs, sizeof(sa::sys_table) * ntab) != hipSuccess) rc = sa_fail(SA_ERR_NOMEM, "tables");
   // on the ladder's stream (waited for below): admission may run while a chunk is
@@ -784,14 +827,13 @@ int prepare_instance(int kind, int L, int nsys, uint64_t seed, int nsweeps, cons
     in = batch_inst();
     return rc;
   }
-  in.bytes = sa_detail::batch_instance_bytes(kind, L, nsys, nsweeps, per_sweep);
+  in.bytes = sa_detail::batch_instance_bytes(kind, L, nsys, nsweeps, per_sweep) + form_bytes(kind, L, nsys, form);
   if (pt) in.pt = *pt;
   return SA_OK;
 }
 
 void attach_instance(sa_batch *b, batch_inst &&in, int *id) {
   in.live = true;
-  in.s_first = in.lad->s;
   b->bytes_live += in.bytes;
   b->inst.push_back(std::move(in));
   *id = (int)b->inst.size() - 1;
@@ -801,7 +843,24 @@ void attach_instance(sa_batch *b, batch_inst &&in, int *id) {
 int add_instance(sa_batch *b, int kind, int L, int nsys, uint64_t seed, int nsweeps, const double *T, int per_sweep,
                  double h, pt_state *pt, int *id) {
   batch_inst in;
-  const int rc = prepare_instance(kind, L, nsys, seed, nsweeps, T, per_sweep, h, pt, in);
+  int rc = prepare_instance(kind, L, nsys, seed, nsweeps, T, per_sweep, h, pt, true, in);
+  if (rc == SA_ERR_NOMEM) {
+    // the instances' tile arrays give way to a new instance: all go back to half-sweeps
+    const int src = sync_batch(b);
+    if (src) return src;
+    for (batch_inst &x : b->inst)
+      if (x.live && x.form) {
+        const int64_t own = x.bytes - form_bytes(x.lad->kind, x.lad->L, x.lad->nsys, x.form);
+        const int lrc = sa_ladder_sync(x.lad);
+        if (lrc) return lrc;
+        drop_extras(x.lad);
+        x.form = FORM_HALF;
+        b->bytes_live += own - x.bytes;
+        x.bytes = own;
+        b->dirty = true;
+      }
+    rc = prepare_instance(kind, L, nsys, seed, nsweeps, T, per_sweep, h, pt, false, in);
+  }
   if (rc) return rc;
   attach_instance(b, std::move(in), id);
   return SA_OK;
@@ -842,7 +901,7 @@ int batch_geometry(int kind, int L, int nsys) {
 }
 
 int batch_prepare(int kind, int L, int nsys, uint64_t seed, int nsweeps, const double *T, int per_sweep, double h,
-                  int pt_every, prepared_instance **out) {
+                  int pt_every, bool tiles, prepared_instance **out) {
   *out = nullptr;
   int rc = batch_geometry(kind, L, nsys);
   if (rc) return rc;
@@ -850,9 +909,9 @@ int batch_prepare(int kind, int L, int nsys, uint64_t seed, int nsweeps, const d
   if (pt_every > 0) {
     if (nsys < 2 || nsweeps % pt_every) return sa_fail(SA_ERR_ARG, "bad parallel-tempering instance");
     pt_state pt = make_pt(nsys, T, h, pt_every);
-    rc = prepare_instance(kind, L, nsys, seed, nsweeps, pt.T.data(), 0, h, &pt, p->in);
+    rc = prepare_instance(kind, L, nsys, seed, nsweeps, pt.T.data(), 0, h, &pt, tiles, p->in);
   } else {
-    rc = prepare_instance(kind, L, nsys, seed, nsweeps, T, per_sweep, h, nullptr, p->in);
+    rc = prepare_instance(kind, L, nsys, seed, nsweeps, T, per_sweep, h, nullptr, tiles, p->in);
   }
   if (rc) return rc;
   *out = p.release();
@@ -874,22 +933,21 @@ void batch_discard(prepared_instance *p) {
 
 int64_t batch_instance_bytes(int kind, int L, int nsys, int nsweeps, int per_sweep) {
   const int ntab = per_sweep ? std::max(1, nsweeps) * nsys : nsys;
-  const int64_t N = (int64_t)L * L * (kind == SA_KIND_3D ? L : 1);
-  const bool second = kFusedBatch && kind == SA_KIND_3D && L % 4 == 0;  // fused-sweep ping-pong array
-  return ladder_bytes(kind, L, nsys) + (int64_t)sizeof(sa::sys_table) * ntab + (second ? (int64_t)nsys * N * 8 : 0);
+  return ladder_bytes(kind, L, nsys) + (int64_t)sizeof(sa::sys_table) * ntab;
 }
+
+int64_t batch_tile_bytes(int kind, int L, int nsys) { return form_bytes(kind, L, nsys, tile_form(kind, L)); }
 
 int batch_launch_chunk(sa_batch *b, int max_sweeps, int *k_out) {
   *k_out = 0;
   // fixed by the caller, tuned, or the next trial
   int trial = -1;
-  if ((!b->block || !b->chunk || !b->fused) && !(b->tuned_block && b->tuned_chunk && b->tuned_fused)) {
+  if ((!b->block || !b->chunk) && !(b->tuned_block && b->tuned_chunk)) {
     trial = (int)b->trials.size();
     if (trial >= kNumCands) {
       int best = 0;
       for (int q = 1; q < kNumCands; ++q)
         if (b->trials[q].second < b->trials[best].second) best = q;
-      b->tuned_fused = kCands[best].fused;
       b->tuned_block = kCands[best].block;
       b->tuned_chunk = kCands[best].chunk;
       trial = -1;
@@ -897,10 +955,8 @@ int batch_launch_chunk(sa_batch *b, int max_sweeps, int *k_out) {
   }
   const int bs = b->block ? b->block : (trial >= 0 ? kCands[trial].block : b->tuned_block);
   const int kfull = b->chunk ? b->chunk : (trial >= 0 ? kCands[trial].chunk : b->tuned_chunk);
-  const int fmode = b->fused ? b->fused : (trial >= 0 ? kCands[trial].fused : b->tuned_fused);
-  const bool fz = fmode == 2;
-  if (b->dirty || b->bmap_bs != bs || b->sched_fused != (fz ? 1 : 0)) {
-    const int rc = rebuild(b, bs, fz);
+  if (b->dirty || b->bmap_bs != bs) {
+    const int rc = rebuild(b, bs);
     if (rc) return rc;
   }
   if (b->ndesc == 0 || max_sweeps <= 0) return SA_OK;
@@ -981,9 +1037,6 @@ int sa_batch_destroy(sa_batch *b) {
     }
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
-  if (b->fork) (void)hipEventDestroy(b->fork);
-  for (auto e : b->side_done) (void)hipEventDestroy(e);
-  for (auto st : b->side) (void)hipStreamDestroy(st);
   hipStream_t s = b->stream;
   delete b;  // device arrays and staging buffers free themselves
   (void)hipStreamDestroy(s);
@@ -1107,7 +1160,7 @@ int sa_batch_set_tuning(sa_batch *b, int key, int value) {
     b->chunk = value;
   } else if (key == SA_TUNE_BATCH_FUSED) {
     if (value < 0 || value > 2) return sa_fail(SA_ERR_ARG, "batch fused must be 0 (auto), 1 (off) or 2 (on)");
-    if (value == 2 && !kFusedBatch) return sa_fail(SA_ERR_ARG, "the fused batch sweep is switched off in this build");
+    if (value == 2) return sa_fail(SA_ERR_ARG, "the fused batch sweep is switched off in this build");
     b->fused = value;
   } else {
     return sa_fail(SA_ERR_ARG, "unknown batch tuning key %d", key);
@@ -1120,7 +1173,7 @@ int sa_batch_get_tuning(sa_batch *b, int key, int *value) {
   if (!b || !value) return sa_fail(SA_ERR_ARG, "null argument");
   if (key == SA_TUNE_BATCH_BLOCK) *value = b->block ? b->block : b->tuned_block;
   else if (key == SA_TUNE_BATCH_CHUNK) *value = b->chunk ? b->chunk : b->tuned_chunk;
-  else if (key == SA_TUNE_BATCH_FUSED) *value = b->fused ? b->fused : b->tuned_fused;
+  else if (key == SA_TUNE_BATCH_FUSED) *value = 1;
   else return sa_fail(SA_ERR_ARG, "unknown batch tuning key %d", key);
   return SA_OK;
 }

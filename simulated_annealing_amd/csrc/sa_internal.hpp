@@ -98,10 +98,12 @@ bool batch_done(const sa_batch *b, int id);
 // An instance prepared off the batch (ladder seeded like main, tables uploaded),
 // from any thread; attaching it (loop thread) makes it part of the next chunk.
 // pt_every > 0: a parallel-tempering instance of nsys temperatures T exchanging
-// every pt_every sweeps (nsweeps a multiple of it).
+// every pt_every sweeps (nsweeps a multiple of it).  tiles: it may hold batch_tile_bytes
+// more for the LDS-resident sweeps (it takes the half-sweep kernels otherwise).
 struct prepared_instance;
 int batch_prepare(int kind, int L, int nsys, uint64_t seed, int nsweeps, const double *T, int per_sweep, double h,
-                  int pt_every, prepared_instance **out);
+                  int pt_every, bool tiles, prepared_instance **out);
+int64_t batch_tile_bytes(int kind, int L, int nsys);
 int batch_attach(sa_batch *b, prepared_instance *p, int *id);
 void batch_discard(prepared_instance *p);
 // an instance's ladder without waiting for the batch (only for an instance that

@@ -42,12 +42,18 @@ struct req_state {
   sa_request_result res{};
   int inst = -1;
   int64_t bytes = 0;
+  bool tiles = false;  // may take the LDS-resident sweeps
+  int64_t extra = 0;   // ... and hold this much beside `bytes` for them
   bool done = false;
 };
 
 int64_t request_bytes(const sa_request &r) {
   const int nsys = r.mode == SA_REQ_PT ? r.nT : 1;
   return sa_detail::batch_instance_bytes(r.kind, r.L, nsys, r.nsweeps, r.mode == SA_REQ_PT ? 0 : 1);
+}
+
+int64_t request_extra(const sa_request &r) {
+  return sa_detail::batch_tile_bytes(r.kind, r.L, r.mode == SA_REQ_PT ? r.nT : 1);
 }
 
 double request_attempts(const sa_request &r) {
@@ -114,14 +120,14 @@ req_state &req(sa_serve *s, int64_t id) {
 }
 
 // the device state of a request, on a preparation thread
-int prepare_request(const sa_request &r, sa_detail::prepared_instance **out) {
+int prepare_request(const sa_request &r, bool tiles, sa_detail::prepared_instance **out) {
   int rc = sa_request_temperatures(&r, nullptr, 0);
   if (rc < 0) return rc;
   std::vector<double> T(rc);
   sa_request_temperatures(&r, T.data(), (int64_t)T.size());
   if (r.mode == SA_REQ_PT)
-    return sa_detail::batch_prepare(r.kind, r.L, r.nT, r.seed, r.nsweeps, T.data(), 0, r.h, r.every, out);
-  return sa_detail::batch_prepare(r.kind, r.L, 1, r.seed, r.nsweeps, T.data(), 1, r.h, 0, out);
+    return sa_detail::batch_prepare(r.kind, r.L, r.nT, r.seed, r.nsweeps, T.data(), 0, r.h, r.every, tiles, out);
+  return sa_detail::batch_prepare(r.kind, r.L, 1, r.seed, r.nsweeps, T.data(), 1, r.h, 0, tiles, out);
 }
 
 void worker_main(sa_serve *s) {
@@ -129,6 +135,7 @@ void worker_main(sa_serve *s) {
   for (;;) {
     int64_t id;
     sa_request r;
+    bool tiles;
     {
       std::unique_lock<std::mutex> g(s->mu);
       s->cv_jobs.wait(g, [&] { return s->stopping || !s->jobs.empty(); });
@@ -136,9 +143,10 @@ void worker_main(sa_serve *s) {
       id = s->jobs.front();
       s->jobs.pop_front();
       r = s->reqs[id].r;
+      tiles = s->reqs[id].tiles;
     }
     sa_detail::prepared_instance *p = nullptr;
-    const int rc = prepare_request(r, &p);
+    const int rc = prepare_request(r, tiles, &p);
     {
       std::lock_guard<std::mutex> g(s->mu);
       s->ready.push_back({id, rc, p});
@@ -211,7 +219,7 @@ int read_results(sa_serve *s, int64_t id) {
 int release(sa_serve *s, int64_t id) {
   req_state &q = req(s, id);
   const int rc = sa_batch_remove(s->b, q.inst);
-  s->bytes -= q.bytes;
+  s->bytes -= q.bytes + q.extra;
   q.inst = -1;
   return rc;
 }
@@ -237,7 +245,14 @@ void dispatch_arrived(sa_serve *s) {
         break;  // wait for memory / a slot (arrival order is kept)
       s->pending.pop_front();
       q.res.admitted = s->now();
-      s->bytes += q.bytes;
+      // the tiles' arrays come out of the budget too, while half of it is free: a tight
+      // budget is left to the requests themselves
+      const int64_t want = request_extra(q.r);
+      if (s->bytes + q.bytes + want <= s->cfg.hbm_budget / 2) {
+        q.tiles = true;
+        q.extra = want;
+      }
+      s->bytes += q.bytes + q.extra;
       s->peak_bytes = std::max(s->peak_bytes, s->bytes);
       s->preparing += 1;
       s->jobs.push_back(id);
@@ -262,7 +277,7 @@ void attach_ready(sa_serve *s) {
     std::lock_guard<std::mutex> g(s->mu);
     s->preparing -= 1;
     if (rc) {
-      s->bytes -= q.bytes;
+      s->bytes -= q.bytes + q.extra;
       finish_locked(s, it.id, rc);
       continue;
     }

@@ -13,13 +13,10 @@ constexpr size_t kMaxLds = 160 * 1024;
 
 struct tile_cfg {
   bool whole;
-  int tx, ty, S, G, C, lg, lp, threads, ns, w0, w1;
+  int S, threads, ns;
+  size_t lds;
+  sa::tile3d_args a;  // geometry only
 };
-
-size_t lds_bytes(const tile_cfg &c, int L) {
-  const int W = c.whole ? L : c.tx + 4, H = c.whole ? L : c.ty + 4;
-  return ((size_t)W * H * c.lp + (L & 1 ? sa::odd_list_words(W, H) : 0)) * 8;
-}
 
 // The tile of the next launch: the one with the least modelled time per sweep, in us.
 // Fitted to 60 measured shapes (3D L 8..128, 1..32 systems), within 25%: a launch with its
@@ -37,32 +34,24 @@ tile_cfg pick(const sa_ladder *l, int64_t left, double &cost) {
   auto consider = [&](bool whole, int tx, int ty, int S) {
     tile_cfg c{};
     c.whole = whole;
-    c.tx = whole ? L : tx;
-    c.ty = whole ? L : ty;
     c.S = S;
-    c.G = (L + S - 1) / S;
-    if (c.G < 2 || c.G > 64) return;
-    c.lg = 1;
-    while ((1 << c.lg) < c.G) ++c.lg;
-    c.C = 64 >> c.lg;
-    const int W = whole ? L : tx + 4, H = whole ? L : ty + 4;
-    if (odd && !whole && (W > L || H > L)) return;
-    c.lp = sa::column_stride(L) % 4 == 0 ? sa::column_stride(L) + 2 : sa::column_stride(L);
-    if (lds_bytes(c, L) > kMaxLds) return;
-    // odd sides: one more column per row at most
-    const int col0 = whole ? (L * L + 1) / 2 : (tx / 2 + 1) * (ty + 2), col1 = whole ? L * L / 2 : tx / 2 * ty;
-    c.w0 = (col0 + c.C - 1) / c.C;
-    c.w1 = (col1 + c.C - 1) / c.C;
-    c.threads = std::max(std::min(16, c.w0) * 64, (H * W / (odd ? 1 : 2) + 63) / 64 * 64);
-    if (c.threads > 1024) return;
+    const int W = whole ? L : tx + 4, H = whole ? L : ty + 4, row = odd ? W : W / 2;
+    if (row * H > 1024) return;
+    // first for a full block, to learn the waves the columns make
+    if (!sa::tile3d_setup(c.a, L, whole, tx, ty, S, 1024)) return;
+    c.threads = std::max(std::min(16, c.a.chunks0) * 64, (row * H + 63) / 64 * 64);
+    c.lds = sa::tile3d_setup(c.a, L, whole, tx, ty, S, c.threads);
+    if (!c.lds || c.lds > kMaxLds) return;
     c.ns = whole ? (int)std::min<int64_t>(left, 64) : 1;
-    const int64_t tiles = whole ? 1 : (int64_t)((L + tx - 1) / tx) * ((L + ty - 1) / ty);
+    const int64_t tiles = (int64_t)c.a.ntx * c.a.nty;
     if (tiles * l->nsys >= (int64_t)1 << 24) return;
     const double per_cu = std::ceil((double)tiles * l->nsys / 256);
     const double wave = S == 2 ? (general ? 0.195 : 0.13) : (general ? 0.29 : 0.25);
-    const double words = (double)l->nsys * l->N, amp = (double)(W * H) / (c.tx * c.ty);
+    const double words = (double)l->nsys * l->N, amp = (double)(W * H) / (c.a.tx * c.a.ty);
     // odd sides: up to three more stages
-    const double t = ((S == 2 ? 4.6 : 6.3) + (odd ? 2.5 : 0) + words * 8 * (amp + 1) / 8e6) / c.ns + per_cu * (c.w0 + c.w1) * wave + (odd && whole ? 2.5 : 0);
+    const double stages = odd ? 2.5 : 0;
+    const double t = ((S == 2 ? 4.6 : 6.3) + words * 8 * (amp + 1) / 8e6) / c.ns + stages +
+                     per_cu * (c.a.chunks0 + c.a.chunks1) * wave;
     if (t < cost) {
       cost = t;
       best = c;
@@ -80,7 +69,7 @@ tile_cfg pick(const sa_ladder *l, int64_t left, double &cost) {
 template <bool COUNTER, bool FAST, int S>
 void launch(const sa::tile3d_args &t, const tile_cfg &c, hipStream_t st) {
   const dim3 grid((unsigned)((t.ntx * t.nty * t.a.nsys + 7) / 8 * 8));
-  const size_t lds = lds_bytes(c, t.a.L);
+  const size_t lds = c.lds;
   auto go = [&](auto whole, auto one) {
     constexpr bool WH = decltype(whole)::value, ON = decltype(one)::value;
     static const hipError_t more = hipFuncSetAttribute((const void *)sa::k_tile3d<COUNTER, FAST, S, WH, ON>,
@@ -98,7 +87,7 @@ void launch(const sa::tile3d_args &t, const tile_cfg &c, hipStream_t st) {
     };
     return c.whole ? go_odd(std::true_type{}) : go_odd(std::false_type{});
   }
-  const bool one = c.w0 * 64 <= c.threads;
+  const bool one = c.a.chunks0 * 64 <= c.threads;
   if constexpr (S == 2) {  // the kept couplings fit the registers
     if (one) return c.whole ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
   }
@@ -149,7 +138,7 @@ void sa_detail::tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t ta
                               uint64_t t, int64_t left) {
   double cost = 0;
   const tile_cfg c = pick(l, left, cost);
-  sa::tile3d_args a{};
+  sa::tile3d_args a = c.a;
   a.a.s = l->s;
   a.a.jx = l->jx;
   a.a.jy = l->jy;
@@ -162,30 +151,10 @@ void sa_detail::tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t ta
   a.a.L = l->L;
   a.a.nsys = l->nsys;
   a.out = c.whole ? l->s : l->s_alt;
-  a.tx = c.tx;
-  a.ty = c.ty;
-  a.ntx = (l->L + c.tx - 1) / c.tx;
-  a.nty = (l->L + c.ty - 1) / c.ty;
-  a.G = c.G;
-  a.C = c.C;
-  a.lg = c.lg;
-  a.lp = c.lp;
   a.jxt = l->jt;
   const int64_t jn = (int64_t)l->L * l->L * sa::column_stride(l->L);
   a.jyt = l->jt + jn;
   a.jzt = l->jt + 2 * jn;
-  a.chunks0 = c.w0;
-  a.chunks1 = c.w1;
-  auto recip = [](int d) { return ((1 << 20) + d - 1) / d; };
-  const int W = c.whole ? l->L : c.tx + 4, H = c.whole ? l->L : c.ty + 4;
-  const int row = l->L & 1 ? W : W / 2;  // columns or pairs of columns a thread loads
-  a.recip_pairs = recip(row * H);
-  a.recip_hw = recip(row);
-  a.recip_ntx = recip(a.ntx);
-  a.recip_per = (uint32_t)((((uint64_t)1 << 32) + a.ntx * a.nty - 1) / (a.ntx * a.nty));  // not used with one tile
-  a.zstep = c.threads / (row * H);
-  a.recip_n0 = recip(c.whole ? l->L / 2 : c.tx / 2 + 1);
-  a.recip_n1 = recip(c.whole ? l->L / 2 : c.tx / 2);
   a.ns = c.ns;
   a.tab_step = tab_step;
   const bool counter = l->rng_mode == SA_RNG_COUNTER;

@@ -27,6 +27,8 @@
 // L=16, held whole, 9.5 -> 2.9; 8 of L=48 with a field 37 -> 19.5.
 #pragma once
 
+#include <algorithm>
+
 #include "sa_kernels.hpp"
 #include "sa_tile2d.hpp"
 
@@ -47,6 +49,43 @@ struct tile3d_args {
   int ns;            // sweeps (1 unless WHOLE)
   int64_t tab_step;  // tables per sweep
 };
+
+__host__ __device__ __forceinline__ int column_stride(int L);
+__host__ __device__ __forceinline__ int odd_list_words(int W, int H);
+
+// The geometry part of the arguments for a tile of tx x ty columns (whole: L x L), S planes
+// per segment and blocks of `threads`; chunks0 / chunks1 are set too.  Returns the LDS bytes,
+// 0 where the form does not apply.
+inline size_t tile3d_setup(tile3d_args &a, int L, bool whole, int tx, int ty, int S, int threads) {
+  const bool odd = L & 1;
+  a.tx = whole ? L : tx;
+  a.ty = whole ? L : ty;
+  const int W = whole ? L : tx + 4, H = whole ? L : ty + 4;
+  if (!whole && (tx > L || ty > L || (odd && (W > L || H > L)))) return 0;
+  a.ntx = (L + a.tx - 1) / a.tx;
+  a.nty = (L + a.ty - 1) / a.ty;
+  a.G = (L + S - 1) / S;
+  if (a.G < 2 || a.G > 64) return 0;
+  a.lg = 1;
+  while ((1 << a.lg) < a.G) ++a.lg;
+  a.C = 64 >> a.lg;
+  a.lp = column_stride(L) % 4 == 0 ? column_stride(L) + 2 : column_stride(L);
+  // odd sides: one more column per row at most
+  const int col0 = whole ? (L * L + 1) / 2 : (tx / 2 + 1) * (ty + 2), col1 = whole ? L * L / 2 : tx / 2 * ty;
+  a.chunks0 = (col0 + a.C - 1) / a.C;
+  a.chunks1 = (col1 + a.C - 1) / a.C;
+  auto recip = [](int d) { return ((1 << 20) + d - 1) / d; };
+  const int row = odd ? W : W / 2;  // columns or pairs of columns a thread loads
+  if (row * H > threads) return 0;
+  a.zstep = threads / (row * H);
+  a.recip_pairs = recip(row * H);
+  a.recip_hw = recip(row);
+  a.recip_ntx = recip(a.ntx);
+  a.recip_per = (uint32_t)((((uint64_t)1 << 32) + a.ntx * a.nty - 1) / (a.ntx * a.nty));  // not used with one tile
+  a.recip_n0 = recip(whole ? std::max(L / 2, 1) : tx / 2 + 1);
+  a.recip_n1 = recip(whole ? std::max(L / 2, 1) : tx / 2);
+  return ((size_t)W * H * a.lp + (odd ? odd_list_words(W, H) : 0)) * 8;
+}
 
 // the two outcomes of a site's update as functions of the bond below it
 struct flips {
