@@ -78,6 +78,8 @@ bool compact_table(int kind, const sa::sys_table &tab);
 // Asynchronous on st; the caller sums the copies.
 void launch_measure(int kind, int L, int64_t N, const uint64_t *s, const uint64_t *jx, const uint64_t *jy,
                     const uint64_t *jz, int n, const int *dlist, sa::sys4 sel, int *cnt, hipStream_t st);
+// sa_digest of all systems' spins in order, computed on the device
+int ladder_digest(sa_ladder *l, uint64_t *digest);
 // device bytes sa_ladder_create allocates for a ladder (the fused 3D sweep's second
 // spin array, allocated on first use, not included)
 int64_t ladder_bytes(int kind, int L, int nsys);

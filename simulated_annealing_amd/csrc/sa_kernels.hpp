@@ -1589,6 +1589,27 @@ static __global__ void k_fill_zero(int *p, int n) {
   if (i < n) p[i] = 0;
 }
 
+// ---------------------------------------------------------------- digest
+// XOR over i < n of the splitmix64 finaliser of w[i] + i * golden (sa_digest with first
+// index 0), into *out (zeroed by the caller).  Memory-bound: each word is read once.
+static __global__ void __launch_bounds__(256) k_digest(const uint64_t *__restrict__ w, int64_t n,
+                                                       unsigned long long *out) {
+  uint64_t d = 0;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    uint64_t z = w[i] + (uint64_t)i * 0x9E3779B97F4A7C15ULL;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
+    d ^= z ^ (z >> 31);
+  }
+#pragma unroll
+  for (int s = 32; s; s >>= 1) d ^= __shfl_xor(d, s);
+  __shared__ uint64_t part[4];
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = d;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicXor(out, (unsigned long long)(part[0] ^ part[1] ^ part[2] ^ part[3]));
+}
+
 // ---------------------------------------------------------------- masked swap
 // a ^= (a^b) & m, b ^= (a^b) & m (src/device.cuh:18-23)
 static __global__ void __launch_bounds__(256) k_swap(uint64_t *a, uint64_t *b, uint64_t mask, int64_t N) {

@@ -183,14 +183,11 @@ int read_results(sa_serve *s, int64_t id) {
   std::memcpy(res.E, E.data(), sizeof res.E);
   std::memcpy(res.M, M.data(), sizeof res.M);
   if (s->cfg.digests) {
-    const int64_t N = sa_ladder_sites(l);
-    std::vector<uint64_t> w((size_t)N);
+    // on the device: reading 24 requests' 48 MB of spins back and hashing them took the
+    // host 21 ms, a third of their service time
     uint64_t d = 0;
-    for (int j = 0; j < nsys; ++j) {
-      rc = sa_ladder_get_spins(l, j, w.data());
-      if (rc) return rc;
-      d ^= sa_digest(w.data(), N, (uint64_t)j * (uint64_t)N);
-    }
+    rc = sa_detail::ladder_digest(l, &d);
+    if (rc) return rc;
     res.spins_digest = d;
   }
   if (q.r.mode == SA_REQ_PT) {

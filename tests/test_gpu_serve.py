@@ -151,3 +151,16 @@ def test_serve_online_submission_from_another_thread(sa):
         d, E, M, _ = alone(sa, r)
         assert x.spins_digest == d
     srv.close()
+
+
+@pytest.mark.parametrize("kind,L,nT", [(1, 3, 2), (1, 16, 1), (2, 9, 5), (2, 24, 3)])
+def test_served_digest_is_the_digest_of_the_spins(sa, kind, L, nT):
+    """the digest is computed on the device: sizes below one block, odd, and of several blocks"""
+    mode = sa.REQ_PT if nT > 1 else sa.REQ_ANNEAL
+    r = sa.make_request(kind, L, mode, 10, 4321, nT=nT, every=10)
+    srv = sa.Server()
+    srv.submit(r)
+    srv.run()
+    d, _, _, _ = alone(sa, r)
+    assert srv.results()[0].spins_digest == d
+    srv.close()
