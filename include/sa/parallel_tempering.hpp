@@ -16,6 +16,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <fstream>
 #include <iostream>
 #include <map>
@@ -23,6 +24,7 @@
 #include <regex>
 #include <string>
 #include <type_traits>
+#include <typeinfo>
 #include <vector>
 
 #include "sa/annealing.hpp"
@@ -67,8 +69,22 @@ class parallel_tempering {
     }
   }
 
+  // n x step(0); one device wait for all of them where every system is a slot of one ladder
+  // (on_device), otherwise one by one
+  void steps(int n) {
+    if (n > 0 && on_device()) {
+      steps_on_device(n);
+      return;
+    }
+    for (int k = 0; k < n; ++k) step(0);
+  }
+
   // src/parallel_tempering.hpp:81-115
   void step(int stride) {
+    if (stride == 0 && on_device()) {
+      steps_on_device(1);
+      return;
+    }
     const bool grouped = stride == 0 && all_on_ladders();
     int i;
     double u;
@@ -300,6 +316,76 @@ class parallel_tempering {
     }
     num_switch_[i](a / (double)64.);
     return mask;
+  }
+
+  // Whether whole steps can run on the device: every system of exactly this project's
+  // classes (a derived class may override swap or measure), all on one ladder, at finite
+  // temperatures whose inverses do not increase (exchange_threshold).
+  bool on_device() const {
+    if (sys_.size() < 2 || steps_ < 1 || T_.size() != sys_.size()) return false;
+    const ladder *l = nullptr;
+    for (system *s : sys_) {
+      hip_sys *h = as_hip(s);
+      if (!h || !plain(*h)) return false;
+      if (l && h->get_ladder().get() != l) return false;
+      l = h->get_ladder().get();
+    }
+    for (size_t i = 0; i + 1 < T_.size(); ++i)
+      if (!(1. / T_[i] - 1. / T_[i + 1] >= 0.) || !std::isfinite(1. / T_[i]) || as_hip(sys_[i])->index() == as_hip(sys_[i + 1])->index())
+        return false;
+    return std::isfinite(1. / T_.back());
+  }
+  static bool plain(const hip_sys &h) {
+    const std::type_info &t = typeid(h);
+    return t == typeid(hip_sys) || t == typeid(::hip_3d) || t == typeid(::hip_2d) || t == typeid(::hip_2d_periodic);
+  }
+  // step(0) n times: the pairs and uniforms do not depend on the energies, so all are drawn
+  // first (in step's order), the device decides each exchange by the threshold that the
+  // uniform comes to, and the energies and masks are folded in afterwards as step does.
+  void steps_on_device(int n) {
+    ladder *l = as_hip(sys_[0])->get_ladder().get();
+    std::vector<int> pair(n), a(n), b(n);
+    std::vector<double> u(n), ha(n), hb(n);
+    std::vector<float> thr(n);
+    for (int k = 0; k < n; ++k) {
+      const int i = uniform_int(gen_, uni_a_, uni_b_);
+      pair[k] = i;
+      u[k] = canonical32(gen_);
+      hip_sys *x = as_hip(sys_[i]), *y = as_hip(sys_[i + 1]);
+      a[k] = x->index();
+      b[k] = y->index();
+      ha[k] = x->get_h();
+      hb[k] = y->get_h();
+      thr[k] = exchange_threshold(1. / T_[i] - 1. / T_[i + 1], u[k]);
+    }
+    std::vector<uint64_t> masks(n);
+    std::vector<int32_t> EM((size_t)n * 384);
+    const int rc = sa_ladder_exchange_steps(l->get(), (int)steps_, n, as_hip(sys_[0])->index(), a.data(), b.data(),
+                                            thr.data(), ha.data(), hb.data(), masks.data(), EM.data());
+    if (rc != SA_OK) {
+      log_error("exchange steps", rc);
+      return;
+    }
+    const double h0 = as_hip(sys_[0])->get_h();
+    for (int k = 0; k < n; ++k) {
+      if (steps_ > 1) min_E_update();
+      const int i = pair[k];
+      stale_.assign(sys_.size(), 1);
+      const double h[3] = {h0, ha[k], hb[k]};
+      const int to[3] = {0, i, i + 1};
+      for (int r = 0; r < 3; ++r) {
+        const int32_t *e = EM.data() + (size_t)k * 384 + r * 128, *m = e + 64;
+        std::vector<float> &E = E_[to[r]];
+        E.resize(64);
+        for (int q = 0; q < 64; ++q) E[q] = (float)((double)e[q] + h[r] * (double)m[q]);
+        stale_[to[r]] = 0;
+      }
+      min_E_update();
+      int acc = 0;
+      for (uint64_t w = masks[k]; w; w &= w - 1) ++acc;
+      num_switch_[i](acc / (double)64.);
+      if (log_) log_->push_back(swap_record{i, u[k], masks[k]});
+    }
   }
 
   void min_E_update() {

@@ -153,6 +153,15 @@ int sa_measure_noalloc(int kind, int L, int nsys, const uint64_t *s, const uint6
  * (swap, src/gpu_3d.cu:310-328, src/cpu_3d.cpp:429-444). */
 int sa_ladder_swap(sa_ladder *l, int a, int b, uint64_t mask);
 
+/* nsteps parallel-tempering steps with the exchange decided on the device (the drivers use
+ * it; one wait for all steps).  Step k: `sweeps` sweeps of every system, measurement of
+ * systems cold, a[k], b[k], then the exchange of the lanes with
+ *   -(e_a - e_b) >= min_dE[k],   e_s = float(E_s + h_s * M_s),
+ * ha[k], hb[k] the two fields.  masks[k]: the exchanged lanes.  EM[k][3][2][64]: E and M of
+ * cold, a[k] and b[k] before the exchange. */
+int sa_ladder_exchange_steps(sa_ladder *l, int sweeps, int nsteps, int cold, const int *a, const int *b,
+                             const float *min_dE, const double *ha, const double *hb, uint64_t *masks, int32_t *EM);
+
 /* Kernel tuning (no effect on results; 0 = automatic everywhere).
  *   SA_TUNE_SYS_PER_THREAD  systems one thread updates per site (1, 2 or 4, must
  *                           divide nsys): more share coupling loads and random words

@@ -66,7 +66,7 @@ int sa_pt_create(int kind, int L, int nT, const double *T, double h, uint64_t se
 
 int sa_pt_step(sa_pt *p, int nsteps) {
   if (!p || nsteps < 0) return SA_ERR_ARG;
-  for (int k = 0; k < nsteps; ++k) p->pt->step(0);
+  p->pt->steps(nsteps);
   p->done += nsteps;
   return SA_OK;
 }

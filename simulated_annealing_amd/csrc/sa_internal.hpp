@@ -46,6 +46,10 @@ struct sa_ladder {
   std::vector<int> cnt_h;  // host copy of the measurement counters
   int *cnt_pin = nullptr;  // pinned landing buffer of the counters (allocated at the first measurement)
   hipEvent_t meas_ev = nullptr;  // recorded after the counters' copy; polled
+  int *xcnt = nullptr;     // counters of a run of exchange steps (allocated at the first)
+  char *x_pin = nullptr;   // pinned: their masks, then E and M
+  bool words_busy = false;  // replay: the staged words may still be on their way (words_ev)
+  hipEvent_t words_ev = nullptr;
   int *sys_list = nullptr;  // device copy of a measured subset (more than 4 systems)
   int sys_per_thread = 0;  // SA_TUNE_SYS_PER_THREAD, 0 = automatic
   int sweep3d_kernel = 0;  // SA_TUNE_SWEEP3D_KERNEL, 0 = automatic
@@ -72,12 +76,13 @@ void make_table(int kind, double T, double h, sa::sys_table &tab, bool &fast, do
 // every table of the kind is compact
 bool compact_table(int kind, const sa::sys_table &tab);
 // Measurement of n systems of s (nsys x N words; listed by dlist in device memory,
-// by sel for up to four, else systems 0..n-1): clears cnt (kMeasureCopies x n x 128
+// by sel for up to four, else systems 0..n-1): clears (if asked) cnt (kMeasureCopies x n x 128
 // ints) with a fill kernel, then per copy, listed system and lane the satisfied
 // -x,-y[,-z] bonds (cnt[..][j][0][lane]) and set spins (cnt[..][j][1][lane]).
 // Asynchronous on st; the caller sums the copies.
 void launch_measure(int kind, int L, int64_t N, const uint64_t *s, const uint64_t *jx, const uint64_t *jy,
-                    const uint64_t *jz, int n, const int *dlist, sa::sys4 sel, int *cnt, hipStream_t st);
+                    const uint64_t *jz, int n, const int *dlist, sa::sys4 sel, int *cnt, hipStream_t st,
+                    bool clear = true);
 // sa_digest of all systems' spins in order, computed on the device
 int ladder_digest(sa_ladder *l, uint64_t *digest);
 // device bytes sa_ladder_create allocates for a ladder (the fused 3D sweep's second

@@ -46,6 +46,9 @@ void free_all(sa_ladder *l) {
   if (l->sys_list) (void)hipFree(l->sys_list);
   if (l->cnt_pin) (void)hipHostFree(l->cnt_pin);
   if (l->meas_ev) (void)hipEventDestroy(l->meas_ev);
+  if (l->words_ev) (void)hipEventDestroy(l->words_ev);
+  if (l->xcnt) (void)hipFree(l->xcnt);
+  if (l->x_pin) (void)hipHostFree(l->x_pin);
   if (l->stream) (void)hipStreamDestroy(l->stream);
 }
 
@@ -55,8 +58,18 @@ int check_sys(const sa_ladder *l, int sys) {
   return SA_OK;
 }
 
+// the staged replay words are free to be overwritten
+int words_idle(sa_ladder *l) {
+  if (l->words_busy) SA_HIP_TRY(hipEventSynchronize(l->words_ev));
+  l->words_busy = false;
+  return SA_OK;
+}
+
 int ensure_words(sa_ladder *l, int64_t sweeps) {
+  if (!l->words_ev) SA_HIP_TRY(hipEventCreateWithFlags(&l->words_ev, hipEventDisableTiming));
   if (l->words_cap >= sweeps) return SA_OK;
+  SA_HIP_TRY(hipStreamSynchronize(l->stream));  // launched sweeps may still read the old buffers
+  l->words_busy = false;
   if (l->words_d) (void)hipFree(l->words_d);
   if (l->words_h) (void)hipHostFree(l->words_h);
   l->words_d = nullptr;
@@ -642,9 +655,10 @@ void sa_detail::make_table(int kind, double T, double h, sa::sys_table &t, bool 
 }
 
 void sa_detail::launch_measure(int kind, int L, int64_t N, const uint64_t *s, const uint64_t *jx, const uint64_t *jy,
-                               const uint64_t *jz, int n, const int *dlist, sa::sys4 sel, int *cnt, hipStream_t st) {
+                               const uint64_t *jz, int n, const int *dlist, sa::sys4 sel, int *cnt, hipStream_t st,
+                               bool clear) {
   const int all_n = 128 * n * sa::measure_copies(n);
-  hipLaunchKernelGGL(sa::k_fill_zero, dim3((all_n + 255) / 256), dim3(256), 0, st, cnt, all_n);
+  if (clear) hipLaunchKernelGGL(sa::k_fill_zero, dim3((all_n + 255) / 256), dim3(256), 0, st, cnt, all_n);
   // cnt layout [copy][listed system][2][64] (the caller sums the copies).  Two systems
   // per block share its coupling loads; one when at most 4 are measured (the exchange
   // step), for more waves in flight.  Steps per thread: as many as leave about 4 blocks
@@ -760,11 +774,14 @@ int sa_ladder_sweep(sa_ladder *l, int nsweeps) {
   if (rc) return rc;
   for (int64_t done = 0; done < nsweeps;) {
     const int64_t n = std::min<int64_t>(per_chunk, nsweeps - done);
+    rc = words_idle(l);  // waits for the previous words' upload, not for its sweeps
+    if (rc) return rc;
     l->eng.fill(l->words_h, n * l->N);
     SA_HIP_TRY(hipMemcpyAsync(l->words_d, l->words_h, n * l->N * 8, hipMemcpyHostToDevice, l->stream));
+    SA_HIP_TRY(hipEventRecord(l->words_ev, l->stream));
+    l->words_busy = true;
     rc = launch_sweeps(l, l->words_d, l->t + done, n);
     if (rc) return rc;
-    SA_HIP_TRY(hipStreamSynchronize(l->stream));
     done += n;
   }
   l->t += nsweeps;
@@ -772,6 +789,23 @@ int sa_ladder_sweep(sa_ladder *l, int nsweeps) {
 }
 
 namespace {
+
+// Waits for everything enqueued.  The host polls an event instead of sleeping in a stream
+// synchronisation: the replica-exchange step waits here between sweeps.
+int wait_stream(sa_ladder *l) {
+  if (!l->meas_ev && hipEventCreateWithFlags(&l->meas_ev, hipEventDisableTiming) != hipSuccess) {
+    l->meas_ev = nullptr;
+    (void)hipGetLastError();
+    SA_HIP_TRY(hipStreamSynchronize(l->stream));
+    return SA_OK;
+  }
+  SA_HIP_TRY(hipEventRecord(l->meas_ev, l->stream));
+  hipError_t e;
+  while ((e = hipEventQuery(l->meas_ev)) == hipErrorNotReady) {
+  }
+  SA_HIP_TRY(e);
+  return SA_OK;
+}
 
 // energies/magnetisations of `n` systems (list = nullptr: systems 0..n-1); results
 // land in cnt_h[(2*j)*64 ...] for the j-th listed system
@@ -789,26 +823,16 @@ int measure_list(sa_ladder *l, const int *list, int n) {
   sa_detail::launch_measure(l->kind, l->L, l->N, l->s, l->jx, l->jy, l->jz, n, dlist, sel, l->cnt, l->stream);
   SA_HIP_TRY(hipGetLastError());
   // The counters land in pinned memory allocated at the first measurement (so
-  // creating a ladder, e.g. per served request, needs no pinned allocation) and the
-  // host polls an event instead of sleeping in a stream synchronisation: the
-  // replica-exchange step waits on this between sweeps.
+  // creating a ladder, e.g. per served request, needs no pinned allocation).
   if (!l->cnt_pin &&
       hipHostMalloc((void **)&l->cnt_pin, sizeof(int) * 128 * l->nsys * sa::kMeasureCopies, hipHostMallocDefault) !=
           hipSuccess)
     l->cnt_pin = nullptr;
-  if (!l->meas_ev && hipEventCreateWithFlags(&l->meas_ev, hipEventDisableTiming) != hipSuccess) l->meas_ev = nullptr;
-  if (l->cnt_pin && l->meas_ev) {
-    SA_HIP_TRY(hipMemcpyAsync(l->cnt_pin, l->cnt, sizeof(int) * all_n, hipMemcpyDeviceToHost, l->stream));
-    SA_HIP_TRY(hipEventRecord(l->meas_ev, l->stream));
-    hipError_t e;
-    while ((e = hipEventQuery(l->meas_ev)) == hipErrorNotReady) {
-    }
-    SA_HIP_TRY(e);
-    std::memcpy(l->cnt_h.data(), l->cnt_pin, sizeof(int) * all_n);
-  } else {
-    SA_HIP_TRY(hipMemcpyAsync(l->cnt_h.data(), l->cnt, sizeof(int) * all_n, hipMemcpyDeviceToHost, l->stream));
-    SA_HIP_TRY(hipStreamSynchronize(l->stream));
-  }
+  int *to = l->cnt_pin ? l->cnt_pin : l->cnt_h.data();
+  SA_HIP_TRY(hipMemcpyAsync(to, l->cnt, sizeof(int) * all_n, hipMemcpyDeviceToHost, l->stream));
+  const int rc = wait_stream(l);
+  if (rc) return rc;
+  if (to != l->cnt_h.data()) std::memcpy(l->cnt_h.data(), to, sizeof(int) * all_n);
   // sum the copies into the first
   for (int c = 1; c < sa::measure_copies(n); ++c)
     for (int q = 0; q < cnt_n; ++q) l->cnt_h[q] += l->cnt_h[(size_t)c * cnt_n + q];
@@ -945,6 +969,70 @@ int sa_ladder_swap(sa_ladder *l, int a, int b, uint64_t mask) {
   hipLaunchKernelGGL(sa::k_swap, dim3((unsigned)blocks), dim3(256), 0, l->stream, l->s + (int64_t)a * l->N,
                      l->s + (int64_t)b * l->N, mask, l->N);
   SA_HIP_TRY(hipGetLastError());
+  return SA_OK;
+}
+
+int sa_ladder_exchange_steps(sa_ladder *l, int sweeps, int nsteps, int cold, const int *a, const int *b,
+                             const float *min_dE, const double *ha, const double *hb, uint64_t *masks, int32_t *EM) {
+  int rc = check_sys(l, cold);
+  if (rc) return rc;
+  if (!a || !b || !min_dE || !ha || !hb || !masks || !EM || sweeps < 0 || nsteps < 0)
+    return sa_fail(SA_ERR_ARG, "exchange steps: bad argument");
+  for (int k = 0; k < nsteps; ++k) {
+    if ((rc = check_sys(l, a[k])) || (rc = check_sys(l, b[k]))) return rc;
+    if (a[k] == b[k]) return sa_fail(SA_ERR_ARG, "exchange of system %d with itself", a[k]);
+  }
+  constexpr int kRun = 128;  // steps between waits
+  constexpr int kCnt = 3 * 128 * sa::kMeasureCopies;
+  constexpr size_t kRec = 384 * sizeof(int32_t);
+  if (!l->xcnt && hipMalloc(&l->xcnt, sizeof(int) * kCnt * kRun) != hipSuccess) {
+    l->xcnt = nullptr;
+    return sa_fail(SA_ERR_NOMEM, "exchange counters");
+  }
+  if (!l->x_pin && hipHostMalloc((void **)&l->x_pin, kRun * (8 + kRec), hipHostMallocDefault) != hipSuccess) {
+    l->x_pin = nullptr;
+    return sa_fail(SA_ERR_NOMEM, "pinned exchange records");
+  }
+  unsigned long long *mask_pin = (unsigned long long *)l->x_pin;
+  int32_t *em_pin = (int32_t *)(l->x_pin + kRun * 8);
+  const int64_t bonds = bonds_per_site(l->kind) * l->N - (l->kind == SA_KIND_2P ? l->L : 0);
+  for (int k0 = 0; k0 < nsteps; k0 += kRun) {
+    const int run = std::min(kRun, nsteps - k0);
+    hipLaunchKernelGGL(sa::k_fill_zero, dim3((unsigned)((run * kCnt + 255) / 256)), dim3(256), 0, l->stream, l->xcnt,
+                       run * kCnt);
+    for (int q = 0; q < run; ++q) {
+      const int k = k0 + q;
+      rc = sa_ladder_sweep(l, sweeps);
+      if (rc) return rc;
+      const bool third = cold != a[k] && cold != b[k];
+      const int n = third ? 3 : 2;
+      int *cnt = l->xcnt + (size_t)q * kCnt;
+      sa_detail::launch_measure(l->kind, l->L, l->N, l->s, l->jx, l->jy, l->jz, n, nullptr,
+                                sa::sys4{{a[k], b[k], third ? cold : a[k], a[k]}}, cnt, l->stream, false);
+      sa::exchange_args x{};
+      x.sa = l->s + (int64_t)a[k] * l->N;
+      x.sb = l->s + (int64_t)b[k] * l->N;
+      x.N = l->N;
+      x.bonds = bonds;
+      x.cnt = cnt;
+      x.n = n;
+      x.copies = sa::measure_copies(n);
+      x.cold = third ? 2 : cold == a[k] ? 0 : 1;
+      x.min_dE = min_dE[k];
+      x.ha = ha[k];
+      x.hb = hb[k];
+      x.EM = em_pin + 384 * q;
+      x.mask = mask_pin + q;
+      // about four words per thread: every block sums the counters first
+      const unsigned blocks = (unsigned)std::min<int64_t>((l->N + 1023) / 1024, 1024);
+      hipLaunchKernelGGL(sa::k_exchange, dim3(blocks), dim3(256), 0, l->stream, x);
+    }
+    SA_HIP_TRY(hipGetLastError());
+    rc = wait_stream(l);
+    if (rc) return rc;
+    std::memcpy(masks + k0, mask_pin, 8 * run);
+    std::memcpy(EM + (size_t)384 * k0, em_pin, kRec * run);
+  }
   return SA_OK;
 }
 
