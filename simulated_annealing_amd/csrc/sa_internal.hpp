@@ -44,8 +44,10 @@ struct sa_ladder {
   uint64_t *words_d = nullptr, *words_h = nullptr;
   int64_t words_cap = 0;  // sweeps that fit in the staging buffers
   std::vector<int> cnt_h;  // host copy of the measurement counters
-  int *cnt_pin = nullptr;  // pinned landing buffer of the counters (allocated at the first measurement)
-  hipEvent_t meas_ev = nullptr;  // recorded after the counters' copy; polled
+  char *cnt_pin = nullptr;  // pinned: the flag and counts of a measurement (allocated at the first)
+  bool cnt_clear = false;   // the counters and the ticket behind them are zero
+  uint64_t meas_seq = 0;    // measurements reported so far (the flag's value)
+  hipEvent_t meas_ev = nullptr;  // what wait_stream polls
   int *xcnt = nullptr;     // counters of a run of exchange steps (allocated at the first)
   char *x_pin = nullptr;   // pinned: their masks, then E and M
   bool words_busy = false;  // replay: the staged words may still be on their way (words_ev)
@@ -82,7 +84,7 @@ bool compact_table(int kind, const sa::sys_table &tab);
 // Asynchronous on st; the caller sums the copies.
 void launch_measure(int kind, int L, int64_t N, const uint64_t *s, const uint64_t *jx, const uint64_t *jy,
                     const uint64_t *jz, int n, const int *dlist, sa::sys4 sel, int *cnt, hipStream_t st,
-                    bool clear = true);
+                    bool clear = true, const sa::meas_report *report = nullptr);
 // sa_digest of all systems' spins in order, computed on the device
 int ladder_digest(sa_ladder *l, uint64_t *digest);
 // device bytes sa_ladder_create allocates for a ladder (the fused 3D sweep's second

@@ -1283,9 +1283,21 @@ template <int SB>
 struct meas_shared {
   uint64_t v[2][SB][kMeasPlanes + 2][64];  // planes of two waves / the block's planes
 };
+//
+// report (may be empty): the block that finishes last sums the copies, writes the counts to
+// host memory and then `seq`, and leaves the counters and the ticket at zero for the next
+// measurement -- one launch, no copy and no event per measurement (a step of a small replay
+// ladder with its measurement 146 -> 116 us, 32 systems of L=128 210 -> 201).
+struct meas_report {
+  unsigned *ticket = nullptr;         // blocks done
+  unsigned total = 0;                 // blocks in all
+  int *out = nullptr;                 // host: [listed system][2][64]
+  unsigned long long *flag = nullptr;  // host
+  unsigned long long seq = 0;
+};
 template <int SB>
 __device__ __forceinline__ void meas_finish(const meas_big (&big)[SB], meas_shared<SB> &sh, int (&red)[SB][2][64],
-                                            int nsys, int sys0, int ns, int unit, int *cnt) {
+                                            int nsys, int sys0, int ns, int unit, int *cnt, const meas_report &rep) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   // the four waves' planes added through LDS: waves 2, 3 into 0, 1, then 1 into 0
   for (int q = threadIdx.x; q < SB * 128; q += blockDim.x) (&red[0][0][0])[q] = 0;
@@ -1345,8 +1357,38 @@ __device__ __forceinline__ void meas_finish(const meas_big (&big)[SB], meas_shar
     atomicAdd(&red[m][isE ? 0 : 1][lane], __popcll(wave_transpose64(v, lane)) << (isE ? b : b - kMeasE - 2));
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < ns * 128; q += blockDim.x)
-    atomicAdd(&cnt[((int64_t)(unit % measure_copies(nsys)) * nsys + sys0) * 128 + q], (&red[0][0][0])[q]);
+  int *mine = cnt + ((int64_t)(unit % measure_copies(nsys)) * nsys + sys0) * 128;
+  if (!rep.ticket) {
+    for (int q = threadIdx.x; q < ns * 128; q += blockDim.x) atomicAdd(&mine[q], (&red[0][0][0])[q]);
+    return;
+  }
+  // Counters, ticket and report are only touched by atomics and system-scope stores, which
+  // act at the device's and the host's coherence points, so their order is all that matters,
+  // not the caches' contents: an addition whose old value has come back is done, and a block
+  // takes its ticket after its additions.  (A device-scope fence per block writes back and
+  // invalidates the L2: measuring 32 systems of L=128 took twice as long with it.)
+  __shared__ int last;
+  int seen = 0;
+  for (int q = threadIdx.x; q < ns * 128; q += blockDim.x) seen |= atomicAdd(&mine[q], (&red[0][0][0])[q]);
+  asm volatile("" ::"v"(seen));        // the old values are used: the additions have returned
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (threadIdx.x == 0) last = atomicAdd(rep.ticket, 1u) == rep.total - 1;
+  __syncthreads();
+  if (!last) return;
+  const int n = nsys * 128, copies = measure_copies(nsys);
+  for (int q = threadIdx.x; q < n; q += blockDim.x) {
+    int v[kMeasureCopies], sum = 0;
+#pragma unroll
+    for (int c = 0; c < kMeasureCopies; ++c) v[c] = c < copies ? atomicExch(&cnt[(int64_t)c * n + q], 0) : 0;
+#pragma unroll
+    for (int c = 0; c < kMeasureCopies; ++c) sum += v[c];
+    __hip_atomic_store(&rep.out[q], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (threadIdx.x == 0) atomicExch(rep.ticket, 0u);
+  __builtin_amdgcn_s_waitcnt(0);  // every count has reached host memory before the flag leaves
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(rep.flag, rep.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Block = one unit (3D: 256 in-plane sites x up to `walk` planes; 2D: 256*walk
@@ -1355,7 +1397,8 @@ template <int KIND, int SB>
 __global__ void __launch_bounds__(256) k_measure(const uint64_t *__restrict__ s_all, const uint64_t *__restrict__ jx,
                                                  const uint64_t *__restrict__ jy, const uint64_t *__restrict__ jz,
                                                  int L, int64_t N, int nsys, const int *__restrict__ sys_list,
-                                                 sys4 sel, int *cnt, int units, int chunks, int walk) {
+                                                 sys4 sel, int *cnt, int units, int chunks, int walk,
+                                                 meas_report rep) {
   __shared__ meas_shared<SB> sh;
   __shared__ int red[SB][2][64];
   const int nq = (nsys + SB - 1) / SB;
@@ -1479,7 +1522,7 @@ __global__ void __launch_bounds__(256) k_measure(const uint64_t *__restrict__ s_
     if (__all(j0 + 8 <= steps)) eight(j0, std::true_type{});
     else eight(j0, std::false_type{});
   }
-  meas_finish<SB>(big, sh, red, nsys, sys0, ns, unit, cnt);
+  meas_finish<SB>(big, sh, red, nsys, sys0, ns, unit, cnt, rep);
 }
 
 // 3D with an even side and spin arrays below 2^31 bytes: a thread owns a pair of
@@ -1492,7 +1535,7 @@ __global__ void __launch_bounds__(256) k_measure3d_pair(const uint64_t *__restri
                                                         const uint64_t *__restrict__ jy,
                                                         const uint64_t *__restrict__ jz, int L, int64_t N, int nsys,
                                                         const int *__restrict__ sys_list, sys4 sel, int *cnt, int units,
-                                                        int chunks, int walk) {
+                                                        int chunks, int walk, meas_report rep) {
   __shared__ meas_shared<SB> sh;
   __shared__ int red[SB][2][64];
   const int nq = (nsys + SB - 1) / SB;
@@ -1581,7 +1624,7 @@ __global__ void __launch_bounds__(256) k_measure3d_pair(const uint64_t *__restri
       planes_add(big[m].m, a[m].m);
     }
   }
-  meas_finish<SB>(big, sh, red, nsys, sys0, ns, unit, cnt);
+  meas_finish<SB>(big, sh, red, nsys, sys0, ns, unit, cnt, rep);
 }
 
 static __global__ void k_fill_zero(int *p, int n) {

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -383,7 +384,7 @@ int sa_ladder_create(int kind, int L, int nsys, sa_ladder **out) {
   if (bad(hipGetDevice(&l->device), "hipGetDevice") || bad(hipStreamCreateWithFlags(&l->stream, hipStreamNonBlocking), "hipStreamCreate") ||
       bad(hipMalloc(&l->s, (size_t)nsys * N * 8), "spins") || bad(hipMalloc(&l->jx, 3 * N * 8), "couplings") ||
       bad(hipMalloc(&l->tab, sizeof(sa::sys_table) * nsys), "tables") ||
-      bad(hipMalloc(&l->cnt, sizeof(int) * 128 * nsys * sa::kMeasureCopies), "counters") ||
+      bad(hipMalloc(&l->cnt, sizeof(int) * (128 * (size_t)nsys * sa::kMeasureCopies + 1)), "counters") ||
       bad(hipMalloc(&l->sys_list, sizeof(int) * nsys), "system list") ||
       bad(hipMemsetAsync(l->s, 0, (size_t)nsys * N * 8, l->stream), "memset") ||
       bad(hipMemsetAsync(l->jx, 0, 3 * N * 8, l->stream), "memset")) {
@@ -610,6 +611,7 @@ int sa_ladder_get_spins(const sa_ladder *l, int sys, uint64_t *s) {
 
 // the measurement counters serve as the result word (same stream)
 int sa_detail::ladder_digest(sa_ladder *l, uint64_t *digest) {
+  l->cnt_clear = false;
   hipLaunchKernelGGL(sa::k_fill_zero, dim3(1), dim3(256), 0, l->stream, l->cnt, 2);
   const int64_t n = l->N * l->nsys;
   hipLaunchKernelGGL(sa::k_digest, dim3((unsigned)std::min<int64_t>((n + 1023) / 1024, 2048)), dim3(256), 0, l->stream,
@@ -656,7 +658,7 @@ void sa_detail::make_table(int kind, double T, double h, sa::sys_table &t, bool 
 
 void sa_detail::launch_measure(int kind, int L, int64_t N, const uint64_t *s, const uint64_t *jx, const uint64_t *jy,
                                const uint64_t *jz, int n, const int *dlist, sa::sys4 sel, int *cnt, hipStream_t st,
-                               bool clear) {
+                               bool clear, const sa::meas_report *report) {
   const int all_n = 128 * n * sa::measure_copies(n);
   if (clear) hipLaunchKernelGGL(sa::k_fill_zero, dim3((all_n + 255) / 256), dim3(256), 0, st, cnt, all_n);
   // cnt layout [copy][listed system][2][64] (the caller sums the copies).  Two systems
@@ -674,22 +676,27 @@ void sa_detail::launch_measure(int kind, int L, int64_t N, const uint64_t *s, co
                                           std::max<int64_t>(1, (length + want - 1) / want));
   const int64_t units = per_plane * ((length + walk - 1) / walk);
   const dim3 grid((unsigned)(((units + 7) / 8) * 8 * nq));
+  sa::meas_report rep;
+  if (report) {
+    rep = *report;
+    rep.total = (unsigned)(units * nq);
+  }
   if (pair) {
     if (sb == 1)
       hipLaunchKernelGGL((sa::k_measure3d_pair<1>), grid, dim3(256), 0, st, s, jx, jy, jz, L, N, n, dlist, sel, cnt,
-                         (int)units, (int)per_plane, walk);
+                         (int)units, (int)per_plane, walk, rep);
     else
       hipLaunchKernelGGL((sa::k_measure3d_pair<2>), grid, dim3(256), 0, st, s, jx, jy, jz, L, N, n, dlist, sel, cnt,
-                         (int)units, (int)per_plane, walk);
+                         (int)units, (int)per_plane, walk, rep);
     return;
   }
 #define SA_MEASURE(KINDV)                                                                                        \
   if (sb == 1)                                                                                                   \
     hipLaunchKernelGGL((sa::k_measure<KINDV, 1>), grid, dim3(256), 0, st, s, jx, jy, jz, L, N, n, dlist, sel, cnt,  \
-                       (int)units, (int)per_plane, walk);                                                        \
+                       (int)units, (int)per_plane, walk, rep);                                                        \
   else                                                                                                           \
     hipLaunchKernelGGL((sa::k_measure<KINDV, 2>), grid, dim3(256), 0, st, s, jx, jy, jz, L, N, n, dlist, sel, cnt,  \
-                       (int)units, (int)per_plane, walk);
+                       (int)units, (int)per_plane, walk, rep);
   if (kind == SA_KIND_3D) {
     SA_MEASURE(sa::KIND_3D)
   } else if (kind == SA_KIND_2D) {
@@ -820,19 +827,48 @@ int measure_list(sa_ladder *l, const int *list, int n) {
     SA_HIP_TRY(hipMemcpyAsync(l->sys_list, list, sizeof(int) * n, hipMemcpyHostToDevice, l->stream));
     dlist = l->sys_list;
   }
+  // The counts land in pinned memory allocated at the first measurement (so creating a
+  // ladder, e.g. per served request, needs no pinned allocation): the flag, then the counts.
+  const size_t pin = 64 + sizeof(int) * 128 * (size_t)l->nsys;
+  if (!l->cnt_pin && hipHostMalloc((void **)&l->cnt_pin, pin, hipHostMallocDefault) == hipSuccess)
+    std::memset(l->cnt_pin, 0, pin);
+  if (!l->cnt_pin) (void)hipGetLastError();
+  if (l->cnt_pin) {
+    unsigned *ticket = (unsigned *)(l->cnt + (size_t)128 * l->nsys * sa::kMeasureCopies);
+    if (!l->cnt_clear) {
+      const int all = 128 * l->nsys * sa::kMeasureCopies + 1;
+      hipLaunchKernelGGL(sa::k_fill_zero, dim3((unsigned)((all + 255) / 256)), dim3(256), 0, l->stream, l->cnt, all);
+    }
+    l->cnt_clear = false;
+    volatile unsigned long long *flag = (volatile unsigned long long *)l->cnt_pin;
+    sa::meas_report rep;
+    rep.ticket = ticket;
+    rep.out = (int *)(l->cnt_pin + 64);
+    rep.flag = (unsigned long long *)l->cnt_pin;
+    rep.seq = ++l->meas_seq;
+    sa_detail::launch_measure(l->kind, l->L, l->N, l->s, l->jx, l->jy, l->jz, n, dlist, sel, l->cnt, l->stream, false,
+                              &rep);
+    SA_HIP_TRY(hipGetLastError());
+    // the host polls the flag; now and then it asks the stream, which also ends the wait if
+    // the launch failed
+    for (unsigned spin = 1; *flag != rep.seq; ++spin) {
+      if (spin % 4096) continue;
+      const hipError_t e = hipStreamQuery(l->stream);
+      if (e == hipErrorNotReady) continue;
+      SA_HIP_TRY(e);
+      if (*flag == rep.seq) break;
+      return sa_fail(SA_ERR_HIP, "the measurement did not report");
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    std::memcpy(l->cnt_h.data(), rep.out, sizeof(int) * cnt_n);
+    l->cnt_clear = true;
+    return SA_OK;
+  }
+  l->cnt_clear = false;
   sa_detail::launch_measure(l->kind, l->L, l->N, l->s, l->jx, l->jy, l->jz, n, dlist, sel, l->cnt, l->stream);
   SA_HIP_TRY(hipGetLastError());
-  // The counters land in pinned memory allocated at the first measurement (so
-  // creating a ladder, e.g. per served request, needs no pinned allocation).
-  if (!l->cnt_pin &&
-      hipHostMalloc((void **)&l->cnt_pin, sizeof(int) * 128 * l->nsys * sa::kMeasureCopies, hipHostMallocDefault) !=
-          hipSuccess)
-    l->cnt_pin = nullptr;
-  int *to = l->cnt_pin ? l->cnt_pin : l->cnt_h.data();
-  SA_HIP_TRY(hipMemcpyAsync(to, l->cnt, sizeof(int) * all_n, hipMemcpyDeviceToHost, l->stream));
-  const int rc = wait_stream(l);
-  if (rc) return rc;
-  if (to != l->cnt_h.data()) std::memcpy(l->cnt_h.data(), to, sizeof(int) * all_n);
+  SA_HIP_TRY(hipMemcpyAsync(l->cnt_h.data(), l->cnt, sizeof(int) * all_n, hipMemcpyDeviceToHost, l->stream));
+  SA_HIP_TRY(hipStreamSynchronize(l->stream));
   // sum the copies into the first
   for (int c = 1; c < sa::measure_copies(n); ++c)
     for (int q = 0; q < cnt_n; ++q) l->cnt_h[q] += l->cnt_h[(size_t)c * cnt_n + q];
