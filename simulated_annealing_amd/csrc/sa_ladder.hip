@@ -748,6 +748,8 @@ int launch_sweeps(sa_ladder *l, const uint64_t *words, uint64_t t, int64_t n) {
       else sa_detail::tile2d_launch(l, l->tab, 0, all_of(l->fast), w, t + k, n - k, ns);
       k += ns;
     } else {
+      // no memory for the tiles' extras: the fused walk writes a second array too
+      if (use_fused(l) && !have_alt(l)) return sa_fail(SA_ERR_NOMEM, "second spin array");
       launch_sweep(l, w, t + k);
       ++k;
     }
@@ -930,23 +932,26 @@ int anneal_run(sa_ladder *l, const double *T, int64_t left, double h, int64_t *d
                             l->stream));
   SA_HIP_TRY(hipMemcpyAsync(l->tab, tabs.data() + (n - 1) * l->nsys, sizeof(sa::sys_table) * l->nsys,
                             hipMemcpyHostToDevice, l->stream));
-  for (int64_t k = 0; k < n;) {  // the same configuration as above until the last, shorter launch
+  // the same configuration as above until the last, shorter launch; should that one need a second
+  // array that is not to be had, the run ends before it
+  int64_t k = 0;
+  while (k < n) {
     int ns;
     double us = 0;
     if (l->kind == SA_KIND_3D) {
       ns = sa_detail::tile3d_sweeps(l, n - k, &second, &us);
-      if (second && !have_alt(l)) return sa_fail(SA_ERR_NOMEM, "second spin array");
+      if (second && !have_alt(l)) break;
       sa_detail::tile3d_launch(l, l->tab_seq + k * l->nsys, l->nsys, fast, nullptr, l->t + k, n - k);
     } else {
       ns = sa_detail::tile2d_sweeps(l, n - k, &second);
-      if (second && !have_alt(l)) return sa_fail(SA_ERR_NOMEM, "second spin array");
+      if (second && !have_alt(l)) break;
       sa_detail::tile2d_launch(l, l->tab_seq + k * l->nsys, l->nsys, fast, nullptr, l->t + k, n - k, ns);
     }
     k += ns;
   }
   SA_HIP_TRY(hipGetLastError());
-  l->t += n;
-  *done = n;
+  l->t += k;
+  *done = k;
   return SA_OK;
 }
 
