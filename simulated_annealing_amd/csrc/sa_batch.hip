@@ -787,10 +787,12 @@ int prepare_instance(int kind, int L, int nsys, uint64_t seed, int nsweeps, cons
   if (!rc) rc = sa_ladder_init_spins(l);
   const int ntab = per_sweep ? std::max(1, nsweeps) * nsys : nsys;
   std::vector<sa::sys_table> tabs(ntab);
+  std::vector<char> fasts(ntab);
   bool fast = true;
   for (int q = 0; q < ntab && !rc; ++q) {
     bool f = false;
     sa_detail::make_table(kind, T[per_sweep && nsweeps == 0 ? q % nsys : q], h, tabs[q], f, nullptr);
+    fasts[q] = f;
     fast = fast && f;
   }
   // what the tiles need beside the instance's own arrays; without it, half-sweeps
@@ -818,8 +820,7 @@ int prepare_instance(int kind, int L, int nsys, uint64_t seed, int nsweeps, cons
                             l->stream) != hipSuccess)
     rc = sa_fail(SA_ERR_HIP, "table upload");
   // fixed temperatures also become the ladder's own tables, for plain sweeps later
-  if (!rc && !per_sweep)
-    for (int j = 0; j < nsys && !rc; ++j) rc = sa_ladder_set_temperature(l, j, T[j], h, nullptr);
+  if (!rc && !per_sweep) rc = sa_detail::ladder_tables(l, std::move(tabs), std::move(fasts));
   if (!rc) rc = sa_ladder_sync(l);
   if (rc) {
     if (in.tabs) (void)hipFree(in.tabs);

@@ -85,6 +85,8 @@ bool compact_table(int kind, const sa::sys_table &tab);
 void launch_measure(int kind, int L, int64_t N, const uint64_t *s, const uint64_t *jx, const uint64_t *jy,
                     const uint64_t *jz, int n, const int *dlist, sa::sys4 sel, int *cnt, hipStream_t st,
                     bool clear = true, const sa::meas_report *report = nullptr);
+// the tables of all systems (nsys of each) in one upload on the ladder's stream
+int ladder_tables(sa_ladder *l, std::vector<sa::sys_table> tabs, std::vector<char> fast);
 // sa_digest of all systems' spins in order, computed on the device
 int ladder_digest(sa_ladder *l, uint64_t *digest);
 // device bytes sa_ladder_create allocates for a ladder (the fused 3D sweep's second

@@ -400,15 +400,15 @@ int sa_ladder_create(int kind, int L, int nsys, sa_ladder **out) {
   l->cnt_h.assign((size_t)128 * nsys * sa::kMeasureCopies, 0);
   l->eng.seed(5489u);
   *out = l;
-  for (int i = 0; i < nsys; ++i) {
-    rc = sa_ladder_set_temperature(l, i, 1.0, 0.0, nullptr);
-    if (rc != SA_OK) {
-      sa_ladder_destroy(l);
-      *out = nullptr;
-      return rc;
-    }
+  sa::sys_table t;
+  bool fast = false;
+  sa_detail::make_table(kind, 1.0, 0.0, t, fast, nullptr);
+  rc = sa_detail::ladder_tables(l, std::vector<sa::sys_table>(nsys, t), std::vector<char>(nsys, fast));
+  if (rc != SA_OK) {
+    sa_ladder_destroy(l);
+    *out = nullptr;
   }
-  return SA_OK;
+  return rc;
 }
 
 int sa_ladder_destroy(sa_ladder *l) {
@@ -626,6 +626,16 @@ int64_t sa_detail::ladder_bytes(int kind, int L, int nsys) {
   const int64_t N = (int64_t)L * L * (kind == SA_KIND_3D ? L : 1);
   return (int64_t)nsys * N * 8 + 3 * N * 8 + (int64_t)sizeof(sa::sys_table) * nsys +
          4 * 128 * nsys * sa::kMeasureCopies + 4 * nsys;
+}
+
+// Every system's table in one upload: one per system took about 10 us each, of 8 to 32 systems,
+// twice for each served request.
+int sa_detail::ladder_tables(sa_ladder *l, std::vector<sa::sys_table> tabs, std::vector<char> fast) {
+  l->htab = std::move(tabs);
+  l->fast = std::move(fast);
+  for (int j = 0; j < l->nsys; ++j) l->compact[j] = compact_table(l->kind, l->htab[j]);
+  SA_HIP_TRY(hipMemcpyAsync(l->tab, l->htab.data(), sizeof(sa::sys_table) * l->nsys, hipMemcpyHostToDevice, l->stream));
+  return SA_OK;
 }
 
 bool sa_detail::compact_table(int kind, const sa::sys_table &t) {
