@@ -129,9 +129,11 @@ bool zscan_ok(const sa_ladder *l) {
 }
 
 // the z-parallel half-sweeps: asked for, or automatically for ladders of at most 2^21
-// site words in all, where they beat the fused walk (us per sweep, fused vs z-parallel:
-// one L=64 system 46.7 / 23.1, four 47.1 / 41.6; one L=128 system 107 / 70; two L=128
-// systems 108 / 134)
+// site words in all that the tiles (tile_sweeps below) do not take -- no memory for their second
+// array or their couplings, tables that are not compact, a number of systems per thread asked
+// for -- where they beat the fused walk (us per sweep, fused vs z-parallel:
+// one L=64 system 46.7 / 12.9, four 47.1 / 27.5; one L=128 system 107 / 63; two L=128
+// systems 108 / 112, four 112 / 214).  The tiles take 7.2 on the one L=64 system.
 bool use_zscan(const sa_ladder *l) {
   if (!zscan_ok(l)) return false;
   if (l->sweep3d_kernel == 3) return true;
@@ -238,7 +240,7 @@ bool all_of(const std::vector<char> &v) {
 // x8 196 / 219; with a field L=64 x32 198 / 90, L=96 x16 264 / 195, L=128 x16 397 / 453.  Without a
 // fused walk (sides it does not divide): half-sweep launches, L=200 370 / 248, L=256 660 / 554.
 int tile_sweeps(const sa_ladder *l, int64_t left, bool *second) {
-  if (l->sys_per_thread || !all_of(l->compact)) return 0;
+  if (l->sys_per_thread || l->captured || !all_of(l->compact)) return 0;
   if (l->kind != SA_KIND_3D) return sa_detail::tile2d_sweeps(l, left, second);
   if (l->sweep3d_kernel || l->rows_per_tile || l->xcd_map >= 0) return 0;
   double us = 0;
@@ -745,6 +747,15 @@ bool have_alt(sa_ladder *l) {
   return false;
 }
 
+// A caller may capture the ladder's stream.  The tiles allocate at their first sweep and leave
+// the spins in the other array; a ladder once captured keeps to the sweeps that work in place
+// (a fused walk aside), so its graph finds the spins where they were.
+void note_capture(sa_ladder *l) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(l->stream, &st) != hipSuccess) (void)hipGetLastError();
+  else if (st != hipStreamCaptureStatusNone) l->captured = true;
+}
+
 // n sweeps at the ladder's own temperatures: words = the replay words of the first (N per sweep)
 int launch_sweeps(sa_ladder *l, const uint64_t *words, uint64_t t, int64_t n) {
   for (int64_t k = 0; k < n;) {
@@ -774,6 +785,7 @@ int sa_ladder_sweep(sa_ladder *l, int nsweeps) {
   if (!l) return sa_fail(SA_ERR_ARG, "null ladder");
   if (nsweeps < 0) return sa_fail(SA_ERR_ARG, "negative sweep count");
   if (nsweeps == 0) return SA_OK;
+  note_capture(l);
   bool second = false;
   if (use_fused(l) && !l->s_alt && !tile_sweeps(l, nsweeps, &second)) {
     const hipError_t e = hipMalloc(&l->s_alt, (size_t)l->nsys * l->N * 8);
@@ -907,6 +919,7 @@ namespace {
 int anneal_run(sa_ladder *l, const double *T, int64_t left, double h, int64_t *done) {
   *done = 0;
   bool second = false;
+  note_capture(l);
   if (l->rng_mode != SA_RNG_COUNTER || left < 2 || !tile_sweeps(l, left, &second)) return SA_OK;
   constexpr int64_t kTables = 4096;  // tables per upload (1.1 MB)
   const int64_t n = std::min<int64_t>(left, std::max<int64_t>(1, kTables / l->nsys));
