@@ -61,14 +61,14 @@ struct sa_ladder {
 };
 
 namespace sa_detail {
-// Sweeps of a 2D ladder with an even side held in LDS (sa_tile2d.hpp).  tile2d_sweeps:
+// Sweeps of a 2D ladder held in LDS (sa_tile2d.hpp).  tile2d_sweeps:
 // sweeps of the next launch when `left` are to be done (0: this ladder takes the
 // half-sweep kernels; *bands: the launch needs the second spin array).  tile2d_launch:
 // that launch, `ns` sweeps from index t on; tab_step = tables per sweep in `tab`.
 int tile2d_sweeps(const sa_ladder *l, int64_t left, bool *bands);
 void tile2d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, bool fast, const uint64_t *words,
                    uint64_t t, int64_t left, int ns);
-// The same for 3D ladders with an even side (sa_tile3d.hpp); *us: the modelled time per sweep.
+// The same for 3D ladders (sa_tile3d.hpp); *us: the modelled time per sweep.
 int tile3d_sweeps(const sa_ladder *l, int64_t left, bool *second, double *us);
 bool tile3d_couplings(sa_ladder *l);
 void tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, bool fast, const uint64_t *words,

@@ -30,7 +30,11 @@ size_t tile_lds(int L, int rows) { return (size_t)rows * 2 * sa::tile2d_half(L) 
 tile_cfg pick(const sa_ladder *l, int64_t left) {
   tile_cfg best{false, 0, 0, 0, 0};
   // asked for a number of systems per thread: the half-sweep kernels, which have that choice
-  if (l->kind == SA_KIND_3D || (l->L & 1) || l->L > kMaxSide || l->sys_per_thread > 0) return best;
+  if (l->kind == SA_KIND_3D || l->L > kMaxSide || l->sys_per_thread > 0) return best;
+  if (l->L & 1) {  // odd sides: the whole lattice (up to 89, always the faster) or not at all
+    const int items = l->L * sa::tile2d_groups(l->L);
+    return items <= kMaxItems ? tile_cfg{true, l->L, (int)std::min<int64_t>(left, 64), 1, items} : best;
+  }
   const int L = l->L, G = sa::tile2d_groups(L);
   double cost = 1e30;
   auto consider = [&](bool wrap, int th, int ns) {
@@ -55,7 +59,9 @@ tile_cfg pick(const sa_ladder *l, int64_t left) {
 template <bool COUNTER, int MODE, int IT>
 void launch(const sa::tile2d_args &t, bool wrap, int threads, size_t lds, hipStream_t st) {
   const dim3 grid((unsigned)(t.a.nsys * t.bands));
-  if (wrap) {
+  if (t.a.L & 1) {
+    hipLaunchKernelGGL((sa::k_tile2d_odd<COUNTER, MODE, IT>), grid, dim3(threads), lds, st, t);
+  } else if (wrap) {
     hipLaunchKernelGGL((sa::k_tile2d<COUNTER, MODE, IT, true>), grid, dim3(threads), lds, st, t);
   } else {
     hipLaunchKernelGGL((sa::k_tile2d<COUNTER, MODE, IT, false>), grid, dim3(threads), lds, st, t);
@@ -65,7 +71,7 @@ void launch(const sa::tile2d_args &t, bool wrap, int threads, size_t lds, hipStr
 template <bool COUNTER, int MODE>
 void launch_it(const sa::tile2d_args &t, const tile_cfg &c, hipStream_t st) {
   const int threads = std::min(1024, (c.items + 63) / 64 * 64);
-  const size_t lds = tile_lds(t.a.L, c.wrap ? t.a.L : c.th + 4 * t.ns);
+  const size_t lds = (t.a.L & 1) ? (size_t)t.a.L * t.a.L * 8 : tile_lds(t.a.L, c.wrap ? t.a.L : c.th + 4 * t.ns);
   if (c.items <= threads) launch<COUNTER, MODE, 1>(t, c.wrap, threads, lds, st);
   else launch<COUNTER, MODE, 2>(t, c.wrap, threads, lds, st);
 }

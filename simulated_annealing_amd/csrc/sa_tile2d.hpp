@@ -1,4 +1,5 @@
-// sa_tile2d.hpp -- several 2D sweeps per launch with the lattice held in LDS (even L).
+// sa_tile2d.hpp -- several 2D sweeps per launch with the lattice held in LDS (even L; odd L
+// where it fits whole, further down).
 //
 // What bounds a 2D lattice of ordinary size is not memory but launches: one half-sweep
 // per launch costs 3-4 us of which the update is a fraction.  Here a workgroup keeps a
@@ -237,6 +238,126 @@ __device__ __forceinline__ void tile2d(const tile2d_args &t, int sys, int band, 
       row[3] = d;
     }
   }
+}
+
+// ---- odd sides: the whole lattice in LDS, rows of L words.  The wrap neighbours in x and in y
+// share a colour: the last column reads the new first one, the last row the new first one, and
+// the corner both (row-major visits, src/cpu_2dp.cpp:106-114).  So a colour is updated in stages
+// with a barrier after each: every site off the last column and row, then those on one of them,
+// then the corner (colour 0).  In place: a stage reads old what later stages update.
+//
+// A thread owns IT items as above; the last item of a row has one column or three.  Bound by
+// the update's chain and the five stages' barriers; what the random word accepts is formed in
+// the first stage only (in each stage: general tables 9.7 instead of 7.8 us per sweep at L=89).
+// Us per sweep, two launches with a thread per wrap group / here: L=17 x24 7.6 / 1.8, L=63 x1
+// 7.6 / 3.1, L=89 x24 8.7 / 6.8, x1024 79 / 24.5, with a field x1 11.8 / 7.8; open x L=63 x8
+// 14.1 / 7.4, L=89 x24 15.0 / 13.0.  In a batch the half-sweeps of many odd instances fill the
+// chip together (52 instances of L 17..89: 10.0 us per sweep, as tiles 10.4), so it keeps them.
+template <bool COUNTER, int MODE, int IT>
+__device__ __forceinline__ void tile2d_odd(const tile2d_args &t, int sys, uint64_t *lds) {
+  const sweep_args &p = t.a;
+  const int L = p.L, G = tile2d_groups(L);
+  uint64_t *s = p.s + (int64_t)sys * p.N;
+  int j_[IT], y_[IT];
+  pair2d J[IT][2];
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int it = (int)threadIdx.x + i * (int)blockDim.x;
+    const bool live = it < L * G;
+    const int y = live ? it / G : 0, j = live ? it - y * G : 0;
+    j_[i] = live ? j : -1;
+    y_[i] = y;
+    if (live) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (4 * j + c < L) lds[y * L + 4 * j + c] = s[(int64_t)y * L + 4 * j + c];
+      const uint64_t *jx = p.jx + (int64_t)y * L, *jn = p.jy + (int64_t)y * L;
+      const uint64_t *js = p.jy + (int64_t)(y == L - 1 ? 0 : y + 1) * L;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int x = min(4 * j + ((y + c) & 1), L - 1), x2 = min(x + 2, L - 1);  // beyond the row: not used
+        pair2d &q = J[i][c];
+        q.w0 = jx[x];
+        q.e0 = jx[x == L - 1 ? 0 : x + 1];
+        q.w1 = jx[x2];
+        q.e1 = jx[x2 == L - 1 ? 0 : x2 + 1];
+        q.n0 = jn[x];
+        q.n1 = jn[x2];
+        q.s0 = js[x];
+        q.s1 = js[x2];
+      }
+    }
+  }
+  __syncthreads();
+  for (int sw = 0; sw < t.ns; ++sw) {
+    const sys_table &tab = p.tab[sys + sw * t.tab_step];
+    const uint64_t *words = COUNTER ? nullptr : p.words + (int64_t)sw * p.N;
+    // what a site's random word accepts, formed in the first stage, which every wave is in
+    // (the levels of spin bit 0 | spin bit 1 << 8; FAST: bit 0 level 3, bit 1 level 4)
+    auto levels = [&](int x, uint64_t g) {
+      if (MODE == T2_FAST) return (g < tab.thr[0][3] ? 1u : 0u) | (g < tab.thr[0][4] ? 2u : 0u);
+      uint32_t k0 = accepted_levels(tab, 0, g), k1 = accepted_levels(tab, 1, g);
+      if (MODE == T2_OPEN && (x == 0 || x == L - 1)) {
+        k0 = accepted_levels(tab, 2, g);
+        k1 = accepted_levels(tab, 3, g);
+      }
+      return k0 | k1 << 8;
+    };
+    auto site = [&](int x, int y, uint64_t jw, uint64_t je, uint64_t jn, uint64_t js, uint32_t k) {
+      uint64_t *row = lds + y * L;
+      const uint64_t si = row[x];
+      uint64_t bw = xor3(jw, si, row[x == 0 ? L - 1 : x - 1]), be = xor3(je, si, row[x == L - 1 ? 0 : x + 1]);
+      if (MODE == T2_OPEN) {  // missing open-x bond counts as satisfied (src/cpu_2dp.cpp:338-339)
+        if (x == 0) bw = ~0ULL;
+        if (x == L - 1) be = ~0ULL;
+      }
+      const uint64_t un = lds[(y == 0 ? L - 1 : y - 1) * L + x], us = lds[(y == L - 1 ? 0 : y + 1) * L + x];
+      const count3 c = count4(bw, be, xor3(jn, si, un), xor3(js, si, us));
+      if (MODE == T2_FAST) row[x] = si ^ sel(c.b2, lvl(k & 2), ~(c.b1 & c.b0) | lvl(k & 1));
+      else row[x] = update_levels(k & 255, k >> 8, c, si);
+    };
+#pragma unroll
+    for (int color = 0; color < 2; ++color) {
+      uint32_t k0[IT], k1[IT];
+      // 0: off the last column and row, 1: on one of them, 2: the corner
+      auto stage_of = [&](int x, int y) { return (x == L - 1 ? 1 : 0) + (y == L - 1 ? 1 : 0); };
+#pragma unroll
+      for (int st = 0; st < 3 - color; ++st) {
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+          const int j = j_[i], y = y_[i];
+          if (j < 0) continue;
+          const int x = 4 * j + ((y + color) & 1), x2 = x + 2;
+          if (st == 0) {
+            if (COUNTER) {
+              const u32x4 blk = counter_block((uint32_t)(x + L * y), p.seed, p.sweep + (uint64_t)sw);
+              k0[i] = levels(x, counter_half(blk, 0));
+              k1[i] = levels(x2, counter_half(blk, 1));
+            } else {
+              const int64_t rank = x < L ? odd_rank(L, 1, color, x, y, 0) : 0;
+              k0[i] = levels(x, words[rank]);
+              k1[i] = levels(x2, x2 < L ? words[rank + 1] : 0);
+            }
+          }
+          const pair2d &q = J[i][color];
+          if (x < L && stage_of(x, y) == st) site(x, y, q.w0, q.e0, q.n0, q.s0, k0[i]);
+          if (x2 < L && stage_of(x2, y) == st) site(x2, y, q.w1, q.e1, q.n1, q.s1, k1[i]);
+        }
+        __syncthreads();
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < IT; ++i)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (j_[i] >= 0 && 4 * j_[i] + c < L) s[(int64_t)y_[i] * L + 4 * j_[i] + c] = lds[y_[i] * L + 4 * j_[i] + c];
+}
+
+template <bool COUNTER, int MODE, int IT>
+__global__ void __launch_bounds__(1024) k_tile2d_odd(tile2d_args t) {
+  extern __shared__ __align__(16) uint64_t lds[];
+  tile2d_odd<COUNTER, MODE, IT>(t, (int)blockIdx.x, lds);
 }
 
 template <bool COUNTER, int MODE, int IT, bool WRAP>
