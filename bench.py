@@ -98,12 +98,11 @@ def batched_vs_plain(sa, n=512):
     Workload: n independent realisations of uneven size (60% 2D periodic with L in
     {32,48,64,96,128}, 40% 3D with L in {16,24,32,48}), each its own linear anneal
     3.0 -> 0.1 over 500, 1000 or 2000 sweeps, counter RNG.  Batched: one Batch
-    (one launch per half-sweep for all unfinished instances, hipGraph chunks, block
-    size and chunk length tuned online inside the timed region).  Plain: a ladder
-    per instance driven by sa_ladder_anneal (temperature upload + sweep launch per
-    sweep, each instance on its own stream; 3D instances on the fused sweep, one
-    launch per sweep, which is faster here than the two z-parallel launches a lone
-    small ladder takes by default).  Set-up (seeding, couplings) is outside
+    (LDS tiles: per sweep one launch for all 3D instances, per four sweeps one for all
+    2D ones; hipGraph chunks, chunk length tuned online inside the timed region).
+    Plain: a ladder per instance driven by sa_ladder_anneal, each on its own stream,
+    in its automatic choice of kernel (tables of many sweeps in one upload, LDS tiles:
+    3D one sweep per launch, 2D several).  Set-up (seeding, couplings) is outside
     both timed regions.  Every instance's final spins are compared bit for bit."""
     from simulated_annealing_amd import workloads
 
@@ -119,8 +118,6 @@ def batched_vs_plain(sa, n=512):
         lad = sa.Ladder(w.kind, w.L, 1)
         lad.set_rng(sa.RNG_COUNTER)
         lad.seed_like_main(w.seed)
-        if w.kind == sa.KIND_3D:  # one launch per sweep: the plain path's fastest form here
-            lad.tune(sa.TUNE_SWEEP3D_KERNEL, 2)
         lads.append(lad)
     for lad in lads:
         lad.sync()

@@ -269,8 +269,9 @@ int sa_pt_destroy(sa_pt *pt);
 /* ---- batched instances (no counterpart in the reference) --------------------
  * Many independent instances of uneven size and kind, each a ladder seeded like
  * main_gpu (set_seed, init_J, set_seed, init_rand; src/main_gpu.cu:262-276) with
- * its own temperatures, swept together: one launch per half-sweep covers every
- * unfinished instance, chunks of sweeps are replayed as captured hipGraphs, and
+ * its own temperatures, swept together: a launch covers every unfinished instance of
+ * its form (3D tiles: one launch per sweep; 2D tiles: one per four sweeps; the rest:
+ * one per half-sweep), chunks of sweeps are replayed as captured hipGraphs, and
  * block size / chunk length are tuned online.  Counter RNG only.  An instance's
  * spins after k sweeps are bit for bit those of its ladder swept k times alone
  * (sa_ladder_set_temperature + sa_ladder_sweep per sweep). */
@@ -314,10 +315,9 @@ int sa_batch_remove(sa_batch *b, int id);
 /* the stream the batch launches on (hipStream_t) */
 void *sa_batch_stream(sa_batch *b);
 /* tuning (no effect on results): threads per block 64/128/256 of the half-sweep
- * kernel, sweeps per captured graph, and whether 3D instances with symmetric tables
- * and L divisible by 4 take the fused single-pass sweep (1 off, 2 on); 0 = picked
- * online by timing the first chunks.  The fused form is switched off in this build:
- * SA_TUNE_BATCH_FUSED = 2 returns SA_ERR_ARG. */
+ * kernel and sweeps per captured graph; 0 = picked online by timing the first chunks.
+ * SA_TUNE_BATCH_FUSED takes 0 and 1, which mean the same; 2 (a fused walk inside the
+ * batch, which is not part of it) returns SA_ERR_ARG. */
 enum sa_batch_tune_key { SA_TUNE_BATCH_BLOCK = 101, SA_TUNE_BATCH_CHUNK = 102, SA_TUNE_BATCH_FUSED = 103 };
 int sa_batch_set_tuning(sa_batch *b, int key, int value);
 int sa_batch_get_tuning(sa_batch *b, int key, int *value);
