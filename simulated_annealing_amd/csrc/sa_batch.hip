@@ -441,9 +441,26 @@ bool tile3d_geometry(sa::tile3d_args &a, int L, int wide, int high) {
   }
 }
 
+bool tiles_3d(int form) { return form == FORM_3D || form == FORM_3D_ODD; }
+
+// A ladder that the batch handed out (sa_batch_ladder) may have been given other couplings:
+// the 3D tiles read a copy of them, which is made again with the schedule.
+void notice_changes(sa_batch *b) {
+  for (int id : b->desc_id) {
+    const batch_inst &in = b->inst[id];
+    if (in.live && tiles_3d(in.form) && !in.lad->jt_current) b->dirty = true;
+  }
+}
+
 // descriptors, the half-sweep block map and the tiles of the unfinished instances,
 // largest remaining work first
 int rebuild(sa_batch *b, int bs) {
+  for (batch_inst &in : b->inst)
+    if (in.live && in.t < in.nsweeps && tiles_3d(in.form) && !in.lad->jt_current) {
+      if (!sa_detail::tile3d_couplings(in.lad)) in.form = FORM_HALF;
+      SA_HIP_TRY(hipGetLastError());
+      SA_HIP_TRY(hipStreamSynchronize(in.lad->stream));
+    }
   std::vector<int> ids;
   for (int i = 0; i < (int)b->inst.size(); ++i)
     if (b->inst[i].live && b->inst[i].t < b->inst[i].nsweeps) ids.push_back(i);
@@ -456,7 +473,7 @@ int rebuild(sa_batch *b, int bs) {
   for (int id : ids) {
     const batch_inst &in = b->inst[id];
     const int64_t side = (in.lad->L + 7) / 8;
-    if (in.form == FORM_3D || in.form == FORM_3D_ODD) tiles8 += side * side * in.lad->nsys;
+    if (tiles_3d(in.form)) tiles8 += side * side * in.lad->nsys;
   }
   const int wide = tiles8 >= 2 * b->cus / 4 ? 8 : 4, high = tiles8 >= 2 * b->cus / 2 ? 8 : 4;
   std::vector<inst_desc> descs(ids.size());
@@ -492,7 +509,7 @@ int rebuild(sa_batch *b, int bs) {
     d.m = 1;
     int64_t n = 0;
     float cost = 0;  // of an entry, about us
-    if ((in.form == FORM_3D || in.form == FORM_3D_ODD) && tile3d_geometry(d.t3, l->L, wide, high)) {
+    if (tiles_3d(in.form) && tile3d_geometry(d.t3, l->L, wide, high)) {
       const int64_t jn = (int64_t)l->L * l->L * sa::column_stride(l->L);
       d.t3.jxt = l->jt;
       d.t3.jyt = l->jt + jn;
@@ -956,6 +973,7 @@ int batch_launch_chunk(sa_batch *b, int max_sweeps, int *k_out) {
   }
   const int bs = b->block ? b->block : (trial >= 0 ? kCands[trial].block : b->tuned_block);
   const int kfull = b->chunk ? b->chunk : (trial >= 0 ? kCands[trial].chunk : b->tuned_chunk);
+  notice_changes(b);
   if (b->dirty || b->bmap_bs != bs) {
     const int rc = rebuild(b, bs);
     if (rc) return rc;
