@@ -308,7 +308,9 @@ int sa_batch_pt_result(sa_batch *b, int id, int64_t capacity, int32_t *pairs, do
                        float *E_min, double *acceptance);
 /* device bytes held by the batch's live instances */
 int64_t sa_batch_bytes(const sa_batch *b);
-/* the instance's ladder (owned by the batch; valid until sa_batch_remove) */
+/* the instance's ladder (owned by the batch; valid until sa_batch_remove).  Between runs it
+ * may be used like any other ladder, also through a handle kept from before; the next
+ * sa_batch_run waits for what it has enqueued and goes on from its spins and couplings. */
 sa_ladder *sa_batch_ladder(sa_batch *b, int id);
 /* free the instance's device memory; its id is not reused */
 int sa_batch_remove(sa_batch *b, int id);

@@ -349,6 +349,7 @@ struct batch_inst {
   sa::sys_table *tabs = nullptr;
   int nsweeps = 0, per_sweep = 0, t = 0;
   bool fast = true, live = false;
+  bool lent = false;  // its ladder was handed out (sa_batch_ladder)
   int64_t work = 0;   // work items per half-sweep (all systems)
   int64_t bytes = 0;  // device memory held
   int form = FORM_HALF;
@@ -443,18 +444,10 @@ bool tile3d_geometry(sa::tile3d_args &a, int L, int wide, int high) {
 
 bool tiles_3d(int form) { return form == FORM_3D || form == FORM_3D_ODD; }
 
-// A ladder that the batch handed out (sa_batch_ladder) may have been given other couplings:
-// the 3D tiles read a copy of them, which is made again with the schedule.
-void notice_changes(sa_batch *b) {
-  for (int id : b->desc_id) {
-    const batch_inst &in = b->inst[id];
-    if (in.live && tiles_3d(in.form) && !in.lad->jt_current) b->dirty = true;
-  }
-}
-
 // descriptors, the half-sweep block map and the tiles of the unfinished instances,
 // largest remaining work first
 int rebuild(sa_batch *b, int bs) {
+  // 3D tiles read a copy of the couplings: made again where the ladder was given others
   for (batch_inst &in : b->inst)
     if (in.live && in.t < in.nsweeps && tiles_3d(in.form) && !in.lad->jt_current) {
       if (!sa_detail::tile3d_couplings(in.lad)) in.form = FORM_HALF;
@@ -973,7 +966,6 @@ int batch_launch_chunk(sa_batch *b, int max_sweeps, int *k_out) {
   }
   const int bs = b->block ? b->block : (trial >= 0 ? kCands[trial].block : b->tuned_block);
   const int kfull = b->chunk ? b->chunk : (trial >= 0 ? kCands[trial].chunk : b->tuned_chunk);
-  notice_changes(b);
   if (b->dirty || b->bmap_bs != bs) {
     const int rc = rebuild(b, bs);
     if (rc) return rc;
@@ -1082,6 +1074,13 @@ int sa_batch_add_pt(sa_batch *b, int kind, int L, int nT, const double *T, doubl
 
 int sa_batch_run(sa_batch *b, int sweeps) {
   if (!b) return sa_fail(SA_ERR_ARG, "null batch");
+  // Between two runs a ladder that was handed out may have been swept (on its own stream, and
+  // into its other spin array), given other couplings or seeded: wait for it and schedule anew.
+  for (const batch_inst &in : b->inst)
+    if (in.live && in.lent) {
+      SA_HIP_TRY(hipStreamSynchronize(in.lad->stream));
+      b->dirty = true;
+    }
   int64_t left = sweeps > 0 ? sweeps : INT64_MAX;
   while (left > 0) {
     int k = 0;
@@ -1146,7 +1145,7 @@ int sa_batch_pt_result(sa_batch *b, int id, int64_t capacity, int32_t *pairs, do
 sa_ladder *sa_batch_ladder(sa_batch *b, int id) {
   if (check_id(b, id)) return nullptr;
   if (sync_batch(b)) return nullptr;
-  b->dirty = true;  // the caller may sweep it (the fused 3D sweep swaps its spin arrays)
+  b->inst[id].lent = true;
   return b->inst[id].lad;
 }
 

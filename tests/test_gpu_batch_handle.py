@@ -1,5 +1,7 @@
 """A batch instance's ladder (sa_batch_ladder) used between two runs, against the oracle bit
-for bit: new couplings take effect in the next run, whichever form sweeps the instance."""
+for bit, whichever form sweeps the instance: new couplings take effect in the next run, and a
+run goes on from the spins that sweeps and swaps of the ladder left, also through a handle that
+was fetched before earlier runs."""
 import numpy as np
 import pytest
 
@@ -42,4 +44,38 @@ def test_new_couplings_take_effect(orc, fetch_again):
     for i, kind, L, seed, s, j in insts:
         advance(orc, kind, L, seed, s, j, 1.1, 5, 6)
         assert (b.spins(i) == s).all(), (kind, L)
+    b.close()
+
+
+@pytest.mark.parametrize("extra", [1, 2, 3])
+def test_sweeps_and_swaps_through_a_kept_handle(orc, extra):
+    b = sa.Batch()
+    insts = []
+    for q, (kind, L) in enumerate(FORMS):
+        i = b.add(kind, L, 400 + q, 100, T=[1.1, 1.1], nsys=2)
+        jx, jy, jz, s, _ = orc.init_system(kind, L, 400 + q)
+        insts.append((i, kind, L, 400 + q, [s, s.copy()], [jx, jy, jz], sa.lib().sa_batch_ladder(b.b, i)))
+    done = 0
+    for n in (5, 3, 6):
+        b.run(n)
+        for i, kind, L, seed, s, j, lad in insts:
+            for x in s:
+                advance(orc, kind, L, seed, x, j, 1.1, done, n)
+        done += n
+        mask = 0x0F0F0F0F0F0F0F0F << (done & 3)
+        for i, kind, L, seed, s, j, lad in insts:  # the ladder's sweeps continue the instance's index
+            sa.check(sa.lib().sa_ladder_set_spins(lad, 1, (~s[1])), "set_spins")
+            s[1] = ~s[1]
+            sa.check(sa.lib().sa_ladder_sweep(lad, extra), "sweep")
+            sa.check(sa.lib().sa_ladder_swap(lad, 0, 1, mask), "swap")
+            for x in s:
+                advance(orc, kind, L, seed, x, j, 1.1, done, extra)
+            d = (s[0] ^ s[1]) & np.uint64(mask)
+            s[0] ^= d
+            s[1] ^= d
+    b.run(2)
+    for i, kind, L, seed, s, j, lad in insts:
+        for k, x in enumerate(s):
+            advance(orc, kind, L, seed, x, j, 1.1, done, 2)
+            assert (b.spins(i, k) == x).all(), (kind, L, k)
     b.close()
