@@ -44,7 +44,6 @@ tile_cfg pick(const sa_ladder *l, int64_t left, double &cost) {
     if (!c.lds || c.lds > kMaxLds) return;
     c.ns = whole ? (int)std::min<int64_t>(left, 64) : 1;
     const int64_t tiles = (int64_t)c.a.ntx * c.a.nty;
-    if (tiles * l->nsys >= (int64_t)1 << 24) return;
     const double per_cu = std::ceil((double)tiles * l->nsys / 256);
     const double wave = S == 2 ? (general ? 0.195 : 0.13) : (general ? 0.29 : 0.25);
     const double words = (double)l->nsys * l->N, amp = (double)(W * H) / (c.a.tx * c.a.ty);
@@ -163,10 +162,18 @@ void sa_detail::tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t ta
     if (c.S == 2) launch<CO, FA, 2>(a, c, l->stream);                   \
     else launch<CO, FA, 4>(a, c, l->stream);                            \
   }
-  SA_T3(true, true)
-  SA_T3(true, false)
-  SA_T3(false, true)
-  SA_T3(false, false)
+  const int64_t most = sa::systems_per_launch((uint32_t)(a.ntx * a.nty), c.threads);
+  for (int64_t left_sys = l->nsys; left_sys > 0;) {
+    a.a.nsys = (int)std::min(left_sys, most);
+    SA_T3(true, true)
+    SA_T3(true, false)
+    SA_T3(false, true)
+    SA_T3(false, false)
+    left_sys -= a.a.nsys;
+    a.a.s += a.a.nsys * l->N;
+    a.out += a.a.nsys * l->N;
+    a.a.tab += a.a.nsys;
+  }
 #undef SA_T3
   if (!c.whole) std::swap(l->s, l->s_alt);
 }

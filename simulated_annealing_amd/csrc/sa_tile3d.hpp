@@ -31,6 +31,7 @@
 
 #include "sa_kernels.hpp"
 #include "sa_tile2d.hpp"
+#include "sa_tile_place.hpp"
 
 namespace sa {
 
@@ -44,7 +45,7 @@ struct tile3d_args {
   const uint64_t *jxt, *jyt, *jzt;  // couplings with z fastest: word (x + L*y) * L + z
   int chunks0, chunks1;  // waves' worth of columns of colour 0 / 1
   int recip_n0, recip_n1, recip_pairs, recip_hw, recip_ntx;  // ceil(2^20 / d): columns per row of colour 0 / 1, pairs of a plane, pairs of a row, tiles of a row
-  uint32_t recip_per;  // ceil(2^32 / tiles of a system)
+  uint32_t recip_per;  // tile_recip(tiles of a system)
   int zstep;         // planes the block's threads load at a time
   int ns;            // sweeps (1 unless WHOLE)
   int64_t tab_step;  // tables per sweep
@@ -74,16 +75,15 @@ inline size_t tile3d_setup(tile3d_args &a, int L, bool whole, int tx, int ty, in
   const int col0 = whole ? (L * L + 1) / 2 : (tx / 2 + 1) * (ty + 2), col1 = whole ? L * L / 2 : tx / 2 * ty;
   a.chunks0 = (col0 + a.C - 1) / a.C;
   a.chunks1 = (col1 + a.C - 1) / a.C;
-  auto recip = [](int d) { return ((1 << 20) + d - 1) / d; };
   const int row = odd ? W : W / 2;  // columns or pairs of columns a thread loads
   if (row * H > threads) return 0;
   a.zstep = threads / (row * H);
-  a.recip_pairs = recip(row * H);
-  a.recip_hw = recip(row);
-  a.recip_ntx = recip(a.ntx);
-  a.recip_per = (uint32_t)((((uint64_t)1 << 32) + a.ntx * a.nty - 1) / (a.ntx * a.nty));  // not used with one tile
-  a.recip_n0 = recip(whole ? std::max(L / 2, 1) : tx / 2 + 1);
-  a.recip_n1 = recip(whole ? std::max(L / 2, 1) : tx / 2);
+  a.recip_pairs = small_recip(row * H);
+  a.recip_hw = small_recip(row);
+  a.recip_ntx = small_recip(a.ntx);
+  a.recip_per = tile_recip((uint32_t)(a.ntx * a.nty));
+  a.recip_n0 = small_recip(whole ? std::max(L / 2, 1) : tx / 2 + 1);
+  a.recip_n1 = small_recip(whole ? std::max(L / 2, 1) : tx / 2);
   return ((size_t)W * H * a.lp + (odd ? odd_list_words(W, H) : 0)) * 8;
 }
 
@@ -131,9 +131,6 @@ template <int S>
 struct seg3d_couplings {
   uint64_t jw[S], je[S], jn[S], js[S], jd[S], ju;  // -x, +x, -y, +y, +z bonds; the first plane's -z bond
 };
-
-// quotient of small non-negative integers (n * (d - 1) < 2^20)
-__device__ __forceinline__ int small_div(int n, int d_recip20) { return (int)(((uint32_t)n * (uint32_t)d_recip20) >> 20); }
 
 // wave `chunk`'s columns of one colour; LDS column row * W/2 + i of a colour is pair column
 // i of a row (tx = 2i + ((row + colour) & 1))
@@ -553,9 +550,8 @@ __global__ void __launch_bounds__(1024) k_tile3d_odd(tile3d_args t) {
   const uint32_t per = (uint32_t)(t.ntx * t.nty);  // blocks to tiles as in k_tile3d
   const uint32_t b = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (b >= per * (uint32_t)t.a.nsys) return;
-  const uint32_t sys = per == 1 ? b : (uint32_t)(((uint64_t)b * t.recip_per) >> 32), r = b - sys * per;
-  const int by = small_div((int)r, t.recip_ntx);
-  tile3d_odd<COUNTER, FAST, S, WHOLE>(t, (int)sys, (int)r - by * t.ntx, by, lds);
+  const tile_place p = place_tile(b, per, t.recip_per, (uint32_t)t.ntx, t.recip_ntx);
+  tile3d_odd<COUNTER, FAST, S, WHOLE>(t, (int)p.sys, (int)p.bx, (int)p.by, lds);
 }
 
 template <bool COUNTER, bool FAST, int S, bool WHOLE, bool ONE>
@@ -568,9 +564,8 @@ __global__ void __launch_bounds__(1024) k_tile3d(tile3d_args t) {
   const uint32_t per = (uint32_t)(t.ntx * t.nty);
   const uint32_t b = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (b >= per * (uint32_t)t.a.nsys) return;
-  const uint32_t sys = per == 1 ? b : (uint32_t)(((uint64_t)b * t.recip_per) >> 32), r = b - sys * per;
-  const int by = small_div((int)r, t.recip_ntx);
-  tile3d<COUNTER, FAST, S, WHOLE, ONE>(t, (int)sys, (int)r - by * t.ntx, by, lds);
+  const tile_place p = place_tile(b, per, t.recip_per, (uint32_t)t.ntx, t.recip_ntx);
+  tile3d<COUNTER, FAST, S, WHOLE, ONE>(t, (int)p.sys, (int)p.bx, (int)p.by, lds);
 }
 
 }  // namespace sa
