@@ -5,6 +5,7 @@
 
 #include "sa_internal.hpp"
 #include "sa_tile2d.hpp"
+#include "sa_tile_place.hpp"
 
 namespace {
 
@@ -108,12 +109,20 @@ void sa_detail::tile2d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t ta
   const int mode = l->kind == SA_KIND_2P ? sa::T2_OPEN : fast ? sa::T2_FAST : sa::T2_GENERAL;
 #define SA_T2(C, M) \
   if (counter == C && mode == M) launch_it<C, M>(a, c, l->stream)
-  SA_T2(true, sa::T2_FAST);
-  SA_T2(true, sa::T2_GENERAL);
-  SA_T2(true, sa::T2_OPEN);
-  SA_T2(false, sa::T2_FAST);
-  SA_T2(false, sa::T2_GENERAL);
-  SA_T2(false, sa::T2_OPEN);
+  const int64_t most = sa::systems_per_launch((uint32_t)c.bands, 1024);  // 4 million lattices held whole
+  for (int64_t left_sys = l->nsys; left_sys > 0;) {
+    a.a.nsys = (int)std::min(left_sys, most);
+    SA_T2(true, sa::T2_FAST);
+    SA_T2(true, sa::T2_GENERAL);
+    SA_T2(true, sa::T2_OPEN);
+    SA_T2(false, sa::T2_FAST);
+    SA_T2(false, sa::T2_GENERAL);
+    SA_T2(false, sa::T2_OPEN);
+    left_sys -= a.a.nsys;
+    a.a.s += a.a.nsys * l->N;
+    a.out += a.a.nsys * l->N;
+    a.a.tab += a.a.nsys;
+  }
 #undef SA_T2
   if (!c.wrap) std::swap(l->s, l->s_alt);
 }

@@ -24,9 +24,12 @@ int main() {
   long checked = 0, wrong = 0;
   for (auto g : grids) {
     const uint32_t ntx = g.first, per = ntx * g.second, rp = sa::tile_recip(per);
-    const int rx = sa::small_recip((int)ntx), threads = 256;
-    const int64_t most = sa::systems_per_launch(per, threads);
-    if (most < 1 || (most * per + 7) / 8 * 8 * threads >= (int64_t)1 << 32) ++wrong;
+    const int rx = sa::small_recip((int)ntx);
+    for (int threads : {64, 256, 1024}) {
+      const int64_t n = sa::systems_per_launch(per, threads);
+      if (n < 1 || (n * per + 7) / 8 * 8 * threads >= (int64_t)1 << 32) ++wrong;
+    }
+    const int64_t most = sa::systems_per_launch(per, 256);
     for (int64_t sys = 0; sys < most; ++sys)
       for (uint32_t r : {0u, per - 1}) {
         const uint32_t b = (uint32_t)sys * per + r;
