@@ -150,7 +150,11 @@ int sa_measure_noalloc(int kind, int L, int nsys, const uint64_t *s, const uint6
                        const uint64_t *jz, int32_t *E, int32_t *M, void *stream);
 
 /* Exchange the lanes selected by `mask` between systems a and b
- * (swap, src/gpu_3d.cu:310-328, src/cpu_3d.cpp:429-444). */
+ * (swap, src/gpu_3d.cu:310-328, src/cpu_3d.cpp:429-444).  Asynchronous.
+ * Counter-mode sweeps and swaps may be captured from the ladder's stream into a graph.  A
+ * ladder that has been captured sweeps in place from then on, so that the graph stays valid:
+ * small ladders are then slower than before, as the tiles in LDS write a second array (the
+ * fused 3D sweep does so always and is captured as it stands). */
 int sa_ladder_swap(sa_ladder *l, int a, int b, uint64_t mask);
 
 /* nsteps parallel-tempering steps with the exchange decided on the device (the drivers use

@@ -53,7 +53,7 @@ struct sa_ladder {
   bool words_busy = false;  // replay: the staged words may still be on their way (words_ev)
   hipEvent_t words_ev = nullptr;
   int *sys_list = nullptr;  // device copy of a measured subset (more than 4 systems)
-  bool captured = false;   // sweeps were captured from the stream: they stay in place
+  bool captured = false;   // sweeps or swaps were captured from the stream: the spins stay in place
   int sys_per_thread = 0;  // SA_TUNE_SYS_PER_THREAD, 0 = automatic
   int sweep3d_kernel = 0;  // SA_TUNE_SWEEP3D_KERNEL, 0 = automatic
   int rows_per_tile = 0;   // SA_TUNE_ROWS_PER_TILE, 0 = automatic

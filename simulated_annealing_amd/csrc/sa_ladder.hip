@@ -747,9 +747,9 @@ bool have_alt(sa_ladder *l) {
   return false;
 }
 
-// A caller may capture the ladder's stream.  The tiles allocate at their first sweep and leave
-// the spins in the other array; a ladder once captured keeps to the sweeps that work in place
-// (a fused walk aside), so its graph finds the spins where they were.
+// A caller may capture the ladder's stream (sweeps and swaps).  The tiles allocate at their
+// first sweep and leave the spins in the other array; a ladder once captured keeps to the sweeps
+// that work in place (a fused walk aside), so its graph finds the spins where they were.
 void note_capture(sa_ladder *l) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(l->stream, &st) != hipSuccess) (void)hipGetLastError();
@@ -1029,6 +1029,7 @@ int sa_ladder_swap(sa_ladder *l, int a, int b, uint64_t mask) {
   rc = check_sys(l, b);
   if (rc) return rc;
   if (a == b || mask == 0) return SA_OK;
+  note_capture(l);
   const int64_t blocks = std::min<int64_t>((l->N + 255) / 256, 2048);
   hipLaunchKernelGGL(sa::k_swap, dim3((unsigned)blocks), dim3(256), 0, l->stream, l->s + (int64_t)a * l->N,
                      l->s + (int64_t)b * l->N, mask, l->N);
