@@ -69,54 +69,22 @@ class parallel_tempering {
     }
   }
 
-  // n x step(0); one device wait for all of them where every system is a slot of one ladder
-  // (on_device), otherwise one by one
+  // n x step(0); where every system is a slot of one ladder (on_device) with one device wait
+  // for up to kRun steps, otherwise one by one
   void steps(int n) {
-    if (n > 0 && on_device()) {
-      steps_on_device(n);
-      return;
+    while (n > 0) {
+      const int run = std::min(n, kRun), done = on_device() ? steps_on_device(run) : 0;
+      n -= done;
+      if (done == run) continue;
+      host_step(0);
+      --n;
     }
-    for (int k = 0; k < n; ++k) step(0);
   }
 
   // src/parallel_tempering.hpp:81-115
   void step(int stride) {
-    if (stride == 0 && on_device()) {
-      steps_on_device(1);
-      return;
-    }
-    const bool grouped = stride == 0 && all_on_ladders();
-    int i;
-    double u;
-    if (grouped) {
-      // Whole step at once: one launch sequence per ladder.  With stride 0 the step
-      // uses only the coldest system's energies (E_min) and the exchanging pair's;
-      // the pair is drawn first (the draws do not depend on the energies), those
-      // systems are measured now and the others when E is next read -- their spins
-      // do not change before that, so the values are the reference's.
-      // The reference folds E[0] into E_min after every sweep of the step, and E[0]
-      // changes only at the last one: the sweeps before it fold the previous step's
-      // E[0] in again.  That is a no-op except after reset() (E_min zeroed, E[0]
-      // still the energies from before), so it is done once here.
-      if (steps_ > 1) min_E_update();
-      sweep_all(steps_);
-      i = uniform_int(gen_, uni_a_, uni_b_);
-      u = canonical32(gen_);
-      measure_some({0, i, i + 1});
-      min_E_update();
-    } else {
-      for (long s = 0; s < steps_; ++s) {
-        sweep_all(1);
-        if (((stride != 0) && ((s % stride) == 0)) || s == (steps_ - 1)) measure_all();
-        if (stride != 0 && (s % stride) == 0) print(PRINT_E);
-        else if (stride == 0) min_E_update();
-      }
-      i = uniform_int(gen_, uni_a_, uni_b_);
-      u = canonical32(gen_);
-    }
-    std::unique_ptr<spin_t[]> mask = creat_mask(i, u);
-    if (log_) log_->push_back(swap_record{i, u, (uint64_t)mask[0]});
-    sys_[i]->swap(sys_[i + 1], std::move(mask));
+    if (stride == 0 && on_device() && steps_on_device(1) == 1) return;
+    host_step(stride);
   }
 
   void print(print_select select) {
@@ -304,6 +272,42 @@ class parallel_tempering {
   }
 
  private:
+  // one step driven by the host
+  void host_step(int stride) {
+    const bool grouped = stride == 0 && all_on_ladders();
+    int i;
+    double u;
+    if (grouped) {
+      // Whole step at once: one launch sequence per ladder.  With stride 0 the step
+      // uses only the coldest system's energies (E_min) and the exchanging pair's;
+      // the pair is drawn first (the draws do not depend on the energies), those
+      // systems are measured now and the others when E is next read -- their spins
+      // do not change before that, so the values are the reference's.
+      // The reference folds E[0] into E_min after every sweep of the step, and E[0]
+      // changes only at the last one: the sweeps before it fold the previous step's
+      // E[0] in again.  That is a no-op except after reset() (E_min zeroed, E[0]
+      // still the energies from before), so it is done once here.
+      if (steps_ > 1) min_E_update();
+      sweep_all(steps_);
+      i = uniform_int(gen_, uni_a_, uni_b_);
+      u = canonical32(gen_);
+      measure_some({0, i, i + 1});
+      min_E_update();
+    } else {
+      for (long s = 0; s < steps_; ++s) {
+        sweep_all(1);
+        if (((stride != 0) && ((s % stride) == 0)) || s == (steps_ - 1)) measure_all();
+        if (stride != 0 && (s % stride) == 0) print(PRINT_E);
+        else if (stride == 0) min_E_update();
+      }
+      i = uniform_int(gen_, uni_a_, uni_b_);
+      u = canonical32(gen_);
+    }
+    std::unique_ptr<spin_t[]> mask = creat_mask(i, u);
+    if (log_) log_->push_back(swap_record{i, u, (uint64_t)mask[0]});
+    sys_[i]->swap(sys_[i + 1], std::move(mask));
+  }
+
   std::unique_ptr<spin_t[]> creat_mask(int i, double rand) {
     const size_t words = E_[i].size() / 64;
     std::unique_ptr<spin_t[]> mask(new spin_t[words > 0 ? words : 1]);
@@ -339,11 +343,15 @@ class parallel_tempering {
     const std::type_info &t = typeid(h);
     return t == typeid(hip_sys) || t == typeid(::hip_3d) || t == typeid(::hip_2d) || t == typeid(::hip_2d_periodic);
   }
-  // step(0) n times: the pairs and uniforms do not depend on the energies, so all are drawn
-  // first (in step's order), the device decides each exchange by the threshold that the
+  static constexpr int kRun = 128;
+  // step(0) up to kRun times: the pairs and uniforms do not depend on the energies, so all are
+  // drawn first (in step's order), the device decides each exchange by the threshold that the
   // uniform comes to, and the energies and masks are folded in afterwards as step does.
-  void steps_on_device(int n) {
+  // Returns the steps done: fewer than n on an error (no memory for the records, say), with
+  // nothing drawn for the others.
+  int steps_on_device(int n) {
     ladder *l = as_hip(sys_[0])->get_ladder().get();
+    const mt19937 before = gen_;
     std::vector<int> pair(n), a(n), b(n);
     std::vector<double> u(n), ha(n), hb(n);
     std::vector<float> thr(n);
@@ -363,8 +371,13 @@ class parallel_tempering {
     const int rc = sa_ladder_exchange_steps(l->get(), (int)steps_, n, as_hip(sys_[0])->index(), a.data(), b.data(),
                                             thr.data(), ha.data(), hb.data(), masks.data(), EM.data());
     if (rc != SA_OK) {
-      log_error("exchange steps", rc);
-      return;
+      if (rc != SA_ERR_NOMEM) log_error("exchange steps", rc);
+      n = sa_ladder_exchange_steps_done(l->get());
+      gen_ = before;
+      for (int k = 0; k < n; ++k) {
+        (void)uniform_int(gen_, uni_a_, uni_b_);
+        (void)canonical32(gen_);
+      }
     }
     const double h0 = as_hip(sys_[0])->get_h();
     for (int k = 0; k < n; ++k) {
@@ -386,6 +399,7 @@ class parallel_tempering {
       num_switch_[i](acc / (double)64.);
       if (log_) log_->push_back(swap_record{i, u[k], masks[k]});
     }
+    return n;
   }
 
   void min_E_update() {

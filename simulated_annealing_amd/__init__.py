@@ -33,7 +33,7 @@ EXPORTS = [
     "sa_ladder_set_spins", "sa_ladder_get_spins", "sa_ladder_set_temperature", "sa_ladder_sweep",
     "sa_ladder_anneal",
     "sa_ladder_measure", "sa_ladder_measure_systems", "sa_measure_noalloc", "sa_ladder_swap",
-    "sa_ladder_exchange_steps", "sa_ladder_sync", "sa_ladder_stream",
+    "sa_ladder_exchange_steps", "sa_ladder_exchange_steps_done", "sa_ladder_sync", "sa_ladder_stream",
     "sa_ladder_set_tuning", "sa_ladder_get_tuning",
     "sa_pt_run", "sa_anneal_run", "sa_anneal_geometric",
     "sa_pt_create", "sa_pt_step", "sa_pt_sync", "sa_pt_steps_done", "sa_pt_result", "sa_pt_ladder",

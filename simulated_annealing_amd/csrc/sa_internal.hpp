@@ -50,6 +50,7 @@ struct sa_ladder {
   hipEvent_t meas_ev = nullptr;  // what wait_stream polls
   int *xcnt = nullptr;     // counters of a run of exchange steps (allocated at the first)
   char *x_pin = nullptr;   // pinned: their masks, then E and M
+  int xdone = 0;           // steps that the last sa_ladder_exchange_steps did
   bool words_busy = false;  // replay: the staged words may still be on their way (words_ev)
   hipEvent_t words_ev = nullptr;
   int *sys_list = nullptr;  // device copy of a measured subset (more than 4 systems)

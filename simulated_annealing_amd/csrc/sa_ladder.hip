@@ -1039,6 +1039,7 @@ int sa_ladder_swap(sa_ladder *l, int a, int b, uint64_t mask) {
 
 int sa_ladder_exchange_steps(sa_ladder *l, int sweeps, int nsteps, int cold, const int *a, const int *b,
                              const float *min_dE, const double *ha, const double *hb, uint64_t *masks, int32_t *EM) {
+  if (l) l->xdone = 0;
   int rc = check_sys(l, cold);
   if (rc) return rc;
   if (!a || !b || !min_dE || !ha || !hb || !masks || !EM || sweeps < 0 || nsteps < 0)
@@ -1052,10 +1053,12 @@ int sa_ladder_exchange_steps(sa_ladder *l, int sweeps, int nsteps, int cold, con
   constexpr size_t kRec = 384 * sizeof(int32_t);
   if (!l->xcnt && hipMalloc(&l->xcnt, sizeof(int) * kCnt * kRun) != hipSuccess) {
     l->xcnt = nullptr;
+    (void)hipGetLastError();
     return sa_fail(SA_ERR_NOMEM, "exchange counters");
   }
   if (!l->x_pin && hipHostMalloc((void **)&l->x_pin, kRun * (8 + kRec), hipHostMallocDefault) != hipSuccess) {
     l->x_pin = nullptr;
+    (void)hipGetLastError();
     return sa_fail(SA_ERR_NOMEM, "pinned exchange records");
   }
   unsigned long long *mask_pin = (unsigned long long *)l->x_pin;
@@ -1063,12 +1066,13 @@ int sa_ladder_exchange_steps(sa_ladder *l, int sweeps, int nsteps, int cold, con
   const int64_t bonds = bonds_per_site(l->kind) * l->N - (l->kind == SA_KIND_2P ? l->L : 0);
   for (int k0 = 0; k0 < nsteps; k0 += kRun) {
     const int run = std::min(kRun, nsteps - k0);
+    int launched = 0;
     hipLaunchKernelGGL(sa::k_fill_zero, dim3((unsigned)((run * kCnt + 255) / 256)), dim3(256), 0, l->stream, l->xcnt,
                        run * kCnt);
     for (int q = 0; q < run; ++q) {
       const int k = k0 + q;
       rc = sa_ladder_sweep(l, sweeps);
-      if (rc) return rc;
+      if (rc) break;
       const bool third = cold != a[k] && cold != b[k];
       const int n = third ? 3 : 2;
       int *cnt = l->xcnt + (size_t)q * kCnt;
@@ -1091,15 +1095,25 @@ int sa_ladder_exchange_steps(sa_ladder *l, int sweeps, int nsteps, int cold, con
       // about four words per thread: every block sums the counters first
       const unsigned blocks = (unsigned)std::min<int64_t>((l->N + 1023) / 1024, 1024);
       hipLaunchKernelGGL(sa::k_exchange, dim3(blocks), dim3(256), 0, l->stream, x);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) {
+        rc = sa_fail(SA_ERR_HIP, "exchange step: %s", hipGetErrorString(e));
+        break;
+      }
+      ++launched;
     }
-    SA_HIP_TRY(hipGetLastError());
-    rc = wait_stream(l);
+    // the steps before one that failed are finished and recorded
+    const int wrc = wait_stream(l);
+    if (wrc) return wrc;
+    std::memcpy(masks + k0, mask_pin, 8 * launched);
+    std::memcpy(EM + (size_t)384 * k0, em_pin, kRec * launched);
+    l->xdone += launched;
     if (rc) return rc;
-    std::memcpy(masks + k0, mask_pin, 8 * run);
-    std::memcpy(EM + (size_t)384 * k0, em_pin, kRec * run);
   }
   return SA_OK;
 }
+
+int sa_ladder_exchange_steps_done(const sa_ladder *l) { return l ? l->xdone : -1; }
 
 int sa_ladder_set_tuning(sa_ladder *l, int key, int value) {
   if (!l) return sa_fail(SA_ERR_ARG, "null ladder");
