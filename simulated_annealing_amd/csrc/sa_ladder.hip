@@ -27,6 +27,9 @@ int sa_fail(int status, const char *fmt, ...) {
   vsnprintf(buf, sizeof buf, fmt, ap);
   va_end(ap);
   g_last_error = buf;
+  // reported here: the runtime keeps a thread's last error until it is read, and the check after
+  // a later launch must not find it
+  if (status == SA_ERR_HIP || status == SA_ERR_NOMEM) (void)hipGetLastError();
   return status;
 }
 
@@ -1053,12 +1056,10 @@ int sa_ladder_exchange_steps(sa_ladder *l, int sweeps, int nsteps, int cold, con
   constexpr size_t kRec = 384 * sizeof(int32_t);
   if (!l->xcnt && hipMalloc(&l->xcnt, sizeof(int) * kCnt * kRun) != hipSuccess) {
     l->xcnt = nullptr;
-    (void)hipGetLastError();
     return sa_fail(SA_ERR_NOMEM, "exchange counters");
   }
   if (!l->x_pin && hipHostMalloc((void **)&l->x_pin, kRun * (8 + kRec), hipHostMallocDefault) != hipSuccess) {
     l->x_pin = nullptr;
-    (void)hipGetLastError();
     return sa_fail(SA_ERR_NOMEM, "pinned exchange records");
   }
   unsigned long long *mask_pin = (unsigned long long *)l->x_pin;
