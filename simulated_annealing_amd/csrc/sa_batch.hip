@@ -856,7 +856,15 @@ int add_instance(sa_batch *b, int kind, int L, int nsys, uint64_t seed, int nswe
   batch_inst in;
   int rc = prepare_instance(kind, L, nsys, seed, nsweeps, T, per_sweep, h, pt, true, in);
   if (rc == SA_ERR_NOMEM) {
-    // the instances' tile arrays give way to a new instance: all go back to half-sweeps
+    // the instances' tile arrays give way to a new instance: all go back to half-sweeps, unless
+    // even that is too little
+    int64_t extras = 0;
+    for (const batch_inst &x : b->inst)
+      if (x.live) extras += form_bytes(x.lad->kind, x.lad->L, x.lad->nsys, x.form);
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
+        (int64_t)free_b + extras < sa_detail::batch_instance_bytes(kind, L, nsys, nsweeps, per_sweep))
+      return rc;
     const int src = sync_batch(b);
     if (src) return src;
     for (batch_inst &x : b->inst)

@@ -35,15 +35,17 @@ def test_ladder_goes_on_after_a_refused_one(orc):
 
 
 def test_batch_goes_on_after_a_refused_instance(orc):
-    """the tiles' arrays give way first; the instances then go on with half-sweeps"""
+    """... and keep their tiles' arrays, which would not have made room for it"""
     b = sa.Batch()
     T = np.array([0.6, 0.9, 1.4])
     insts = [(b.add_pt(2, 12, T, 70, 2, 9), 2, 12, 70), (b.add_pt(1, 96, T, 71, 2, 9), 1, 96, 71)]
     b.run(5)
-    before = lambda: refused(lambda: b.add(*TOO_LARGE[:2], 1, 10, T=[1.0] * TOO_LARGE[2], nsys=TOO_LARGE[2]))  # noqa: E731
-    assert "memory" in before()
+    held = b.bytes()
+    refuse = lambda: refused(lambda: b.add(*TOO_LARGE[:2], 1, 10, T=[1.0] * TOO_LARGE[2], nsys=TOO_LARGE[2]))  # noqa: E731
+    assert "memory" in refuse()
     b.run(6)
-    assert "memory" in before()
+    assert "memory" in refuse()
+    assert b.bytes() == held
     assert b.run() == 0
     for i, kind, L, seed in insts:
         want = orc.pt_run(kind, L, T, 0.0, seed, 2, 9, rng_mode=1)
