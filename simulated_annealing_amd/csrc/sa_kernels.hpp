@@ -1386,9 +1386,10 @@ __device__ __forceinline__ void meas_finish(const meas_big (&big)[SB], meas_shar
     __hip_atomic_store(&rep.out[q], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
   if (threadIdx.x == 0) atomicExch(rep.ticket, 0u);
-  __builtin_amdgcn_s_waitcnt(0);  // every count has reached host memory before the flag leaves
+  // every wave's counts have left before the barrier, and the flag is a release for the host
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if (threadIdx.x == 0) __hip_atomic_store(rep.flag, rep.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (threadIdx.x == 0) __hip_atomic_store(rep.flag, rep.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Block = one unit (3D: 256 in-plane sites x up to `walk` planes; 2D: 256*walk

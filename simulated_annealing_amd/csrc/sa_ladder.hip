@@ -3,7 +3,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -867,7 +866,7 @@ int measure_list(sa_ladder *l, const int *list, int n) {
       hipLaunchKernelGGL(sa::k_fill_zero, dim3((unsigned)((all + 255) / 256)), dim3(256), 0, l->stream, l->cnt, all);
     }
     l->cnt_clear = false;
-    volatile unsigned long long *flag = (volatile unsigned long long *)l->cnt_pin;
+    auto flag = [l] { return __atomic_load_n((const unsigned long long *)l->cnt_pin, __ATOMIC_ACQUIRE); };
     sa::meas_report rep;
     rep.ticket = ticket;
     rep.out = (int *)(l->cnt_pin + 64);
@@ -878,15 +877,14 @@ int measure_list(sa_ladder *l, const int *list, int n) {
     SA_HIP_TRY(hipGetLastError());
     // the host polls the flag; now and then it asks the stream, which also ends the wait if
     // the launch failed
-    for (unsigned spin = 1; *flag != rep.seq; ++spin) {
+    for (unsigned spin = 1; flag() != rep.seq; ++spin) {
       if (spin % 4096) continue;
       const hipError_t e = hipStreamQuery(l->stream);
       if (e == hipErrorNotReady) continue;
       SA_HIP_TRY(e);
-      if (*flag == rep.seq) break;
+      if (flag() == rep.seq) break;
       return sa_fail(SA_ERR_HIP, "the measurement did not report");
     }
-    std::atomic_thread_fence(std::memory_order_acquire);
     std::memcpy(l->cnt_h.data(), rep.out, sizeof(int) * cnt_n);
     l->cnt_clear = true;
     return SA_OK;
