@@ -44,6 +44,7 @@
 
 #include "sa/exchange.hpp"
 #include "sa_internal.hpp"
+#include "sa_per_device.hpp"
 #include "sa_tile2d.hpp"
 #include "sa_tile3d.hpp"
 
@@ -368,7 +369,7 @@ const int kNumCands = 2;
 
 struct sa_batch {
   hipStream_t stream = nullptr;
-  int cus = 256;
+  int device = 0, cus = 256;
   std::vector<batch_inst> inst;  // indexed by id
   // device state of the current schedule
   dev_array<inst_desc> d_desc;
@@ -611,9 +612,11 @@ int graph_for(sa_batch *b, int k, hipGraphExec_t &out) {
     return SA_OK;
   }
   hipGraph_t g = nullptr;
-  static const hipError_t more = hipFuncSetAttribute((const void *)k_batch_tile3d,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
-  (void)more;
+  // more than 64 KB of dynamic LDS has to be asked for
+  static sa::per_device_once once;
+  SA_HIP_TRY((hipError_t)once(b->device, [] {
+    return hipFuncSetAttribute((const void *)k_batch_tile3d, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
+  }));
   SA_HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   const int erc = enqueue_sweeps(b, k);
   const hipError_t ee = hipStreamEndCapture(b->stream, &g);
@@ -1031,9 +1034,8 @@ extern "C" {
 int sa_batch_create(sa_batch **out) {
   if (!out) return sa_fail(SA_ERR_ARG, "null output handle");
   sa_batch *b = new sa_batch();
-  int dev = 0;
   hipDeviceProp_t prop;
-  if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
+  if (hipGetDevice(&b->device) == hipSuccess && hipGetDeviceProperties(&prop, b->device) == hipSuccess &&
       prop.multiProcessorCount > 0)
     b->cus = prop.multiProcessorCount;
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess || hipEventCreate(&b->ev0) != hipSuccess ||

@@ -72,8 +72,8 @@ void tile2d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, boo
 // The same for 3D ladders (sa_tile3d.hpp); *us: the modelled time per sweep.
 int tile3d_sweeps(const sa_ladder *l, int64_t left, bool *second, double *us);
 bool tile3d_couplings(sa_ladder *l);
-void tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, bool fast, const uint64_t *words,
-                   uint64_t t, int64_t left);
+int tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, bool fast, const uint64_t *words,
+                  uint64_t t, int64_t left);
 // acceptance thresholds of one temperature/field for a ladder of `kind`; fast =
 // the table qualifies for the symmetric low-levels-always kernels
 void make_table(int kind, double T, double h, sa::sys_table &tab, bool &fast, double *boltz_out);

@@ -767,8 +767,10 @@ int launch_sweeps(sa_ladder *l, const uint64_t *words, uint64_t t, int64_t n) {
     if (ns > 0 && second && !have_alt(l)) ns = 0;
     if (ns > 0 && l->kind == SA_KIND_3D && !sa_detail::tile3d_couplings(l)) ns = 0;
     if (ns > 0) {
-      if (l->kind == SA_KIND_3D) sa_detail::tile3d_launch(l, l->tab, 0, all_of(l->fast), w, t + k, n - k);
-      else sa_detail::tile2d_launch(l, l->tab, 0, all_of(l->fast), w, t + k, n - k, ns);
+      const int rc =
+          l->kind == SA_KIND_3D ? sa_detail::tile3d_launch(l, l->tab, 0, all_of(l->fast), w, t + k, n - k) : SA_OK;
+      if (rc) return rc;
+      if (l->kind != SA_KIND_3D) sa_detail::tile2d_launch(l, l->tab, 0, all_of(l->fast), w, t + k, n - k, ns);
       k += ns;
     } else {
       // no memory for the tiles' extras: the fused walk writes a second array too
@@ -965,7 +967,8 @@ int anneal_run(sa_ladder *l, const double *T, int64_t left, double h, int64_t *d
     if (l->kind == SA_KIND_3D) {
       ns = sa_detail::tile3d_sweeps(l, n - k, &second, &us);
       if (second && !have_alt(l)) break;
-      sa_detail::tile3d_launch(l, l->tab_seq + k * l->nsys, l->nsys, fast, nullptr, l->t + k, n - k);
+      const int rc = sa_detail::tile3d_launch(l, l->tab_seq + k * l->nsys, l->nsys, fast, nullptr, l->t + k, n - k);
+      if (rc) return rc;
     } else {
       ns = sa_detail::tile2d_sweeps(l, n - k, &second);
       if (second && !have_alt(l)) break;

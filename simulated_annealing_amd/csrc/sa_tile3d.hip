@@ -5,6 +5,7 @@
 #include <cmath>
 
 #include "sa_internal.hpp"
+#include "sa_per_device.hpp"
 #include "sa_tile3d.hpp"
 
 namespace {
@@ -65,24 +66,33 @@ tile_cfg pick(const sa_ladder *l, int64_t left, double &cost) {
   return best;
 }
 
+// more than 64 KB of dynamic LDS has to be asked for, once per kernel and device
+template <class K>
+int allow_lds(sa::per_device_once &once, int device, K kernel) {
+  return once(device, [&] {
+    return hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
+  });
+}
+
+// 0 or the error of the LDS request (nothing launched)
 template <bool COUNTER, bool FAST, int S>
-void launch(const sa::tile3d_args &t, const tile_cfg &c, hipStream_t st) {
+int launch(const sa::tile3d_args &t, const tile_cfg &c, int device, hipStream_t st) {
   const dim3 grid((unsigned)((t.ntx * t.nty * t.a.nsys + 7) / 8 * 8));
   const size_t lds = c.lds;
   auto go = [&](auto whole, auto one) {
-    constexpr bool WH = decltype(whole)::value, ON = decltype(one)::value;
-    static const hipError_t more = hipFuncSetAttribute((const void *)sa::k_tile3d<COUNTER, FAST, S, WH, ON>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
-    (void)more;  // more than 64 KB of dynamic LDS
-    hipLaunchKernelGGL((sa::k_tile3d<COUNTER, FAST, S, WH, ON>), grid, dim3(c.threads), lds, st, t);
+    constexpr auto kernel = sa::k_tile3d<COUNTER, FAST, S, decltype(whole)::value, decltype(one)::value>;
+    static sa::per_device_once once;
+    if (const int e = allow_lds(once, device, kernel)) return e;
+    hipLaunchKernelGGL(kernel, grid, dim3(c.threads), lds, st, t);
+    return 0;
   };
   if (t.a.L & 1) {
     auto go_odd = [&](auto whole) {
-      constexpr bool WH = decltype(whole)::value;
-      static const hipError_t more = hipFuncSetAttribute((const void *)sa::k_tile3d_odd<COUNTER, FAST, S, WH>,
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
-      (void)more;
-      hipLaunchKernelGGL((sa::k_tile3d_odd<COUNTER, FAST, S, WH>), grid, dim3(c.threads), lds, st, t);
+      constexpr auto kernel = sa::k_tile3d_odd<COUNTER, FAST, S, decltype(whole)::value>;
+      static sa::per_device_once once;
+      if (const int e = allow_lds(once, device, kernel)) return e;
+      hipLaunchKernelGGL(kernel, grid, dim3(c.threads), lds, st, t);
+      return 0;
     };
     return c.whole ? go_odd(std::true_type{}) : go_odd(std::false_type{});
   }
@@ -90,7 +100,7 @@ void launch(const sa::tile3d_args &t, const tile_cfg &c, hipStream_t st) {
   if constexpr (S == 2) {  // the kept couplings fit the registers
     if (one) return c.whole ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
   }
-  c.whole ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
+  return c.whole ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
 }
 
 // in (rows x cols) to out (cols x rows, `stride` words per row), 32 x 32 words at a time;
@@ -133,8 +143,8 @@ int sa_detail::tile3d_sweeps(const sa_ladder *l, int64_t left, bool *second, dou
   return c.S > 0 ? c.ns : 0;
 }
 
-void sa_detail::tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, bool fast, const uint64_t *words,
-                              uint64_t t, int64_t left) {
+int sa_detail::tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t tab_step, bool fast, const uint64_t *words,
+                             uint64_t t, int64_t left) {
   double cost = 0;
   const tile_cfg c = pick(l, left, cost);
   sa::tile3d_args a = c.a;
@@ -157,18 +167,18 @@ void sa_detail::tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t ta
   a.ns = c.ns;
   a.tab_step = tab_step;
   const bool counter = l->rng_mode == SA_RNG_COUNTER;
-#define SA_T3(CO, FA)                                                   \
-  if (counter == CO && fast == FA) {                                    \
-    if (c.S == 2) launch<CO, FA, 2>(a, c, l->stream);                   \
-    else launch<CO, FA, 4>(a, c, l->stream);                            \
-  }
+#define SA_T3(CO, FA)                                                                                             \
+  if (counter == CO && fast == FA)                                                                                \
+    e = c.S == 2 ? launch<CO, FA, 2>(a, c, l->device, l->stream) : launch<CO, FA, 4>(a, c, l->device, l->stream);
   const int64_t most = sa::systems_per_launch((uint32_t)(a.ntx * a.nty), c.threads);
   for (int64_t left_sys = l->nsys; left_sys > 0;) {
+    int e = 0;
     a.a.nsys = (int)std::min(left_sys, most);
     SA_T3(true, true)
     SA_T3(true, false)
     SA_T3(false, true)
     SA_T3(false, false)
+    if (e) return sa_fail(SA_ERR_HIP, "LDS of the 3D tiles: %s", hipGetErrorString((hipError_t)e));
     left_sys -= a.a.nsys;
     a.a.s += a.a.nsys * l->N;
     a.out += a.a.nsys * l->N;
@@ -176,4 +186,5 @@ void sa_detail::tile3d_launch(sa_ladder *l, const sa::sys_table *tab, int64_t ta
   }
 #undef SA_T3
   if (!c.whole) std::swap(l->s, l->s_alt);
+  return SA_OK;
 }
