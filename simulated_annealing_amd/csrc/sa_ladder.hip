@@ -857,8 +857,9 @@ int measure_list(sa_ladder *l, const int *list, int n) {
   }
   // The counts land in pinned memory allocated at the first measurement (so creating a
   // ladder, e.g. per served request, needs no pinned allocation): the flag, then the counts.
+  // Coherent: the host polls the flag while the kernel that stores it still runs.
   const size_t pin = 64 + sizeof(int) * 128 * (size_t)l->nsys;
-  if (!l->cnt_pin && hipHostMalloc((void **)&l->cnt_pin, pin, hipHostMallocDefault) == hipSuccess)
+  if (!l->cnt_pin && hipHostMalloc((void **)&l->cnt_pin, pin, hipHostMallocCoherent) == hipSuccess)
     std::memset(l->cnt_pin, 0, pin);
   if (!l->cnt_pin) (void)hipGetLastError();
   if (l->cnt_pin) {
