@@ -115,9 +115,12 @@ int sa_ladder_set_temperature(sa_ladder *l, int sys, double T, double h, double 
 
 /* `nsweeps` sweeps of every system (sweep(), src/gpu_3d.cu:100-114 and
  * src/cpu_3d.cpp:94-105): per sweep, the offset-0 then the offset-1 sites in the
- * reference CPU order.  Asynchronous on the ladder's stream in counter mode; in
- * replay mode the host draws the words and the call returns when they are
- * consumed. */
+ * reference CPU order.  Asynchronous on the ladder's stream; in replay mode the host
+ * draws the words and the call returns when the last of them are on their way.  The
+ * first sweep of a ladder may take device memory for a second spin array and, in 3D,
+ * a second copy of the couplings, kept until the ladder is destroyed; where that is
+ * not to be had it takes kernels that work in place (the fused 3D sweep, which has no
+ * such form, returns SA_ERR_NOMEM). */
 int sa_ladder_sweep(sa_ladder *l, int nsweeps);
 
 /* An anneal on the ladder: before sweep t, system j gets temperature T[t*nsys+j]
@@ -198,8 +201,8 @@ void *sa_ladder_stream(sa_ladder *l);
 /* Parallel tempering as main_gpu runs it (src/main_gpu.cu:262-416,
  * src/parallel_tempering.hpp:54-115): nT systems seeded with `seed`
  * (set_seed, init_J, set_seed, init_rand), temperatures sorted ascending,
- * `nsteps` x step(0) with `sweeps` sweeps per step, swap decisions on the host from
- * mt19937(123).  One ladder holds all temperatures.  Outputs may be NULL:
+ * `nsteps` x step(0) with `sweeps` sweeps per step, pairs and uniforms drawn on the host
+ * from mt19937(123), swaps decided on the device.  One ladder holds all temperatures.  Outputs may be NULL:
  * pairs[nsteps], us[nsteps], masks[nsteps], E_last[nT*64] (measure() vectors after
  * the last step), spins[nT*N]. */
 int sa_pt_run(int kind, int L, int nT, const double *T, double h, uint64_t seed, int sweeps, int nsteps,
@@ -355,7 +358,7 @@ typedef struct sa_request_result {
   int status; /* SA_OK, an sa_status for a refused request, SA_ERR_STATE while unfinished */
   int steps;  /* PT exchange attempts logged */
   double arrival, admitted, finished; /* server clock, seconds */
-  int64_t bytes;   /* device memory held while admitted */
+  int64_t bytes;   /* sa_request_bytes of the request (the tiles' arrays not included) */
   double attempts; /* spin-flip attempts: sites x 64 x systems x sweeps */
   uint64_t spins_digest; /* sa_digest over all systems' spin words (system j from index j*N) */
   uint64_t log_digest;   /* PT: chained splitmix64 of (pair, uniform bits, mask) per step */
@@ -366,7 +369,7 @@ typedef struct sa_serve_config {
   int64_t hbm_budget; /* device bytes for admitted requests (0: half the free memory) */
   int max_active;     /* requests on the device at once (0: 512) */
   int chunk;          /* sweeps between admission points (0: 10) */
-  int digests;        /* 1: read final spins back and digest them */
+  int digests;        /* 1: digest the final spins (on the device) */
   int prep_threads;   /* host threads preparing admitted requests (0: automatic) */
 } sa_serve_config;
 typedef struct sa_serve_stats {
@@ -393,8 +396,10 @@ int sa_serve_get_stats(sa_serve *s, sa_serve_stats *st);
 /* the temperatures a request runs at (nsweeps for an anneal, nT for PT); returns the
  * count, T may be NULL */
 int sa_request_temperatures(const sa_request *r, double *T, int64_t capacity);
-/* device bytes a request holds while admitted (what admission charges against
- * hbm_budget), or an sa_status for an invalid request */
+/* device bytes a request needs while admitted, which admission charges against hbm_budget, or
+ * an sa_status for an invalid request.  While half of the budget is free, a request also holds (and
+ * is charged for) the second spin array and coupling copy of the sweeps in LDS tiles; the
+ * server's bytes and peak_bytes include them. */
 int64_t sa_request_bytes(const sa_request *r);
 /* XOR over i of splitmix64(w[i] + (first_index + i) * 0x9E3779B97F4A7C15) */
 uint64_t sa_digest(const uint64_t *w, int64_t n, uint64_t first_index);

@@ -4,7 +4,7 @@
 // What bounds a 2D lattice of ordinary size is not memory but launches: one half-sweep
 // per launch costs 3-4 us of which the update is a fraction.  Here a workgroup keeps a
 // tile in LDS through `ns` whole sweeps and touches memory only at the start and the end:
-//   WRAP: the whole lattice (at most 2048 items, L up to 90), updated in place; one workgroup per system.
+//   WRAP: the whole lattice (at most 2048 items, L up to 88), updated in place; one workgroup per system.
 //   bands: TH full rows plus 2*ns halo rows on either side.  Half-sweep h (0 .. 2*ns-1)
 //     updates the rows at least h+1 away from the tile's edge, so after ns sweeps the TH
 //     rows in the middle are exact and the halo's have been recomputed redundantly (the

@@ -22,9 +22,8 @@
 // cache line of its own, and the address unit took 9 of a sweep's 22 thousand cycles for
 // them), and both planes of a segment are one 128-bit access.
 //
-// One L=64 system: 12.6 -> 7.3 us per sweep, of which 4.3 are the kernel (load 1.1, colour 0
-// 1.6, colour 1 0.7, store 0.4) and the rest the launch; 16 systems of L=32 15.6 -> 7.4; 12 of
-// L=16, held whole, 9.5 -> 2.9; 8 of L=48 with a field 37 -> 19.5.
+// One L=64 system: 12.6 -> 7.2 us per sweep (kernel trace: 6.0 at least); 16 systems of L=32
+// 15.6 -> 7.4; 12 of L=16, held whole, 9.5 -> 2.9; 8 of L=48 with a field 37 -> 19.5.
 #pragma once
 
 #include <algorithm>
@@ -326,8 +325,8 @@ __device__ __forceinline__ void tile3d_update(const tile3d_args &t, const sys_ta
 }
 
 // Tile (bx, by) of system sys.  ONE: a wave has at most one chunk of columns per colour,
-// whose places and couplings it then keeps: both colours' couplings are in flight while
-// the tile is loaded, and with several sweeps they are loaded once.
+// whose places and couplings it then keeps: colour 0's couplings are in flight while the tile
+// is loaded, colour 1's while colour 0 is updated, and with several sweeps both are loaded once.
 template <bool COUNTER, bool FAST, int S, bool WHOLE, bool ONE>
 __device__ __forceinline__ void tile3d(const tile3d_args &t, int sys, int bx, int by, uint64_t *lds) {
   const sweep_args &p = t.a;
@@ -362,7 +361,7 @@ __device__ __forceinline__ void tile3d(const tile3d_args &t, int sys, int bx, in
   {
     uint64_t a[4], b[4];
     fetch(zt, a, b);
-    if (ONE) {  // while they are on their way: places, couplings and random words of both colours
+    if (ONE) {  // while they are on their way: both colours' places and random words, colour 0's couplings
       q0 = tile3d_segment<S, WHOLE>(t, 0, wv, ox, oy);
       tile3d_load<S>(t, q0, d0);
       q1 = tile3d_segment<S, WHOLE>(t, 1, wv, ox, oy);
