@@ -390,8 +390,8 @@ struct sa_batch {
   dev_array<swap_item> d_swap;
   dev_array<int> d_cnt;
   pinned h_cnt;
-  // tuning: 0 = automatic (fused: 0 or 1, the fused band walk is not in the batch)
-  int block = 0, chunk = 0, fused = 0;
+  // tuning: 0 = automatic
+  int block = 0, chunk = 0;
   int tuned_block = 0, tuned_chunk = 0;
   std::vector<std::pair<int, float>> trials;  // (candidate, ms per work item)
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1189,7 +1189,6 @@ int sa_batch_set_tuning(sa_batch *b, int key, int value) {
   } else if (key == SA_TUNE_BATCH_FUSED) {
     if (value < 0 || value > 2) return sa_fail(SA_ERR_ARG, "batch fused must be 0 (auto), 1 (off) or 2 (on)");
     if (value == 2) return sa_fail(SA_ERR_ARG, "the fused batch sweep is switched off in this build");
-    b->fused = value;
   } else {
     return sa_fail(SA_ERR_ARG, "unknown batch tuning key %d", key);
   }
