@@ -166,8 +166,9 @@ int sa_ladder_swap(sa_ladder *l, int a, int b, uint64_t mask);
  *   -(e_a - e_b) >= min_dE[k],   e_s = float(E_s + h_s * M_s),
  * ha[k], hb[k] the two fields.  masks[k]: the exchanged lanes.  EM[k][3][2][64]: E and M of
  * cold, a[k] and b[k] before the exchange.  On an error the steps before the failing one may
- * be done: sa_ladder_exchange_steps_done returns how many steps the last call did (and
- * recorded), -1 for a null ladder. */
+ * be done: sa_ladder_exchange_steps_done returns how many steps the last call did and
+ * recorded (after SA_ERR_HIP, of the up to 128 steps since the last wait none is counted),
+ * -1 for a null ladder. */
 int sa_ladder_exchange_steps(sa_ladder *l, int sweeps, int nsteps, int cold, const int *a, const int *b,
                              const float *min_dE, const double *ha, const double *hb, uint64_t *masks, int32_t *EM);
 int sa_ladder_exchange_steps_done(const sa_ladder *l);

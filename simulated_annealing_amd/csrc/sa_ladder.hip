@@ -1098,14 +1098,12 @@ int sa_ladder_exchange_steps(sa_ladder *l, int sweeps, int nsteps, int cold, con
       // about four words per thread: every block sums the counters first
       const unsigned blocks = (unsigned)std::min<int64_t>((l->N + 1023) / 1024, 1024);
       hipLaunchKernelGGL(sa::k_exchange, dim3(blocks), dim3(256), 0, l->stream, x);
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess) {
-        rc = sa_fail(SA_ERR_HIP, "exchange step: %s", hipGetErrorString(e));
-        break;
-      }
       ++launched;
     }
-    // the steps before one that failed are finished and recorded
+    SA_HIP_TRY(hipGetLastError());
+    // no memory for a sweep: the steps before it are finished and recorded (a runtime error may
+    // be of any launch of the run)
+    if (rc && rc != SA_ERR_NOMEM) return rc;
     const int wrc = wait_stream(l);
     if (wrc) return wrc;
     std::memcpy(masks + k0, mask_pin, 8 * launched);
